@@ -135,6 +135,8 @@ struct alamo_el_s {
     int dense_M = 0;
     double* dense_I = nullptr;     // identity, the unit vectors of the assembly
     double* dense_A = nullptr;     // operator, column-major
+    double* bottom_vals = nullptr; // its rows without the zeros, over the diagonal (k_bottom_rows)
+    unsigned short* bottom_cols = nullptr;
     // direct bottom (ALAMO_EL_BOTTOM_DIRECT): the finest MG level with at
     // most kDirectMax unknowns and the FP64 inverse of its operator
     int direct_level = -1;
@@ -179,7 +181,7 @@ constexpr int kRedBlocks = 1024;
 // (FP32 solve at 129^3: 23.9 ms against 24.1 with 2048, 24.2 with 4096,
 // 24.4 with 768 and 25.6 with 512)
 constexpr int kDotBlocks = 1024;
-constexpr int kDenseMax = 1536;  // unknowns; LDS of the dense BiCGStab = 9 M doubles
+constexpr int kDenseMax = 1536;  // unknowns: two threads a node in one workgroup of k_bottom_bicgstab
 constexpr int kDirectMax = 4096; // unknowns of the direct bottom level (an M x M FP64 inverse)
 // Weights of the red-black Gauss-Seidel smoother.  Interior rows: 0.9; the
 // undamped 1.0 converges fastest on a polycrystal (V-cycle factor 0.775 vs
@@ -505,8 +507,17 @@ struct Cycle {
         const double* b = lv.d.res;
         if (!std::is_same<T, double>::value) launch_copy_cast(lv);
         if (h->dense_A) {
-            ael::k_bottom_bicgstab_dense<<<1, kBlock, sizeof(double) * 9 * Mb, s>>>(
-                x, b, h->dense_A, lv.d.diag, Mb, h->omega, bottom_max_iter, bottom_tol, nuf, h->bottom_status);
+            const int Nb = (int)lv.L.N;
+            const unsigned nt = (unsigned)((2 * Nb + 63) / 64 * 64);
+            const size_t lds = sizeof(double) * 5 * Mb;  // at most 61 KB
+            if (Nb <= ael::kBottomRegN)
+                ael::k_bottom_bicgstab<true><<<1, nt, lds, s>>>(x, b, h->bottom_vals, h->bottom_cols, lv.d.diag, Nb,
+                                                                h->omega, bottom_max_iter, bottom_tol, nuf,
+                                                                h->bottom_status);
+            else
+                ael::k_bottom_bicgstab<false><<<1, nt, lds, s>>>(x, b, h->bottom_vals, h->bottom_cols, lv.d.diag, Nb,
+                                                                 h->omega, bottom_max_iter, bottom_tol, nuf,
+                                                                 h->bottom_status);
             if (!std::is_same<T, double>::value)
                 ael::k_cast<double, float><<<nblk(Mb), kBlock, 0, s>>>(lv.d.cor, lv.f.cor, Mb);
             return;
@@ -648,10 +659,13 @@ int assemble_dense(alamo_el_t h, hipStream_t s) {
     const int M = (int)(3 * lb.L.N);
     if (M > kDenseMax) return 0;
     if (h->dense_M != M) {
-        for (double* p : {h->dense_I, h->dense_A})
+        for (void* p : {(void*)h->dense_I, (void*)h->dense_A, (void*)h->bottom_vals, (void*)h->bottom_cols})
             if (p) (void)hipFree(p);
-        h->dense_I = h->dense_A = nullptr;
+        h->dense_I = h->dense_A = h->bottom_vals = nullptr;
+        h->bottom_cols = nullptr;
         ALLOC(h->dense_I, (long)M * M);
+        ALLOC(h->bottom_vals, (long)ael::kRowSlots * M);
+        ALLOC(h->bottom_cols, (long)ael::kRowSlots * lb.L.N);
         ALLOC(h->dense_A, (long)M * M);
         ael::k_eye<<<nblk((long)M * M), kBlock, 0, s>>>(h->dense_I, M);
         h->dense_M = M;
@@ -663,6 +677,8 @@ int assemble_dense(alamo_el_t h, hipStream_t s) {
         default: ael::k_assemble_dense<2><<<grid, kBlock, 0, s>>>(h->dense_I, lb.d.C, h->bct_dev, h->uniform, lb.L, h->dense_A); break;
     }
     psi_post_columns(h, lb, h->dense_I, h->dense_A, M, s);
+    ael::k_bottom_rows<<<(unsigned)((lb.L.N + 63) / 64), 64, 0, s>>>(h->dense_A, lb.d.diag, (int)lb.L.N, h->bottom_vals,
+                                                                     h->bottom_cols);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1376,7 +1392,8 @@ int alamo_el_destroy(alamo_el_t h) {
     for (void* p : {(void*)h->bct_dev, (void*)h->bcv_dev, (void*)h->red_partial, (void*)h->red_out,
                     (void*)h->bottom_work, (void*)h->bottom_status, (void*)h->gu9, (void*)h->dw9, (void*)h->csoa,
                     (void*)h->kv, (void*)h->kz, (void*)h->kw, (void*)h->kh, (void*)h->kpart,
-                    (void*)h->dense_I, (void*)h->dense_A, (void*)h->nn_in, (void*)h->nn_out,
+                    (void*)h->dense_I, (void*)h->dense_A, (void*)h->bottom_vals,
+                    (void*)h->bottom_cols, (void*)h->nn_in, (void*)h->nn_out,
                     (void*)h->nn_bc, (void*)h->nn_t, (void*)h->nn_fmean})
         if (p) (void)hipFree(p);
     if (h->red_host) (void)hipHostFree(h->red_host);

@@ -1358,130 +1358,6 @@ __global__ void __launch_bounds__(kBlock) k_transpose(const double* __restrict__
     }
 }
 
-// Block-wide max (op 0) or sum (op 1) for kBlock threads; all threads get it.
-__device__ __forceinline__ double blk_reduce256(double v, int op, double* red) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double o = __shfl_xor(v, off);
-        v = op == 0 ? fmax(v, o) : v + o;
-    }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = 0.0;
-    for (int q = 0; q < kBlock / 64; ++q) r = op == 0 ? fmax(r, red[q]) : r + red[q];
-    return r;
-}
-
-// The reference bottom solve on the dense coarsest operator: MLCGSolver
-// BiCGStab with the diagonal as left preconditioner, then the smoothing of a
-// failed solve (see k_bottom_solve for the stencil form of the same
-// algorithm).  Vectors live in LDS (9 M doubles).  One workgroup of kBlock.
-__global__ void __launch_bounds__(kBlock)
-    k_bottom_bicgstab_dense(double* __restrict__ xg, const double* __restrict__ rhs, const double* __restrict__ Acol,
-                            const double* __restrict__ diag, int M, double omega, int maxiter, double eps_rel, int nuf,
-                            int* __restrict__ status) {
-    extern __shared__ double sm[];
-    __shared__ double red[kBlock / 64];
-    double *x = sm, *r = sm + M, *rh = sm + 2 * M, *p = sm + 3 * M, *v = sm + 4 * M, *s = sm + 5 * M,
-           *t = sm + 6 * M, *b = sm + 7 * M, *d = sm + 8 * M;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    auto matvec = [&](const double* in, double* out) {
-        __syncthreads();
-        for (int row = tid; row < M; row += nt) {
-            double acc = 0.0;
-            for (int c = 0; c < M; ++c) acc += Acol[(long)c * M + row] * in[c];
-            out[row] = acc;
-        }
-        __syncthreads();
-    };
-    for (int q = tid; q < M; q += nt) { x[q] = 0.0; b[q] = rhs[q]; d[q] = diag[q]; }
-    __syncthreads();
-    matvec(x, v);
-    double loc = 0.0;
-    for (int q = tid; q < M; q += nt) {
-        const double rq = (b[q] + (-1.0) * v[q]) / d[q];
-        r[q] = rq;
-        rh[q] = rq;
-        loc = fmax(loc, fabs(rq));
-    }
-    const double rnorm0 = blk_reduce256(loc, 0, red);
-    double rnorm = rnorm0, rho_1 = 0.0, alpha = 0.0, omg = 0.0;
-    int ret = 0;
-    if (rnorm0 != 0.0) {
-        for (int iter = 1; iter <= maxiter; ++iter) {
-            loc = 0.0;
-            for (int q = tid; q < M; q += nt) loc += rh[q] * r[q];
-            const double rho = blk_reduce256(loc, 1, red);
-            if (rho == 0.0) { ret = 1; break; }
-            if (iter == 1) {
-                for (int q = tid; q < M; q += nt) p[q] = r[q];
-            } else {
-                const double beta = (rho / rho_1) * (alpha / omg);
-                for (int q = tid; q < M; q += nt) p[q] = r[q] + beta * (p[q] + (-omg) * v[q]);
-            }
-            matvec(p, v);
-            loc = 0.0;
-            for (int q = tid; q < M; q += nt) {
-                v[q] /= d[q];
-                loc += rh[q] * v[q];
-            }
-            const double rhTv = blk_reduce256(loc, 1, red);
-            if (rhTv != 0.0) alpha = rho / rhTv;
-            else { ret = 2; break; }
-            loc = 0.0;
-            for (int q = tid; q < M; q += nt) {
-                x[q] += alpha * p[q];
-                const double sq = 1.0 * r[q] + (-alpha) * v[q];
-                s[q] = sq;
-                loc = fmax(loc, fabs(sq));
-            }
-            rnorm = blk_reduce256(loc, 0, red);
-            if (rnorm < eps_rel * rnorm0) break;
-            matvec(s, t);
-            double l1 = 0.0, l2 = 0.0;
-            for (int q = tid; q < M; q += nt) {
-                t[q] /= d[q];
-                l1 += t[q] * t[q];
-                l2 += t[q] * s[q];
-            }
-            const double tt = blk_reduce256(l1, 1, red);
-            const double ts = blk_reduce256(l2, 1, red);
-            if (tt != 0.0) omg = ts / tt;
-            else { ret = 3; break; }
-            loc = 0.0;
-            for (int q = tid; q < M; q += nt) {
-                x[q] += omg * s[q];
-                const double rq = 1.0 * s[q] + (-omg) * t[q];
-                r[q] = rq;
-                loc = fmax(loc, fabs(rq));
-            }
-            rnorm = blk_reduce256(loc, 0, red);
-            if (rnorm < eps_rel * rnorm0) break;
-            if (omg == 0.0) { ret = 4; break; }
-            rho_1 = rho;
-        }
-        if (ret == 0 && rnorm > eps_rel * rnorm0) ret = 8;
-        if (!((ret == 0 || ret == 8) && rnorm < rnorm0))
-            for (int q = tid; q < M; q += nt) x[q] = 0.0;
-        if (ret != 0 && ret != 9)
-            for (int q = tid; q < M; q += nt) x[q] = 0.0;
-        const int nsm = ret == 0 ? 0 : nuf;
-        for (int sw = 0; sw < 2 * nsm; ++sw) {
-            matvec(x, v);
-            for (int q = tid; q < M; q += nt) {
-                const double Rx = v[q] - x[q] * d[q];
-                t[q] = (1.0 - omega) * x[q] + omega * (b[q] - Rx) / d[q];
-            }
-            __syncthreads();
-            for (int q = tid; q < M; q += nt) x[q] = t[q];
-        }
-    }
-    __syncthreads();
-    for (int q = tid; q < M; q += nt) xg[q] = x[q];
-    if (tid == 0) status[0] = ret;
-}
-
 // h[i] partials of V_i . w for i < k <= kMultiDotMax (V: k vectors of length
 // M, stride M).  Each thread reads w[q] once and keeps the k running sums in
 // registers, so one pass streams V and w once; the block then reduces each
