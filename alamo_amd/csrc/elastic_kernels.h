@@ -215,10 +215,13 @@ __device__ __forceinline__ void bc_set(const int* __restrict__ t3, const T u[3],
 }
 
 __device__ __forceinline__ void node_ijk(long id, const Lvl& L, int& i, int& j, int& k) {
-    const long t = id / L.nx;
-    i = (int)(id - t * L.nx);
-    k = (int)(t / L.ny);
-    j = (int)(t - (long)k * L.ny);
+    // 32-bit: a box holds fewer than 2^29 nodes (checked at create), and a
+    // 64-bit division takes several times the instructions of a 32-bit one
+    const unsigned q = (unsigned)id, nx = (unsigned)L.nx, ny = (unsigned)L.ny;
+    const unsigned t = q / nx, kk = t / ny;
+    i = (int)(q - t * nx);
+    k = (int)kk;
+    j = (int)(t - kk * ny);
 }
 
 // One-sided first derivative at the faces, central inside (src/Numeric/Stencil.H:70-191).

@@ -64,29 +64,30 @@ __host__ __device__ inline long boundary_count(const Lvl& L) { return L.N - inte
 
 // The t-th boundary node, t < boundary_count(L): the planes k = 0 and
 // k = nz-1 whole, then for each inner plane its ring of face nodes.
-__device__ __forceinline__ void boundary_node(const Lvl& L, long t, int& i, int& j, int& k) {
-    const long plane = (long)L.nx * L.ny;
+__device__ __forceinline__ void boundary_node(const Lvl& L, long t64, int& i, int& j, int& k) {
+    const unsigned nx = (unsigned)L.nx, ny = (unsigned)L.ny, plane = nx * ny;  // 32-bit as in node_ijk
+    unsigned t = (unsigned)t64;
     if (t < 2 * plane) {
         const bool top = t >= plane;
-        const long r = top ? t - plane : t;
+        const unsigned r = top ? t - plane : t, q = r / nx;
         k = top ? L.nz - 1 : 0;
-        j = (int)(r / L.nx);
-        i = (int)(r - (long)j * L.nx);
+        j = (int)q;
+        i = (int)(r - q * nx);
         return;
     }
     t -= 2 * plane;
-    const long ring = 2L * L.nx + 2L * (L.ny - 2);
-    const long kk = t / ring;
-    long r = t - kk * ring;
+    const unsigned ring = 2 * nx + 2 * (ny - 2);
+    const unsigned kk = t / ring;
+    unsigned r = t - kk * ring;
     k = 1 + (int)kk;
-    if (r < L.nx) {
+    if (r < nx) {
         j = 0;
         i = (int)r;
-    } else if (r < 2L * L.nx) {
+    } else if (r < 2 * nx) {
         j = L.ny - 1;
-        i = (int)(r - L.nx);
+        i = (int)(r - nx);
     } else {
-        r -= 2L * L.nx;
+        r -= 2 * nx;
         j = 1 + (int)(r >> 1);
         i = (r & 1) ? L.nx - 1 : 0;
     }
@@ -96,17 +97,16 @@ __device__ __forceinline__ void boundary_node(const Lvl& L, long t, int& i, int&
 __device__ __forceinline__ bool slab_interior_node(const Lvl& L, long ib, int& i, int& j, int& k, long& id) {
     const int ni = L.nx - 2, nj = L.ny - 2, nk = L.nz - 2;
     if (ni <= 0 || nj <= 0 || nk <= 0) return false;
-    const int x = (int)(ib % kXcd);
-    const long lb = ib / kXcd;
-    const int j0 = (int)((long)x * nj / kXcd), j1 = (int)((long)(x + 1) * nj / kXcd);
-    const long per_plane = (long)(j1 - j0) * ni;
-    const long t = lb * blockDim.x + threadIdx.x;
-    if (t >= per_plane * nk) return false;
-    const long kk = t / per_plane;
-    const long r = t - kk * per_plane;
-    const int jj = (int)(r / ni);
-    i = 1 + (int)(r - (long)jj * ni);
-    j = 1 + j0 + jj;
+    const unsigned x = (unsigned)ib % kXcd, lb = (unsigned)ib / kXcd;
+    const unsigned j0 = x * (unsigned)nj / kXcd, j1 = (x + 1) * (unsigned)nj / kXcd;
+    const unsigned per_plane = (j1 - j0) * (unsigned)ni;
+    const unsigned t = lb * blockDim.x + threadIdx.x;  // below 2^29 + the padding of the last workgroups
+    if (t >= per_plane * (unsigned)nk) return false;
+    const unsigned kk = t / per_plane;
+    const unsigned r = t - kk * per_plane;
+    const unsigned jj = r / (unsigned)ni;
+    i = 1 + (int)(r - jj * (unsigned)ni);
+    j = 1 + (int)(j0 + jj);
     k = 1 + (int)kk;
     id = ((long)k * L.ny + j) * L.nx + i;
     return true;

@@ -249,15 +249,14 @@ inline unsigned tile_blocks(const TileGrid& G) {
 // Tile (it, jt) and chunk kc of interior workgroup ib; false for the
 // padding workgroups of XCDs with fewer j-tiles (uniform over the workgroup).
 __device__ __forceinline__ bool tile_of(const TileGrid& G, long ib, int& it, int& jt, int& kc) {
-    const int x = (int)(ib % kXcd);
-    const long lb = ib / kXcd;
-    const int t0 = (int)((long)x * G.nty / kXcd), t1 = (int)((long)(x + 1) * G.nty / kXcd);
-    const long per = (long)(t1 - t0) * G.ntx;
-    if (per == 0 || lb >= per * G.nkc) return false;
+    const unsigned x = (unsigned)ib % kXcd, lb = (unsigned)ib / kXcd;
+    const int t0 = (int)(x * (unsigned)G.nty / kXcd), t1 = (int)((x + 1) * (unsigned)G.nty / kXcd);
+    const unsigned per = (unsigned)(t1 - t0) * (unsigned)G.ntx;
+    if (per == 0 || lb >= per * (unsigned)G.nkc) return false;
     kc = (int)(lb / per);
-    const long r = lb - (long)kc * per;
-    jt = t0 + (int)(r / G.ntx);
-    it = (int)(r - (long)(jt - t0) * G.ntx);
+    const unsigned r = lb - (unsigned)kc * per;
+    jt = t0 + (int)(r / (unsigned)G.ntx);
+    it = (int)(r - (unsigned)(jt - t0) * (unsigned)G.ntx);
     return true;
 }
 
