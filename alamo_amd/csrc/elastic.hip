@@ -216,10 +216,16 @@ constexpr long kNtMinBytes = 64l << 20;
 // set) replaces both targets: the tests use it to reach every chunk length
 // on small boxes.
 constexpr long kTileTarget64 = 2 * 2 * 256, kTileTarget32 = 4 * 256;
-ael::TileGrid tile_grid_of(const Lvl& L, long target) {
+// The isotropic tiled kernel: at most 3 workgroups a CU in FP64, 7 in FP32.
+// FP64 sweeps with 512, 640, 768, 1024 and 2048 workgroups as the target:
+// 129 x 113 x 97 nodes 37.2, 34.1, 31.1, 31.7, 32.8 us; 65^3 nodes, in chunks of
+// 2 planes (which read 4) 9.2 us, in chunks of 1 (which read 3) 10.7; 201^3
+// nodes take the longest chunk for all, 211 us.
+constexpr long kTileTargetIso64 = 3 * 256, kTileTargetIso32 = 7 * 256;
+ael::TileGrid tile_grid_of(const Lvl& L, long target, bool up = false) {
     const char* e = std::getenv("ALAMO_EL_TILE_TARGET");
     const long t = e ? std::atol(e) : 0;
-    return ael::tile_grid<TileT>(L, t > 0 ? t : target);
+    return ael::tile_grid<TileT>(L, t > 0 ? t : target, up);
 }
 
 int stencil_variant() {
@@ -265,15 +271,18 @@ bool launch_tiled(alamo_el_t h, const Level& l, const TX* x, const T* b, const T
         if (l.pidx && vecs<T>(lv).pal)
             ael::k_stencil_lds<TileT, T, OP, true, 2, TX, PER><<<grid, TileT::NT, 0, s>>>(
                 x, b, diag, vecs<T>(lv).pal, vecs<T>(lv).Cb, vecs<T>(lv).C, h->bct_dev, u, L, w, gm, nbb, G, l.dwbase,
-                vecs<T>(lv).D, l.nflag, out, l.pidx, l.pidx_b);
+                vecs<T>(lv).D, l.nflag, out, l.pidx, l.pidx_b,
+                ael::Spc<T>(L));
         else if ((long)sizeof(T) * 21 * L.N >= kNtMinBytes)
             ael::k_stencil_lds<TileT, T, OP, true, 1, TX, PER><<<grid, TileT::NT, 0, s>>>(
                 x, b, diag, vecs<T>(lv).Ct, vecs<T>(lv).Cb, vecs<T>(lv).C, h->bct_dev, u, L, w, gm, nbb, G, l.dwbase,
-                vecs<T>(lv).D, l.nflag, out, nullptr, nullptr);
+                vecs<T>(lv).D, l.nflag, out, nullptr, nullptr,
+                ael::Spc<T>(L));
         else
             ael::k_stencil_lds<TileT, T, OP, true, 0, TX, PER><<<grid, TileT::NT, 0, s>>>(
                 x, b, diag, vecs<T>(lv).Ct, vecs<T>(lv).Cb, vecs<T>(lv).C, h->bct_dev, u, L, w, gm, nbb, G, l.dwbase,
-                vecs<T>(lv).D, l.nflag, out, nullptr, nullptr);
+                vecs<T>(lv).D, l.nflag, out, nullptr, nullptr,
+                ael::Spc<T>(L));
     };
     if (L.per) go(std::true_type{});
     else go(std::false_type{});
@@ -297,8 +306,20 @@ void launch_stencil_raw(alamo_el_t h, const Level& l, const T* x, const T* b, co
         return;
     }
     if (launch_tiled<T, OP, T>(h, l, x, b, diag, C, out, s)) return;
+    const ael::Spc<T> H(L);
+    if (h->sym == 0 && l.tiled && var == kVariantSlab) {
+        const ael::TileGrid& G = sizeof(T) == 8 ? l.tg : l.tg32;
+        const unsigned nb = ael::slab_boundary_blocks(L, kBlock), gi = nb + ael::tile_blocks(G);
+        if (L.per)
+            ael::k_stencil_iso<TileT, T, OP, true><<<gi, TileT::NT, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, nb, G,
+                                                                            out, H);
+        else
+            ael::k_stencil_iso<TileT, T, OP><<<gi, TileT::NT, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, nb, G, out,
+                                                                      H);
+        return;
+    }
     const unsigned g = ael::slab_blocks(L, kBlock), nbb = ael::slab_boundary_blocks(L, kBlock);
-    const bool masked = var == kVariantSlab || var == kVariantSlabOnly;
+    const bool masked = (var == kVariantSlab || var == kVariantSlabOnly) && h->sym != 0;
     const unsigned char* gm = masked ? l.gmask : nullptr;
     Level& lv = const_cast<Level&>(l);
     const bool have_d = l.dwbase && (l.nflag == 0 || vecs<T>(lv).D);
@@ -312,19 +333,19 @@ void launch_stencil_raw(alamo_el_t h, const Level& l, const T* x, const T* b, co
         switch (h->sym) {
             case 0:
                 ael::k_stencil_slab<T, 0, OP, false, P><<<g, kBlock, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, gm, nbb,
-                                                                          dwb, Dc, nf, out);
+                                                                          dwb, Dc, nf, out, H);
                 break;
             case 1:
                 if (dc)
                     ael::k_stencil_slab<T, 1, OP, true, P><<<g, kBlock, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, gm,
-                                                                             nbb, dwb, Dc, nf, out);
+                                                                             nbb, dwb, Dc, nf, out, H);
                 else
                     ael::k_stencil_slab<T, 1, OP, false, P><<<g, kBlock, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, gm,
-                                                                              nbb, dwb, Dc, nf, out);
+                                                                              nbb, dwb, Dc, nf, out, H);
                 break;
             default:
                 ael::k_stencil_slab<T, 2, OP, false, P><<<g, kBlock, 0, s>>>(x, b, diag, C, h->bct_dev, u, L, w, gm, nbb,
-                                                                          dwb, Dc, nf, out);
+                                                                          dwb, Dc, nf, out, H);
                 break;
         }
     };
@@ -862,6 +883,13 @@ int assemble_direct(alamo_el_t h, hipStream_t s) {
 // Levels whose interior is at least kTiledMin nodes along every axis use the
 // LDS-tiled MajorMinor kernel (unless ALAMO_EL_STENCIL=slab-only).
 constexpr int kTiledMin = 32;
+// Isotropic levels also need this many interior nodes: FP64 sweeps of 41^3 and
+// 49^3 nodes take 6.8 and 8.3 us in tiles (2 x 6 of them a plane, many lanes past
+// the box) and 7.0 and 7.8 us by node, of 65^3 nodes 9.2 and 12.1.
+constexpr long kTiledMinIso = 128l << 10;
+bool tiled_level(const Lvl& L) {
+    return stencil_variant() == kVariantSlab && L.nx - 2 >= kTiledMin && L.ny - 2 >= kTiledMin && L.nz - 2 >= kTiledMin;
+}
 
 // The palette of a tiled level (ael::k_pal_index): the distinct 21-slot
 // tensors of its nodes when there are at most ael::kPalMax of them and at most
@@ -973,8 +1001,7 @@ int build_palette(alamo_el_t h, Level& l, hipStream_t s) {
 
 int build_gradc(alamo_el_t h, Level& l, hipStream_t s) {
     if (h->sym != 1) return 0;
-    l.tiled = stencil_variant() == kVariantSlab && l.L.nx - 2 >= kTiledMin && l.L.ny - 2 >= kTiledMin &&
-              l.L.nz - 2 >= kTiledMin;
+    l.tiled = tiled_level(l.L);
     static_assert(TileT::NT == kBlock, "tiled and slab launches share the block size");
     l.tg = tile_grid_of(l.L, kTileTarget64);
     l.tg32 = tile_grid_of(l.L, kTileTarget32);
@@ -1055,11 +1082,14 @@ int build_gradc(alamo_el_t h, Level& l, hipStream_t s) {
 }
 
 int build_gmask(alamo_el_t h, Level& l, hipStream_t s) {
-    switch (h->sym) {
-        case 0: ael::k_grad_mask<2><<<nblk(l.L.N), kBlock, 0, s>>>(l.d.C, l.L, l.gmask); break;
-        case 1: ael::k_grad_mask<21><<<nblk(l.L.N), kBlock, 0, s>>>(l.d.C, l.L, l.gmask); break;
-        default: ael::k_grad_mask<9><<<nblk(l.L.N), kBlock, 0, s>>>(l.d.C, l.L, l.gmask); break;
+    if (h->sym == 0) {  // the isotropic rows read lambda and mu around the node and take no mask
+        l.tiled = tiled_level(l.L) && ael::interior_count(l.L) >= kTiledMinIso;
+        l.tg = tile_grid_of(l.L, kTileTargetIso64, true);
+        l.tg32 = tile_grid_of(l.L, kTileTargetIso32, true);
+        return 0;
     }
+    if (h->sym == 1) ael::k_grad_mask<21><<<nblk(l.L.N), kBlock, 0, s>>>(l.d.C, l.L, l.gmask);
+    else ael::k_grad_mask<9><<<nblk(l.L.N), kBlock, 0, s>>>(l.d.C, l.L, l.gmask);
     HIPCHK(hipGetLastError());
     return build_gradc(h, l, s);
 }

@@ -319,6 +319,27 @@ __device__ __forceinline__ void gradc_mm(const T* __restrict__ C, const Lvl& L, 
     }
 }
 
+// The grid spacings' factors of an interior row: first derivatives 1 / 2h_a,
+// second derivatives 1 / h_a^2 and the mixed ones 1 / 4 h_a h_b.  The stencil
+// kernels take them as an argument: uniform values then sit in scalar
+// registers (computed in the kernel they hold 18 vector registers in FP64).
+template <typename T>
+struct Spc {
+    T h2[3], ii[3], ixy, ixz, iyz;
+    __host__ __device__ __forceinline__ explicit Spc(const Lvl& L) {
+        const T ihx = T(1) / T(L.dx), ihy = T(1) / T(L.dy), ihz = T(1) / T(L.dz);
+        h2[0] = T(0.5) * ihx;
+        h2[1] = T(0.5) * ihy;
+        h2[2] = T(0.5) * ihz;
+        ii[0] = ihx * ihx;
+        ii[1] = ihy * ihy;
+        ii[2] = ihz * ihz;
+        ixy = T(0.25) * ihx * ihy;
+        ixz = T(0.25) * ihx * ihz;
+        iyz = T(0.25) * ihy * ihz;
+    }
+};
+
 // Interior row of Fapply for MajorMinor C, the same sums as contract3 and
 // contract2_col but streamed over the 21 slots: each slot is loaded once,
 // used for every term it enters, and dropped, so only the 18 second
@@ -342,25 +363,21 @@ __device__ __forceinline__ void mm_load(const T* __restrict__ u, const T* __rest
     for (int s = 0; s < 21; ++s) cv[s] = ld32(C + (size_t)s * N, o);
 }
 template <typename T>
-__device__ __forceinline__ void mm_compute(const T uv[3][19], const T cv[21], const Lvl& L, T out[3], T e1[6]) {
-    const T ihx = T(1) / T(L.dx), ihy = T(1) / T(L.dy), ihz = T(1) / T(L.dz);
-    const T hx2 = T(0.5) * ihx, hy2 = T(0.5) * ihy, hz2 = T(0.5) * ihz;
-    const T ixx = ihx * ihx, iyy = ihy * ihy, izz = ihz * ihz;
-    const T ixy = T(0.25) * ihx * ihy, ixz = T(0.25) * ihx * ihz, iyz = T(0.25) * ihy * ihz;
+__device__ __forceinline__ void mm_compute(const T uv[3][19], const T cv[21], const Spc<T>& H, T out[3], T e1[6]) {
     T gu[3][3], B[3][3][3];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
         const T* f = uv[p];
         const T c0 = f[0], xp = f[1], xm = f[2], yp = f[3], ym = f[4], zp = f[5], zm = f[6];
-        gu[p][0] = (xp - xm) * hx2;
-        gu[p][1] = (yp - ym) * hy2;
-        gu[p][2] = (zp - zm) * hz2;
-        B[p][0][0] = (xp - T(2) * c0 + xm) * ixx;
-        B[p][1][1] = (yp - T(2) * c0 + ym) * iyy;
-        B[p][2][2] = (zp - T(2) * c0 + zm) * izz;
-        B[p][0][1] = (f[7] + f[8] - f[9] - f[10]) * ixy;
-        B[p][0][2] = (f[11] + f[12] - f[13] - f[14]) * ixz;
-        B[p][1][2] = (f[15] + f[16] - f[17] - f[18]) * iyz;
+        gu[p][0] = (xp - xm) * H.h2[0];
+        gu[p][1] = (yp - ym) * H.h2[1];
+        gu[p][2] = (zp - zm) * H.h2[2];
+        B[p][0][0] = (xp - T(2) * c0 + xm) * H.ii[0];
+        B[p][1][1] = (yp - T(2) * c0 + ym) * H.ii[1];
+        B[p][2][2] = (zp - T(2) * c0 + zm) * H.ii[2];
+        B[p][0][1] = (f[7] + f[8] - f[9] - f[10]) * H.ixy;
+        B[p][0][2] = (f[11] + f[12] - f[13] - f[14]) * H.ixz;
+        B[p][1][2] = (f[15] + f[16] - f[17] - f[18]) * H.iyz;
         B[p][1][0] = B[p][0][1];
         B[p][2][0] = B[p][0][2];
         B[p][2][1] = B[p][1][2];
@@ -391,7 +408,7 @@ __device__ __forceinline__ void mm_core(const T* __restrict__ u, const T* __rest
                                         T out[3], T e1[6]) {
     T uv[3][19], cv[21];
     mm_load<T>(u, C, L, o, uv, cv);
-    mm_compute<T>(uv, cv, L, out, e1);
+    mm_compute<T>(uv, cv, Spc<T>(L), out, e1);
 }
 
 template <typename T>
@@ -488,12 +505,104 @@ __device__ __forceinline__ void apply_boundary(const TU* __restrict__ u, const T
     bc_set<T>(bct + 3 * reg, uu, gu, sg, nrm, out);
 }
 
+// Interior row of Fapply for an isotropic C = (lambda, mu):
+//   f_i = mu lap(u_i) + (lambda + mu) d_i(div u)
+//         + sum_a (d_a mu)(d_a u_i + d_i u_a) + (d_i lambda) div u,
+// the sums of contract3 and contract2_col with the terms that share a
+// derivative collected.  The operands at node o: of each component the centre,
+// x+, x-, y+, y-, z+, z-, then the corners (++, --, +-, -+) of its two mixed
+// derivatives (component p has no use for the one without p): xy, xz | xy, yz |
+// xz, yz; and lambda, mu at the centre and its six neighbours (an axis along
+// which they do not change adds an exact zero).
+template <typename T>
+__device__ __forceinline__ void iso_load(const T* __restrict__ u, const T* __restrict__ C, const Lvl& L, unsigned o,
+                                         T uv[3][15], T cv[2][7]) {
+    const unsigned N = (unsigned)L.N, sy = (unsigned)L.nx, sz = (unsigned)(L.nx * L.ny);
+    const unsigned nb[7] = {o, o + 1, o - 1, o + sy, o - sy, o + sz, o - sz};
+    const unsigned mix[3][4] = {{o + 1 + sy, o - 1 - sy, o + 1 - sy, o - 1 + sy},
+                                {o + 1 + sz, o - 1 - sz, o + 1 - sz, o - 1 + sz},
+                                {o + sy + sz, o - sy - sz, o + sy - sz, o - sy + sz}};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        const T* f = u + (size_t)p * N;
+#pragma unroll
+        for (int n = 0; n < 7; ++n) uv[p][n] = ld32(f, nb[n]);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            uv[p][7 + n] = ld32(f, mix[p == 2 ? 1 : 0][n]);
+            uv[p][11 + n] = ld32(f, mix[p == 0 ? 1 : 2][n]);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int n = 0; n < 7; ++n) cv[s][n] = ld32(C + (size_t)s * N, nb[n]);
+}
+// What the row takes of component p: its gradient, d_p d_p u_p, its Laplacian
+// and its two mixed derivatives.
+template <typename T>
+struct IsoD {
+    T g[3], dd, lap, m0, m1;
+};
+template <typename T>
+__device__ __forceinline__ IsoD<T> iso_derivs(int p, const T f[15], const Spc<T>& H) {
+    IsoD<T> r;
+    T d2[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        r.g[a] = (f[1 + 2 * a] - f[2 + 2 * a]) * H.h2[a];
+        d2[a] = (f[1 + 2 * a] - T(2) * f[0] + f[2 + 2 * a]) * H.ii[a];
+    }
+    r.lap = d2[0] + d2[1] + d2[2];
+    r.dd = d2[p];
+    r.m0 = (f[7] + f[8] - f[9] - f[10]) * (p == 2 ? H.ixz : H.ixy);
+    r.m1 = (f[11] + f[12] - f[13] - f[14]) * (p == 0 ? H.ixz : H.iyz);
+    return r;
+}
+// The row; dg: its diagonal, -2 (mu sum_l 1/h_l^2 + (lambda + mu) / h_i^2)
+// (Gradient_Diagonal through contract3).
+template <typename T>
+__device__ __forceinline__ void iso_row(const IsoD<T> D[3], const T cv[2][7], const Spc<T>& H, bool uniform, T out[3],
+                                        T dg[3]) {
+    const T lam = cv[0][0], mu = cv[1][0], lm = lam + mu;
+    // d_i(div u): the xy derivatives of u_0 and u_1, the xz of u_0 and u_2, the yz of u_1 and u_2
+    const T dv[3] = {D[0].dd + D[1].m0 + D[2].m0, D[0].m0 + D[1].dd + D[2].m1, D[0].m1 + D[1].m1 + D[2].dd};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) out[i] = mu * D[i].lap + lm * dv[i];
+    if (!uniform) {
+        const T tr = D[0].g[0] + D[1].g[1] + D[2].g[2];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const T gl = (cv[0][1 + 2 * a] - cv[0][2 + 2 * a]) * H.h2[a];
+            const T gm = (cv[1][1 + 2 * a] - cv[1][2 + 2 * a]) * H.h2[a];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) out[i] += gm * (D[i].g[a] + D[a].g[i]);
+            out[a] += gl * tr;
+        }
+    }
+    const T s = mu * (H.ii[0] + H.ii[1] + H.ii[2]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) dg[i] = T(-2) * (s + lm * H.ii[i]);
+}
+template <typename T>
+__device__ __forceinline__ void iso_compute(const T uv[3][15], const T cv[2][7], const Spc<T>& H, bool uniform, T out[3],
+                                            T dg[3]) {
+    IsoD<T> D[3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) D[p] = iso_derivs<T>(p, uv[p], H);
+    iso_row<T>(D, cv, H, uniform, out, dg);
+}
+
 // Interior row of Fapply at node id (no face of the box through it).
 template <typename T, int SYM>
 __device__ __forceinline__ void apply_interior(const T* __restrict__ u, const T* __restrict__ C, int uniform,
                                                const Lvl& L, long id, T out[3], unsigned gmask) {
     if constexpr (SYM == 1) {
         apply_interior_mm<T>(u, C, L, (unsigned)id, out, gmask, uniform != 0);
+    } else if constexpr (SYM == 0) {
+        T uv[3][15], cv[2][7], dg[3];
+        iso_load<T>(u, C, L, (unsigned)id, uv, cv);
+        iso_compute<T>(uv, cv, Spc<T>(L), uniform != 0, out, dg);
     } else {
         constexpr int NC = NComp<SYM>::value;
         const long N = L.N, sy = L.nx, sz = (long)L.nx * L.ny;

@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(kBlock)
     k_stencil_slab(const T* __restrict__ x, const T* __restrict__ b, const T* __restrict__ diag,
                    const T* __restrict__ C, const int* __restrict__ bct, int uniform, Lvl L, T omega,
                    const unsigned char* __restrict__ gmask, unsigned nbb, const int* __restrict__ dwbase,
-                   const T* __restrict__ Dc, int nflag, T* __restrict__ out) {
+                   const T* __restrict__ Dc, int nflag, T* __restrict__ out, Spc<T> H) {
     int i, j, k;
     long id;
     T o[3];
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(kBlock)
             }
             __builtin_amdgcn_sched_barrier(0);
             T e1[6];
-            mm_compute<T>(uv, cv, L, o, e1);
+            mm_compute<T>(uv, cv, H, o, e1);
             const unsigned long long bal = __ballot(gm != 0u);
             if (!uniform && gm != 0u) {
                 const unsigned p = (unsigned)dwb + (unsigned)__popcll(bal & lanes_below());
@@ -234,6 +234,20 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
             for (int p = 0; p < 3; ++p)
                 st32(out + (size_t)p * L.N, o32, finish_op<T, OP>(o[p], xv[p], bv[p], dv[p], omega));
+            return;
+        } else if constexpr (SYM == 0) {
+            // Every load of the node first, as for MajorMinor; the Jacobi
+            // diagonal from the lambda and mu already there instead of a load.
+            const unsigned o32 = (unsigned)id;
+            T uv[3][15], cv[2][7], bv[3], dg[3];
+            iso_load<T>(x, C, L, o32, uv, cv);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1) ? ld32(b + (size_t)p * L.N, o32) : T(0);
+            __builtin_amdgcn_sched_barrier(0);
+            iso_compute<T>(uv, cv, H, uniform != 0, o, dg);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                st32(out + (size_t)p * L.N, o32, finish_op<T, OP>(o[p], uv[p][0], bv[p], dg[p], omega));
             return;
         } else {
             apply_interior<T, SYM>(x, C, uniform, L, id, o, gmask ? (unsigned)gmask[id] : 7u);

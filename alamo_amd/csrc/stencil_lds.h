@@ -224,16 +224,17 @@ __global__ void __launch_bounds__(kBlock) k_pack_bnd_c(const double* __restrict_
 }
 
 // Tile grid of the interior of L: chunks of kc planes, with kc chosen so
-// that the launch has about target workgroups (1 to 16 planes per chunk).
+// that the launch has about target workgroups, at most target with up (1 to
+// 16 planes per chunk).
 template <class TS>
-inline TileGrid tile_grid(const Lvl& L, long target) {
+inline TileGrid tile_grid(const Lvl& L, long target, bool up = false) {
     TileGrid G{0, 0, 0, 1};
     const int ni = L.nx - 2, nj = L.ny - 2, nk = L.nz - 2;
     if (ni <= 0 || nj <= 0 || nk <= 0) return G;
     G.ntx = (ni + TS::TX - 1) / TS::TX;
     G.nty = (nj + TS::TY - 1) / TS::TY;
     const long per_plane = (long)G.ntx * G.nty;
-    long kc = ((long)nk * per_plane + target / 2) / target;  // nearest
+    long kc = ((long)nk * per_plane + (up ? target - 1 : target / 2)) / target;  // or the nearest
     kc = kc < 1 ? 1 : (kc > kMaxChunk ? kMaxChunk : kc);
     G.kc = (int)kc;
     G.nkc = (nk + G.kc - 1) / G.kc;
@@ -346,7 +347,7 @@ __global__ void __launch_bounds__(TS::NT)
                   const int* __restrict__ bct, int uniform,
                   Lvl L, T omega, const unsigned char* __restrict__ gmask, unsigned nbb, TileGrid G,
                   const int* __restrict__ dwbase, const T* __restrict__ Dc, int nflag, T* __restrict__ out,
-                  const PalIdx* __restrict__ pidx, const PalIdx* __restrict__ pidx_b) {
+                  const PalIdx* __restrict__ pidx, const PalIdx* __restrict__ pidx_b, Spc<T> H) {
     static_assert(OP == 0 || std::is_same<T, TX>::value, "a narrower x is for Fapply only");
     __shared__ T su[3][TS::RING];  // [ring slot][component][hy][hx], padded to RING
     // The nbb boundary workgroups (a multiple of kXcd, so that tile ib keeps
@@ -441,10 +442,6 @@ __global__ void __launch_bounds__(TS::NT)
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
-    const T ihx = T(1) / T(L.dx), ihy = T(1) / T(L.dy), ihz = T(1) / T(L.dz);
-    const T hx2 = T(0.5) * ihx, hy2 = T(0.5) * ihy, hz2 = T(0.5) * ihz;
-    const T ixx = ihx * ihx, iyy = ihy * ihy, izz = ihz * ihz;
-    const T ixy = T(0.25) * ihx * ihy, ixz = T(0.25) * ihx * ihz, iyz = T(0.25) * ihy * ihz;
     const int c0 = (ty + 1) * kHX + (tx + 1);  // centre position in the halo tile
 
     for (int kk = 0; kk < nstep; ++kk) {
@@ -499,15 +496,15 @@ __global__ void __launch_bounds__(TS::NT)
                 const T cc = uc[c0];
                 const T xp = uc[c0 + 1], xm = uc[c0 - 1], yp = uc[c0 + kHX], ym = uc[c0 - kHX];
                 const T zp = up[c0], zm = um[c0];
-                gu[p][0] = (xp - xm) * hx2;
-                gu[p][1] = (yp - ym) * hy2;
-                gu[p][2] = (zp - zm) * hz2;
-                B[p][0][0] = (xp - T(2) * cc + xm) * ixx;
-                B[p][1][1] = (yp - T(2) * cc + ym) * iyy;
-                B[p][2][2] = (zp - T(2) * cc + zm) * izz;
-                B[p][0][1] = (uc[c0 + 1 + kHX] + uc[c0 - 1 - kHX] - uc[c0 + 1 - kHX] - uc[c0 - 1 + kHX]) * ixy;
-                B[p][0][2] = (up[c0 + 1] + um[c0 - 1] - um[c0 + 1] - up[c0 - 1]) * ixz;
-                B[p][1][2] = (up[c0 + kHX] + um[c0 - kHX] - um[c0 + kHX] - up[c0 - kHX]) * iyz;
+                gu[p][0] = (xp - xm) * H.h2[0];
+                gu[p][1] = (yp - ym) * H.h2[1];
+                gu[p][2] = (zp - zm) * H.h2[2];
+                B[p][0][0] = (xp - T(2) * cc + xm) * H.ii[0];
+                B[p][1][1] = (yp - T(2) * cc + ym) * H.ii[1];
+                B[p][2][2] = (zp - T(2) * cc + zm) * H.ii[2];
+                B[p][0][1] = (uc[c0 + 1 + kHX] + uc[c0 - 1 - kHX] - uc[c0 + 1 - kHX] - uc[c0 - 1 + kHX]) * H.ixy;
+                B[p][0][2] = (up[c0 + 1] + um[c0 - 1] - um[c0 + 1] - up[c0 - 1]) * H.ixz;
+                B[p][1][2] = (up[c0 + kHX] + um[c0 - kHX] - um[c0 + kHX] - up[c0 - kHX]) * H.iyz;
                 B[p][1][0] = B[p][0][1];
                 B[p][2][0] = B[p][0][2];
                 B[p][2][1] = B[p][1][2];
@@ -526,7 +523,7 @@ __global__ void __launch_bounds__(TS::NT)
                 // Diagonal of an interior row, from the C already in registers
                 // instead of a load: (C : Gradient_Diagonal)_p = -2 sum_l C_plpl / h_l^2
                 // (src/Operator/Elastic.cpp:321-374, src/Numeric/Stencil.H:900-963).
-                const T m[3] = {T(-2) * ixx, T(-2) * iyy, T(-2) * izz};
+                const T m[3] = {T(-2) * H.ii[0], T(-2) * H.ii[1], T(-2) * H.ii[2]};
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
                     T d = T(0);
@@ -562,6 +559,171 @@ __global__ void __launch_bounds__(TS::NT)
         if (more) {
             __syncthreads();  // every read of slot sb (the plane behind) is done
             tile_store<TS, T>(su[sb], pre);
+            __syncthreads();
+        }
+    }
+}
+
+// --- Isotropic levels ------------------------------------------------------
+// The same march for an isotropic C: u, lambda and mu of three planes live in
+// LDS rings with a one-node halo, and each thread holds its share of plane k+2
+// of both in registers while plane k is computed.  The per-node kernel reads
+// 59 neighbour values a node through L1; a workgroup of it covers two rows, so
+// the rows and planes around them come from L2 about six times.  Here a plane
+// of a tile is read once per march (1.33 times with the halo), 40.8 KB of LDS
+// and at most 128 registers leave 4 workgroups a CU in FP64.  A Jacobi sweep
+// takes its interior diagonal from lambda and mu.  Boundary nodes as in
+// k_stencil_lds.  FP64 sweep: 31.7 us at 129 x 113 x 97 nodes (45.2 by node;
+// 88 B a node: 3.9 TB/s), 211 us at 201^3 (322; 3.4 TB/s, 4.2 with the halos).
+template <class TS, int NF>
+struct PlaneShare {
+    static constexpr int PRE = (NF * TS::HP + TS::NT - 1) / TS::NT;  // values per thread per plane of NF fields
+};
+template <class TS, int NF, typename T>
+__device__ __forceinline__ void plane_fetch(const T* __restrict__ u, const Lvl& L, int it, int jt, int k,
+                                            T pre[PlaneShare<TS, NF>::PRE]) {
+    const unsigned N = (unsigned)L.N, plane = (unsigned)k * (unsigned)(L.nx * L.ny);
+#pragma unroll
+    for (int m = 0; m < PlaneShare<TS, NF>::PRE; ++m) {  // clamped in-grid nodes, as in tile_fetch
+        const int q = min((int)threadIdx.x + m * TS::NT, NF * TS::HP - 1);
+        const int c = q / TS::HP, pos = q - c * TS::HP;
+        const int hy = pos / TS::HX, hx = pos - hy * TS::HX;
+        const int gi = min(it * TS::TX + hx, L.nx - 1), gj = min(jt * TS::TY + hy, L.ny - 1);
+        pre[m] = ld32(u, (unsigned)c * N + plane + (unsigned)(gj * L.nx + gi));
+    }
+}
+template <class TS, int NF, typename T>
+__device__ __forceinline__ void plane_store(T* __restrict__ s, const T pre[PlaneShare<TS, NF>::PRE]) {
+#pragma unroll
+    for (int m = 0; m < PlaneShare<TS, NF>::PRE; ++m) {
+        const int q = (int)threadIdx.x + m * TS::NT;
+        if ((m + 1) * TS::NT <= NF * TS::HP || q < NF * TS::HP) s[q] = pre[m];
+    }
+}
+template <class TS, typename T, int OP, bool PER = false>
+__global__ void __launch_bounds__(TS::NT)
+    k_stencil_iso(const T* __restrict__ x, const T* __restrict__ b, const T* __restrict__ diag, const T* __restrict__ C,
+                  const int* __restrict__ bct, int uniform, Lvl L, T omega, unsigned nbb, TileGrid G,
+                  T* __restrict__ out, Spc<T> H) {
+    constexpr int HX = TS::HX, HP = TS::HP;
+    __shared__ T su[3][3 * HP];  // [ring slot][component][hy][hx]
+    __shared__ T sc[3][2 * HP];  // lambda, mu
+    const unsigned ntb = gridDim.x - nbb;  // tile workgroups; the boundary ones come after them
+    if (blockIdx.x >= ntb) {
+        const long t = (long)(blockIdx.x - ntb) * blockDim.x + threadIdx.x;
+        if (t >= boundary_count(L)) return;
+        int i, j, k;
+        boundary_node(L, t, i, j, k);
+        const long id = ((long)k * L.ny + j) * L.nx + i;
+        T nrm[3], o[3];
+        const int reg = region_of<T, PER>(i, j, k, L, nrm);
+        if (!PER || reg >= 0) apply_boundary<T, 0, T, PER>(x, C, bct, L, i, j, k, id, reg, nrm, o);
+        else apply_interior_wrap<T, 0>(x, C, uniform, L, i, j, k, id, o);  // a periodic face
+        const unsigned n32 = (unsigned)id;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const size_t off = (size_t)p * L.N;
+            const T xv = (OP == 2) ? ld32(x + off, n32) : T(0);
+            const T bv = (OP >= 1) ? ld32(b + off, n32) : T(0);
+            const T dv = (OP == 2) ? ld32(diag + off, n32) : T(1);
+            st32(out + off, n32, finish_op<T, OP>(o[p], xv, bv, dv, omega));
+        }
+        return;
+    }
+    int it, jt, kc;
+    if (!tile_of(G, (long)blockIdx.x, it, jt, kc)) return;  // whole workgroup, before any barrier
+    const int tx = (int)threadIdx.x % TS::TX, ty = (int)threadIdx.x / TS::TX;
+    const int i = 1 + it * TS::TX + tx, j = 1 + jt * TS::TY + ty;
+    const bool valid = i <= L.nx - 2 && j <= L.ny - 2;
+    const int k0 = 1 + kc * G.kc, k1 = min(k0 + G.kc, L.nz - 1);  // planes [k0, k1)
+    const unsigned N = (unsigned)L.N, sxy = (unsigned)(L.nx * L.ny);
+    const unsigned col = (unsigned)(j * L.nx + i);
+    const int d = (kc & 1) ? 1 : -1;  // the march, as in k_stencil_lds
+    const int kfirst = d > 0 ? k0 : k1 - 1, nstep = k1 - k0;
+    T pu[PlaneShare<TS, 3>::PRE], pc[PlaneShare<TS, 2>::PRE];
+    {
+        T qu[3][PlaneShare<TS, 3>::PRE], qc[3][PlaneShare<TS, 2>::PRE];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            plane_fetch<TS, 3>(x, L, it, jt, kfirst + d * (s - 1), qu[s]);
+            plane_fetch<TS, 2>(C, L, it, jt, kfirst + d * (s - 1), qc[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            plane_store<TS, 3>(su[s], qu[s]);
+            plane_store<TS, 2>(sc[s], qc[s]);
+        }
+    }
+    __syncthreads();
+    const int c0 = (ty + 1) * HX + (tx + 1);  // centre position in the halo tile
+    for (int kk = 0; kk < nstep; ++kk) {
+        const int k = kfirst + d * kk;
+        const int sb = kk % 3, sn = (kk + 1) % 3, sa = (kk + 2) % 3;  // slots behind, centre, ahead
+        const int sm = d > 0 ? sb : sa, sp = d > 0 ? sa : sb;         // slots of planes k-1 and k+1
+        const bool more = kk + 1 < nstep;
+        const unsigned o = (unsigned)k * sxy + col;
+        // every global load of the plane leaves here, before the LDS work
+        T bv[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1 && valid) ? ld32(b + (size_t)p * N, o) : T(0);
+        if (more) {
+            plane_fetch<TS, 3>(x, L, it, jt, k + 2 * d, pu);
+            plane_fetch<TS, 2>(C, L, it, jt, k + 2 * d, pc);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (valid) {
+            // one component at a time (the barriers keep the compiler from
+            // reading all three's neighbours at once, which costs a wave a SIMD)
+            IsoD<T> D[3];
+            T cv[2][7], ov[3], dg[3];
+            const int nb[4] = {c0 + 1, c0 - 1, c0 + HX, c0 - HX};
+            const int xy[4] = {c0 + 1 + HX, c0 - 1 - HX, c0 + 1 - HX, c0 - 1 + HX};
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                const T *um = su[sm] + p * HP, *uc = su[sn] + p * HP, *up = su[sp] + p * HP;
+                T f[15];
+                f[0] = uc[c0];
+#pragma unroll
+                for (int n = 0; n < 4; ++n) f[1 + n] = uc[nb[n]];
+                f[5] = up[c0];
+                f[6] = um[c0];
+                const int m1 = p == 2 ? 7 : 11, m2 = 11;  // where xz (components 0, 2) and yz (1, 2) go
+                if (p < 2)
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) f[7 + n] = uc[xy[n]];
+                if (p != 1) {
+                    f[m1] = up[c0 + 1];
+                    f[m1 + 1] = um[c0 - 1];
+                    f[m1 + 2] = um[c0 + 1];
+                    f[m1 + 3] = up[c0 - 1];
+                }
+                if (p != 0) {
+                    f[m2] = up[c0 + HX];
+                    f[m2 + 1] = um[c0 - HX];
+                    f[m2 + 2] = um[c0 + HX];
+                    f[m2 + 3] = up[c0 - HX];
+                }
+                D[p] = iso_derivs<T>(p, f, H);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const T* cc = sc[sn] + s * HP;
+                cv[s][0] = cc[c0];
+#pragma unroll
+                for (int n = 0; n < 4; ++n) cv[s][1 + n] = cc[nb[n]];
+                cv[s][5] = sc[sp][s * HP + c0];
+                cv[s][6] = sc[sm][s * HP + c0];
+            }
+            iso_row<T>(D, cv, H, uniform != 0, ov, dg);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                st32(out + (size_t)p * N, o, finish_op<T, OP>(ov[p], su[sn][p * HP + c0], bv[p], dg[p], omega));
+        }
+        if (more) {
+            __syncthreads();  // every read of slot sb (the plane behind) is done
+            plane_store<TS, 3>(su[sb], pu);
+            plane_store<TS, 2>(sc[sb], pc);
             __syncthreads();
         }
     }
