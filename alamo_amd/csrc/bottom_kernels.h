@@ -165,38 +165,38 @@ __global__ void __launch_bounds__(kBottomBlock)
 // work on the node, which read vals[((r * kRowHalf + k) * N + node) * 2 + half].
 constexpr int kRowSlots = 58, kRowHalf = kRowSlots / 2;
 
-// One thread per node: its columns in ascending order from the dense operator
-// A (column-major, M x M).  A node with more than kRowSlots columns would
-// break the bound above: its values become NaN, which the solve reports.
+// One wave per node: its columns in ascending order from the dense operator A
+// (column-major, M x M), 64 candidates at a time.  A node with more than
+// kRowSlots columns would break the bound above: its values become NaN, which
+// the solve reports.
 __global__ void __launch_bounds__(64) k_bottom_rows(const double* __restrict__ A, const double* __restrict__ diag, int N,
                                                     double* __restrict__ vals, unsigned short* __restrict__ cols) {
-    const int node = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (node >= N) return;
-    const int M = 3 * N;
-    auto put = [&](int u, int c, double a0, double a1, double a2) {
+    const int node = (int)blockIdx.x, M = 3 * N, lane = (int)threadIdx.x;
+    const double d[3] = {diag[node], diag[N + node], diag[2 * N + node]};
+    auto put = [&](int u, int c, const double a[3]) {
         const int half = u / kRowHalf, k = u - half * kRowHalf;
         const long at = ((long)k * N + node) * 2 + half, plane = 2L * kRowHalf * N;
         cols[at] = (unsigned short)c;
-        vals[at] = a0 / diag[node];
-        vals[at + plane] = a1 / diag[N + node];
-        vals[at + 2 * plane] = a2 / diag[2 * N + node];
+        for (int r = 0; r < 3; ++r) vals[at + r * plane] = a[r];
     };
     int n = 0;
-#pragma unroll 8
-    for (int c = 0; c < M; ++c) {
-        const double* col = A + (long)c * M + node;
-        const double a0 = col[0], a1 = col[N], a2 = col[2 * N];
-        if (a0 == 0.0 && a1 == 0.0 && a2 == 0.0) continue;
-        if (n < kRowSlots) put(n, c, a0, a1, a2);
-        ++n;
+#pragma unroll 4
+    for (int c0 = 0; c0 < M; c0 += 64) {
+        const int c = c0 + lane;
+        double a[3];
+        for (int r = 0; r < 3; ++r) a[r] = c < M ? A[(long)c * M + r * N + node] : 0.0;
+        const bool have = a[0] != 0.0 || a[1] != 0.0 || a[2] != 0.0;
+        const unsigned long long bal = __ballot(have);
+        const int u = n + (int)__popcll(bal & (lane ? ~0ull >> (64 - lane) : 0ull));
+        if (have && u < kRowSlots) {
+            for (int r = 0; r < 3; ++r) a[r] /= d[r];
+            put(u, c, a);
+        }
+        n += (int)__popcll(bal);
     }
-    const double pad = n > kRowSlots ? __longlong_as_double(0x7ff8000000000000ll) : 0.0;
-    for (int u = n > kRowSlots ? 0 : n; u < kRowSlots; ++u) {
-        const int half = u / kRowHalf, k = u - half * kRowHalf;
-        const long at = ((long)k * N + node) * 2 + half, plane = 2L * kRowHalf * N;
-        cols[at] = (unsigned short)node;
-        vals[at] = vals[at + plane] = vals[at + 2 * plane] = pad;
-    }
+    const bool over = n > kRowSlots;
+    const double pad[3] = {over ? __longlong_as_double(0x7ff8000000000000ll) : 0.0, 0.0, 0.0};
+    for (int u = (over ? 0 : n) + lane; u < kRowSlots; u += 64) put(u, node, pad);
 }
 
 template <int CTRL>

@@ -133,7 +133,7 @@ struct alamo_el_s {
     double* csoa = nullptr;
     // dense coarsest level (when it has at most kDenseMax unknowns)
     int dense_M = 0;
-    double* dense_I = nullptr;     // identity, the unit vectors of the assembly
+    double* dense_I = nullptr;     // identity, the unit vectors of the assembly (the block's start)
     double* dense_A = nullptr;     // operator, column-major
     double* bottom_vals = nullptr; // its rows without the zeros, over the diagonal (k_bottom_rows)
     unsigned short* bottom_cols = nullptr;
@@ -680,14 +680,14 @@ int assemble_dense(alamo_el_t h, hipStream_t s) {
     const int M = (int)(3 * lb.L.N);
     if (M > kDenseMax) return 0;
     if (h->dense_M != M) {
-        for (void* p : {(void*)h->dense_I, (void*)h->dense_A, (void*)h->bottom_vals, (void*)h->bottom_cols})
-            if (p) (void)hipFree(p);
-        h->dense_I = h->dense_A = h->bottom_vals = nullptr;
-        h->bottom_cols = nullptr;
-        ALLOC(h->dense_I, (long)M * M);
-        ALLOC(h->bottom_vals, (long)ael::kRowSlots * M);
-        ALLOC(h->bottom_cols, (long)ael::kRowSlots * lb.L.N);
-        ALLOC(h->dense_A, (long)M * M);
+        // one block: the identity, the operator, its rows' values and columns
+        if (h->dense_I) (void)hipFree(h->dense_I);
+        h->dense_I = h->dense_A = nullptr;
+        const long MM = (long)M * M, R = (long)ael::kRowSlots * M;
+        ALLOC(h->dense_I, 2 * MM + R + (ael::kRowSlots * lb.L.N + 3) / 4);
+        h->dense_A = h->dense_I + MM;
+        h->bottom_vals = h->dense_A + MM;
+        h->bottom_cols = reinterpret_cast<unsigned short*>(h->bottom_vals + R);
         ael::k_eye<<<nblk((long)M * M), kBlock, 0, s>>>(h->dense_I, M);
         h->dense_M = M;
     }
@@ -698,8 +698,7 @@ int assemble_dense(alamo_el_t h, hipStream_t s) {
         default: ael::k_assemble_dense<2><<<grid, kBlock, 0, s>>>(h->dense_I, lb.d.C, h->bct_dev, h->uniform, lb.L, h->dense_A); break;
     }
     psi_post_columns(h, lb, h->dense_I, h->dense_A, M, s);
-    ael::k_bottom_rows<<<(unsigned)((lb.L.N + 63) / 64), 64, 0, s>>>(h->dense_A, lb.d.diag, (int)lb.L.N, h->bottom_vals,
-                                                                     h->bottom_cols);
+    ael::k_bottom_rows<<<(unsigned)lb.L.N, 64, 0, s>>>(h->dense_A, lb.d.diag, (int)lb.L.N, h->bottom_vals, h->bottom_cols);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1422,8 +1421,7 @@ int alamo_el_destroy(alamo_el_t h) {
     for (void* p : {(void*)h->bct_dev, (void*)h->bcv_dev, (void*)h->red_partial, (void*)h->red_out,
                     (void*)h->bottom_work, (void*)h->bottom_status, (void*)h->gu9, (void*)h->dw9, (void*)h->csoa,
                     (void*)h->kv, (void*)h->kz, (void*)h->kw, (void*)h->kh, (void*)h->kpart,
-                    (void*)h->dense_I, (void*)h->dense_A, (void*)h->bottom_vals,
-                    (void*)h->bottom_cols, (void*)h->nn_in, (void*)h->nn_out,
+                    (void*)h->dense_I, (void*)h->nn_in, (void*)h->nn_out,
                     (void*)h->nn_bc, (void*)h->nn_t, (void*)h->nn_fmean})
         if (p) (void)hipFree(p);
     if (h->red_host) (void)hipHostFree(h->red_host);
