@@ -505,11 +505,11 @@ __device__ __forceinline__ void apply_boundary(const TU* __restrict__ u, const T
     bc_set<T>(bct + 3 * reg, uu, gu, sg, nrm, out);
 }
 
-// Interior row of Fapply for an isotropic C = (lambda, mu):
-//   f_i = mu lap(u_i) + (lambda + mu) d_i(div u)
-//         + sum_a (d_a mu)(d_a u_i + d_i u_a) + (d_i lambda) div u,
-// the sums of contract3 and contract2_col with the terms that share a
-// derivative collected.  The operands at node o: of each component the centre,
+// Interior row of Fapply for an isotropic C = (lambda, mu), the sums of contract3
+// and contract2_col:
+//   f_i = sum_j (mu (d_j d_j u_i + d_i d_j u_j) + lambda d_i d_j u_j)
+//         + sum_a (d_a mu)(d_a u_i + d_i u_a) + (d_i lambda) div u.
+// The operands at node o: of each component the centre,
 // x+, x-, y+, y-, z+, z-, then the corners (++, --, +-, -+) of its two mixed
 // derivatives (component p has no use for the one without p): xy, xz | xy, yz |
 // xz, yz; and lambda, mu at the centre and its six neighbours (an axis along
@@ -538,37 +538,46 @@ __device__ __forceinline__ void iso_load(const T* __restrict__ u, const T* __res
 #pragma unroll
         for (int n = 0; n < 7; ++n) cv[s][n] = ld32(C + (size_t)s * N, nb[n]);
 }
-// What the row takes of component p: its gradient, d_p d_p u_p, its Laplacian
-// and its two mixed derivatives.
+// What the row takes of component p: its gradient, its second derivatives along
+// the axes and its two mixed derivatives.
 template <typename T>
 struct IsoD {
-    T g[3], dd, lap, m0, m1;
+    T g[3], d2[3], m0, m1;
 };
 template <typename T>
 __device__ __forceinline__ IsoD<T> iso_derivs(int p, const T f[15], const Spc<T>& H) {
     IsoD<T> r;
-    T d2[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         r.g[a] = (f[1 + 2 * a] - f[2 + 2 * a]) * H.h2[a];
-        d2[a] = (f[1 + 2 * a] - T(2) * f[0] + f[2 + 2 * a]) * H.ii[a];
+        r.d2[a] = (f[1 + 2 * a] - T(2) * f[0] + f[2 + 2 * a]) * H.ii[a];
     }
-    r.lap = d2[0] + d2[1] + d2[2];
-    r.dd = d2[p];
     r.m0 = (f[7] + f[8] - f[9] - f[10]) * (p == 2 ? H.ixz : H.ixy);
     r.m1 = (f[11] + f[12] - f[13] - f[14]) * (p == 0 ? H.ixz : H.iyz);
     return r;
 }
-// The row; dg: its diagonal, -2 (mu sum_l 1/h_l^2 + (lambda + mu) / h_i^2)
-// (Gradient_Diagonal through contract3).
+// The row, summed in the order of contract3 and contract2_col: the damped
+// Jacobi iteration is unstable on a sharp inclusion and magnifies a difference
+// in rounding, so the row keeps that of the reference's sums.  dg: its diagonal
+// (Gradient_Diagonal through contract3), in the order of k_diagonal.
 template <typename T>
 __device__ __forceinline__ void iso_row(const IsoD<T> D[3], const T cv[2][7], const Spc<T>& H, bool uniform, T out[3],
                                         T dg[3]) {
-    const T lam = cv[0][0], mu = cv[1][0], lm = lam + mu;
-    // d_i(div u): the xy derivatives of u_0 and u_1, the xz of u_0 and u_2, the yz of u_1 and u_2
-    const T dv[3] = {D[0].dd + D[1].m0 + D[2].m0, D[0].m0 + D[1].dd + D[2].m1, D[0].m1 + D[1].m1 + D[2].dd};
+    const T lam = cv[0][0], mu = cv[1][0];
+    // M[p][q]: the derivative of component p along axes p and q
+    const T M[3][3] = {{D[0].d2[0], D[0].m0, D[0].m1}, {D[1].m0, D[1].d2[1], D[1].m1}, {D[2].m0, D[2].m1, D[2].d2[2]}};
 #pragma unroll
-    for (int i = 0; i < 3; ++i) out[i] = mu * D[i].lap + lm * dv[i];
+    for (int i = 0; i < 3; ++i) {
+        T r = T(0), d = T(0);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            r += mu * (D[i].d2[j] + M[j][i]) + lam * M[j][i];
+            const T q = T(-2) * H.ii[j];
+            d += j == i ? mu * (q + q) + lam * q : mu * q;
+        }
+        out[i] = r;
+        dg[i] = d;
+    }
     if (!uniform) {
         const T tr = D[0].g[0] + D[1].g[1] + D[2].g[2];
 #pragma unroll
@@ -576,13 +585,9 @@ __device__ __forceinline__ void iso_row(const IsoD<T> D[3], const T cv[2][7], co
             const T gl = (cv[0][1 + 2 * a] - cv[0][2 + 2 * a]) * H.h2[a];
             const T gm = (cv[1][1 + 2 * a] - cv[1][2 + 2 * a]) * H.h2[a];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) out[i] += gm * (D[i].g[a] + D[a].g[i]);
-            out[a] += gl * tr;
+            for (int i = 0; i < 3; ++i) out[i] += gm * (D[i].g[a] + D[a].g[i]) + (i == a ? gl * tr : T(0));
         }
     }
-    const T s = mu * (H.ii[0] + H.ii[1] + H.ii[2]);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) dg[i] = T(-2) * (s + lm * H.ii[i]);
 }
 template <typename T>
 __device__ __forceinline__ void iso_compute(const T uv[3][15], const T cv[2][7], const Spc<T>& H, bool uniform, T out[3],

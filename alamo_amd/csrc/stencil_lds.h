@@ -601,7 +601,7 @@ __device__ __forceinline__ void plane_store(T* __restrict__ s, const T pre[Plane
     }
 }
 template <class TS, typename T, int OP, bool PER = false>
-__global__ void __launch_bounds__(TS::NT)
+__global__ void __launch_bounds__(TS::NT) __attribute__((amdgpu_waves_per_eu(4)))
     k_stencil_iso(const T* __restrict__ x, const T* __restrict__ b, const T* __restrict__ diag, const T* __restrict__ C,
                   const int* __restrict__ bct, int uniform, Lvl L, T omega, unsigned nbb, TileGrid G,
                   T* __restrict__ out, Spc<T> H) {
