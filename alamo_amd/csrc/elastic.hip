@@ -67,6 +67,12 @@ void launch_interp3(const T* crse, const T* held, const ael::Lvl& Lc, T* fine, c
         ael::k_interp_cell<T, false><<<nblk8(Lc.N), kBlock, 0, s>>>(crse, nullptr, Lc, fine, Lf, zero_first);
 }
 
+// Full weighting of ncomp components.
+template <typename T>
+void launch_restrict(const T* fine, const ael::Lvl& Lf, T* crse, const ael::Lvl& Lc, int ncomp, hipStream_t s) {
+    ael::k_restrict<T><<<dim3(nblk8(Lc.N), ncomp), kBlock, 0, s>>>(fine, Lf, crse, Lc);
+}
+
 int ncomp_of(int sym) { return sym == 0 ? 2 : (sym == 1 ? 21 : (sym == 2 ? 9 : -1)); }
 
 template <typename T>
@@ -494,14 +500,14 @@ struct Cycle {
     }
     void corr_res(int l, T* r, const T* x, const T* b) { launch_residual<T>(h, L(l), x, b, V(l).C, r, s); }
     void restrict_res(int lf, const T* fine, T* crse) {
-        ael::k_restrict<T><<<nblk8(L(lf + 1).L.N), kBlock, 0, s>>>(fine, L(lf).L, crse, L(lf + 1).L, 3);
+        launch_restrict<T>(fine, L(lf).L, crse, L(lf + 1).L, 3, s);
     }
     // restriction into V(lf + 1).res that also writes that level's first
     // Jacobi sweep from zero into its tmp
     void restrict_res_fz(int lf, const T* fine) {
         Vecs<T>& c = V(lf + 1);
-        ael::k_restrict_fz<T><<<nblk8(L(lf + 1).L.N), kBlock, 0, s>>>(fine, L(lf).L, c.res, L(lf + 1).L, 3, c.diag,
-                                                                      (T)h->omega, c.tmp);
+        ael::k_restrict_fz<T><<<dim3(nblk8(L(lf + 1).L.N), 3), kBlock, 0, s>>>(fine, L(lf).L, c.res, L(lf + 1).L, c.diag,
+                                                                               (T)h->omega, c.tmp);
     }
     void interp(int lf, T* fine, const T* crse, int zero_first) {
         launch_interp3<T>(crse, nullptr, L(lf + 1).L, fine, L(lf).L, zero_first, s);
@@ -1099,7 +1105,7 @@ int prepare(alamo_el_t h, hipStream_t s) {
     for (size_t l = 1; l < h->lv.size(); ++l) {
         Level& c = h->lv[l];
         Level& f = h->lv[l - 1];
-        ael::k_restrict<double><<<nblk8(c.L.N), kBlock, 0, s>>>(f.d.C, f.L, c.d.C, c.L, h->nc);
+        launch_restrict<double>(f.d.C, f.L, c.d.C, c.L, h->nc, s);
         int rc = build_gmask(h, c, s);
         if (rc) return rc;
         if (h->psi_set) {
@@ -1180,7 +1186,7 @@ int coarse_rhs(alamo_el_t h, int L, const double* b, double* bc, hipStream_t s) 
     const double* src = l0.d.tmp;
     for (int l = 1; l <= L; ++l) {
         double* dst = l == L ? bc : h->lv[l].d.tmp;
-        ael::k_restrict<double><<<nblk8(h->lv[l].L.N), kBlock, 0, s>>>(src, h->lv[l - 1].L, dst, h->lv[l].L, 3);
+        launch_restrict<double>(src, h->lv[l - 1].L, dst, h->lv[l].L, 3, s);
         src = dst;
     }
     ael::k_inject_boundary<<<nblk(h->lv[L].L.N), kBlock, 0, s>>>(b, l0.L, 1 << L, bc, h->lv[L].L);
@@ -1654,8 +1660,7 @@ int alamo_el_residual(alamo_el_t h, int mglev, const double* x, const double* b,
 
 int alamo_el_restrict(alamo_el_t h, int cmglev, double* crse, const double* fine, hipStream_t s) {
     if (bad_level(h, cmglev) || cmglev == 0 || !crse || !fine) return fail(ALAMO_EL_EINVAL, "bad argument");
-    ael::k_restrict<double><<<nblk8(h->lv[cmglev].L.N), kBlock, 0, s>>>(fine, h->lv[cmglev - 1].L, crse,
-                                                                        h->lv[cmglev].L, 3);
+    launch_restrict<double>(fine, h->lv[cmglev - 1].L, crse, h->lv[cmglev].L, 3, s);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1683,7 +1688,7 @@ int alamo_el_level_op32(alamo_el_t h, int mglev, int op, const float* x, const f
         case 1: launch_residual<float>(h, l, x, b, l.f.C, out, s); break;
         case 2: launch_jacobi<float>(h, l, x, b, l.f.diag, l.f.C, out, s); break;
         case 3:
-            ael::k_restrict<float><<<nblk8(h->lv[mglev + 1].L.N), kBlock, 0, s>>>(x, l.L, out, h->lv[mglev + 1].L, 3);
+            launch_restrict<float>(x, l.L, out, h->lv[mglev + 1].L, 3, s);
             break;
         default:
             launch_interp3<float>(x, nullptr, h->lv[mglev + 1].L, out, l.L, 0, s);

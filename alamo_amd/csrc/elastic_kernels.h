@@ -794,75 +794,82 @@ __global__ void __launch_bounds__(kBlock) k_diagonal(const T* __restrict__ C, co
     }
 }
 
-// Nodal full-weighting restriction of ncomp components from level Lf to Lc
-// (src/Operator/Operator.cpp:280-353); the same weights average C between MG
-// levels (src/Operator/Elastic.cpp:786-834).
-// NC > 0 fixes the component count at compile time: the loop unrolls and
-// every component's loads are issued before the first one's arithmetic (the
-// coarse levels' launches are set by that latency, not by their bytes).
-template <typename T, bool WRAP, int NC = 0>
-__device__ __forceinline__ void restrict_node_w(const T* __restrict__ fine, const Lvl& Lf, T* __restrict__ crse,
-                                                const Lvl& Lc, int ncomp, long cid) {
-    int I, J, K;
-    node_ijk(cid, Lc, I, J, K);
-    const int hx = Lc.nx - 1, hy = Lc.ny - 1, hz = Lc.nz - 1;
-    // faces of a periodic axis take the full weights, their fine neighbours
-    // across the face wrapped (the coarse domain is grown there,
-    // src/Operator/Operator.cpp:268)
-    const bool px = WRAP && (Lc.per & 1), py = WRAP && ((Lc.per >> 1) & 1), pz = WRAP && ((Lc.per >> 2) & 1);
-    const bool bi = !px && (I == 0 || I == hx), bj = !py && (J == 0 || J == hy), bk = !pz && (K == 0 || K == hz);
-    const long sy = Lf.nx, sz = (long)Lf.nx * Lf.ny;
-    // the fine node's -1 and +1 neighbours, wrapped on a periodic axis
-    long om[3] = {-1, -sy, -sz}, op[3] = {1, sy, sz};
-    if constexpr (WRAP) nb_offsets(Lf, 2 * I, 2 * J, 2 * K, om, op);
-    const long x1m = om[0], x1p = op[0], sym = om[1], syp = op[1], szm = om[2], szp = op[2];
-    const long f0 = (2L * K) * sz + (2L * J) * sy + 2L * I;
-    const int nc = NC > 0 ? NC : ncomp;
-    T vout[NC > 0 ? NC : 1];
-#pragma unroll
-    for (int n = 0; n < nc; ++n) {
-        const T* F = fine + n * Lf.N + f0;
-        T v;
-        if (bi && bj && bk) v = F[0];
-        else if (bj && bk) v = T(0.25) * F[x1m] + T(0.5) * F[0] + T(0.25) * F[x1p];
-        else if (bk && bi) v = T(0.25) * F[sym] + T(0.5) * F[0] + T(0.25) * F[syp];
-        else if (bi && bj) v = T(0.25) * F[szm] + T(0.5) * F[0] + T(0.25) * F[szp];
-        else if (bi)
-            v = (+F[sym + szm] + T(2) * F[szm] + F[syp + szm] + T(2) * F[sym] + T(4) * F[0] + T(2) * F[syp] +
-                 F[sym + szp] + T(2) * F[szp] + F[syp + szp]) / T(16);
-        else if (bj)
-            v = (+F[x1m + szm] + T(2) * F[x1m] + F[x1m + szp] + T(2) * F[szm] + T(4) * F[0] + T(2) * F[szp] +
-                 F[x1p + szm] + T(2) * F[x1p] + F[x1p + szp]) / T(16);
-        else if (bk)
-            v = (+F[x1m + sym] + T(2) * F[sym] + F[x1p + sym] + T(2) * F[x1m] + T(4) * F[0] + T(2) * F[x1p] +
-                 F[x1m + syp] + T(2) * F[syp] + F[x1p + syp]) / T(16);
-        else
-            v = (F[x1m + sym + szm] + F[x1m + sym + szp] + F[x1m + syp + szm] + F[x1m + syp + szp] +
-                 F[x1p + sym + szm] + F[x1p + sym + szp] + F[x1p + syp + szm] + F[x1p + syp + szp]) / T(64) +
-                (F[sym + szm] + F[sym + szp] + F[syp + szm] + F[syp + szp] + F[x1m + szm] + F[x1p + szm] +
-                 F[x1m + szp] + F[x1p + szp] + F[x1m + sym] + F[x1m + syp] + F[x1p + sym] + F[x1p + syp]) / T(32) +
-                (F[x1m] + F[sym] + F[szm] + F[x1p] + F[syp] + F[szp]) / T(16) + F[0] / T(8);
-        if constexpr (NC > 0) vout[n] = v;
-        else crse[n * Lc.N + cid] = v;
-    }
-    if constexpr (NC > 0) {
-#pragma unroll
-        for (int n = 0; n < NC; ++n) crse[n * Lc.N + cid] = vout[n];
-    }
-}
-template <typename T, int NC = 0>
-__device__ __forceinline__ void restrict_node(const T* __restrict__ fine, const Lvl& Lf, T* __restrict__ crse,
-                                              const Lvl& Lc, int ncomp, long cid) {
-    if (Lc.per) restrict_node_w<T, true, NC>(fine, Lf, crse, Lc, ncomp, cid);
-    else restrict_node_w<T, false, NC>(fine, Lf, crse, Lc, ncomp, cid);
+// The nodal full weighting of the 27 values v[k][j][i] around a fine node, b[a]
+// set where the node lies on a face normal to axis a (the values across it are
+// not used): the interior, face, edge and corner sums of the reference
+// (src/Operator/Operator.cpp:280-353), each in the reference's order, chosen
+// without a branch.  The order matters: the damped Jacobi iteration is unstable
+// on a sharp inclusion and magnifies differences in rounding.
+template <typename T>
+__device__ __forceinline__ T pick(bool c, T a, T b) {  // by value: a conditional of array elements would select addresses
+    return c ? a : b;
 }
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_restrict(const T* __restrict__ fine, Lvl Lf, T* __restrict__ crse,
-                                                     Lvl Lc, int ncomp) {
+__device__ __forceinline__ T full_weight(const T v[3][3][3], const bool b[3]) {
+    const T inner =
+        (v[0][0][0] + v[2][0][0] + v[0][2][0] + v[2][2][0] + v[0][0][2] + v[2][0][2] + v[0][2][2] + v[2][2][2]) / T(64) +
+        (v[0][0][1] + v[2][0][1] + v[0][2][1] + v[2][2][1] + v[0][1][0] + v[0][1][2] + v[2][1][0] + v[2][1][2] +
+         v[1][0][0] + v[1][2][0] + v[1][0][2] + v[1][2][2]) / T(32) +
+        (v[1][1][0] + v[1][0][1] + v[0][1][1] + v[1][1][2] + v[1][2][1] + v[2][1][1]) / T(16) + v[1][1][1] / T(8);
+    // the face's values q[outer][inner]: (z, y) on an x face, (x, z) on a y face, (y, x) on a z face
+    T q[3][3];
+#pragma unroll
+    for (int o = 0; o < 3; ++o)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) q[o][i] = pick(b[0], v[o][i][1], pick(b[1], v[i][1][o], v[1][o][i]));
+    const T face = (q[0][0] + T(2) * q[0][1] + q[0][2] + T(2) * q[1][0] + T(4) * q[1][1] + T(2) * q[1][2] + q[2][0] +
+                    T(2) * q[2][1] + q[2][2]) / T(16);
+    const T em = pick(b[0], pick(b[1], v[0][1][1], v[1][0][1]), v[1][1][0]);
+    const T ep = pick(b[0], pick(b[1], v[2][1][1], v[1][2][1]), v[1][1][2]);
+    const T edge = T(0.25) * em + T(0.5) * v[1][1][1] + T(0.25) * ep;
+    const int n = (int)b[0] + (int)b[1] + (int)b[2];
+    return pick(n == 0, inner, pick(n == 1, face, pick(n == 2, edge, v[1][1][1])));
+}
+// Nodal full-weighting restriction from level Lf to Lc; the same weights average
+// C between MG levels (src/Operator/Elastic.cpp:786-834).  The value of one
+// component (F: its fine field) at coarse node cid.  Every node loads 27 values
+// (a position beyond a face reads the node's own, unused): a wave with corners,
+// edges, faces and interior nodes in it ran all eight formulas, each with a
+// memory round trip of its own.  The faces of a periodic axis (WRAP) take the
+// full weights, their fine neighbours across the face wrapped (the coarse domain
+// is grown there, src/Operator/Operator.cpp:268).
+template <typename T, bool WRAP>
+__device__ __forceinline__ T restrict_value(const T* __restrict__ F, const Lvl& Lf, const Lvl& Lc, long cid) {
+    int pos[3];
+    node_ijk(cid, Lc, pos[0], pos[1], pos[2]);
+    const int nc[3] = {Lc.nx, Lc.ny, Lc.nz};
+    const int st[3] = {1, Lf.nx, Lf.nx * Lf.ny};
+    int off[3][3];
+    bool b[3];
+    long wm[3], wp[3];
+    if constexpr (WRAP) nb_offsets(Lf, 2 * pos[0], 2 * pos[1], 2 * pos[2], wm, wp);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        b[a] = !(WRAP && ((Lc.per >> a) & 1)) && (pos[a] == 0 || pos[a] == nc[a] - 1);
+        off[a][0] = b[a] ? 0 : WRAP ? (int)wm[a] : -st[a];
+        off[a][1] = 0;
+        off[a][2] = b[a] ? 0 : WRAP ? (int)wp[a] : st[a];
+    }
+    const int f0 = 2 * (pos[0] + pos[1] * st[1] + pos[2] * st[2]);
+    T v[3][3][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) v[k][j][i] = ld32(F, (unsigned)(f0 + off[2][k] + off[1][j] + off[0][i]));
+    return full_weight<T>(v, b);
+}
+// One thread per coarse node and component (blockIdx.y).  Average over the
+// levels below 65^3 nodes, with the first sweep, FP64: 8.2 us with one thread for
+// the three components and a branch per kind of node, 3.2 us now; FP32, levels
+// below 129^3: 9.1 and 7.5 us.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_restrict(const T* __restrict__ fine, Lvl Lf, T* __restrict__ crse, Lvl Lc) {
     const long cid = xcd_node();
     if (cid >= Lc.N) return;
-    if (ncomp == 3) restrict_node<T, 3>(fine, Lf, crse, Lc, 3, cid);
-    else restrict_node<T>(fine, Lf, crse, Lc, ncomp, cid);
+    const T* F = fine + (size_t)blockIdx.y * Lf.N;
+    crse[blockIdx.y * Lc.N + cid] = Lc.per ? restrict_value<T, true>(F, Lf, Lc, cid) : restrict_value<T, false>(F, Lf, Lc, cid);
 }
 
 // Restriction followed by the first Jacobi sweep from zero on the coarse
@@ -870,24 +877,16 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const T* __restrict__ fine,
 // values), in one launch.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_restrict_fz(const T* __restrict__ fine, Lvl Lf, T* __restrict__ crse,
-                                                        Lvl Lc, int ncomp, const T* __restrict__ diag, T omega,
+                                                        Lvl Lc, const T* __restrict__ diag, T omega,
                                                         T* __restrict__ tmp) {
     const long cid = xcd_node();
     if (cid >= Lc.N) return;
-    if (ncomp == 3) {
-        restrict_node<T, 3>(fine, Lf, crse, Lc, 3, cid);
-#pragma unroll
-        for (int n = 0; n < 3; ++n) {
-            const long q = n * Lc.N + cid;
-            tmp[q] = omega * crse[q] / diag[q];
-        }
-        return;
-    }
-    restrict_node<T>(fine, Lf, crse, Lc, ncomp, cid);
-    for (int n = 0; n < ncomp; ++n) {
-        const long q = n * Lc.N + cid;
-        tmp[q] = omega * crse[q] / diag[q];
-    }
+    const T* F = fine + (size_t)blockIdx.y * Lf.N;
+    const long q = blockIdx.y * Lc.N + cid;
+    const T d = diag[q];
+    const T v = Lc.per ? restrict_value<T, true>(F, Lf, Lc, cid) : restrict_value<T, false>(F, Lf, Lc, cid);
+    crse[q] = v;
+    tmp[q] = omega * v / d;
 }
 
 // Nodal injection crse(I,J,K) = fine(2I,2J,2K): amrex::average_down on nodal
