@@ -8,7 +8,7 @@
 // interpolated from the parent level (the "ghostnodes" coarse-fine
 // treatment), the nodes 2 clo .. 2 chi are the patch's unknowns.
 #pragma once
-#include "elastic_kernels.h"
+#include "stencil.h"
 
 namespace ael {
 
@@ -77,16 +77,19 @@ __global__ void __launch_bounds__(kBlock) k_tag_cells(const double* __restrict__
     tags[((long)k * (L.ny - 1) + j) * (L.nx - 1) + i] = eta_tagged(eta, ncomp, L, thr, id, i, j, k) ? 1 : 0;
 }
 
-// v = 0 on ghost nodes (mode 0) or v = src on ghost nodes (mode 1).
+// v = 0 on ghost nodes (src null) or v = src on ghost nodes.  One thread per
+// node on the handle's faces (a launch over the whole patch only to find its
+// shell took 16 us on average over the patches of a three-level solve, this 6).
 __global__ void __launch_bounds__(kBlock) k_patch_ghost(double* __restrict__ v, const double* __restrict__ src, Lvl L,
-                                                        Patch P, int mode) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= L.N) return;
+                                                        Patch P) {
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= boundary_count(L)) return;
     int i, j, k;
-    node_ijk(id, L, i, j, k);
+    boundary_node(L, t, i, j, k);
     if (!ghost_node(L, P, i, j, k)) return;
+    const long id = ((long)k * L.ny + j) * L.nx + i;
 #pragma unroll
-    for (int p = 0; p < 3; ++p) v[p * L.N + id] = mode ? src[p * L.N + id] : 0.0;
+    for (int p = 0; p < 3; ++p) v[p * L.N + id] = src ? src[p * L.N + id] : 0.0;
 }
 
 // Trilinear value of component p of the parent field c (level Lc, whole
@@ -106,22 +109,67 @@ __device__ __forceinline__ double parent_trilinear(const double* __restrict__ c,
     return acc * w;
 }
 
-// Trilinear interpolation of the parent field c onto the patch handle field f:
-// mode 0: f = P c everywhere, mode 1: f += P c everywhere, mode 2: f = P c on
-// ghost nodes only.
-__global__ void __launch_bounds__(kBlock) k_patch_interp(const double* __restrict__ c, Lvl Lc, int pox, int poy,
-                                                         int poz, double* __restrict__ f, Lvl Lf, Patch P, int mode) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= Lf.N) return;
+// f = P c on the patch's ghost nodes (P c: the trilinear interpolation of the
+// parent field c).  One thread per node on the handle's faces.
+__global__ void __launch_bounds__(kBlock) k_patch_interp_ghost(const double* __restrict__ c, Lvl Lc, int pox, int poy,
+                                                               int poz, double* __restrict__ f, Lvl Lf, Patch P) {
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= boundary_count(Lf)) return;
     int i, j, k;
-    node_ijk(id, Lf, i, j, k);
-    if (mode == 2 && !ghost_node(Lf, P, i, j, k)) return;
+    boundary_node(Lf, t, i, j, k);
+    if (!ghost_node(Lf, P, i, j, k)) return;
+    const long id = ((long)k * Lf.ny + j) * Lf.nx + i;
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
-        const double acc = parent_trilinear(c, Lc, pox, poy, poz, P.ox + i, P.oy + j, P.oz + k, p);
-        double* q = f + p * Lf.N + id;
-        *q = mode == 1 ? *q + acc : acc;
+    for (int p = 0; p < 3; ++p)
+        f[p * Lf.N + id] = parent_trilinear(c, Lc, pox, poy, poz, P.ox + i, P.oy + j, P.oz + k, p);
+}
+
+// f += P c on the whole patch, by parent cell as k_interp_cell: a thread loads
+// the 8 parent values of its cell and adds to the up to 8 fine nodes 2I + a of
+// it that the handle holds (its node 0 may be odd: a ghost layer).  (nbx, nby,
+// nbz): parent cells the handle's nodes touch, from parent node (P.ox >> 1, ..).
+// One thread per fine node, its loads in loops over the parity, took 90 us on
+// average over the patches of a three-level solve; this takes 57.
+__global__ void __launch_bounds__(kBlock) k_patch_interp_add(const double* __restrict__ c, Lvl Lc, int pox, int poy,
+                                                             int poz, double* __restrict__ f, Lvl Lf, Patch P, int nbx,
+                                                             int nby, int nbz) {
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (unsigned)nbx * nby * nbz) return;
+    const unsigned q = t / nbx;
+    const int I = (P.ox >> 1) + (int)(t - q * nbx), K = (P.oz >> 1) + (int)(q / nby), J = (P.oy >> 1) + (int)(q % nby);
+    // the fine nodes 2I, 2I + 1 (and of the other axes) that the handle holds
+    const int fi = 2 * I - P.ox, fj = 2 * J - P.oy, fk = 2 * K - P.oz;
+    const bool hx[2] = {fi >= 0, fi + 1 < Lf.nx}, hy[2] = {fj >= 0, fj + 1 < Lf.ny}, hz[2] = {fk >= 0, fk + 1 < Lf.nz};
+    // the parent node above is read only where the handle holds an odd node (it exists then)
+    const long ox = hx[1] ? 1 : 0, oy = hy[1] ? Lc.nx : 0, oz = hz[1] ? (long)Lc.nx * Lc.ny : 0;
+    const long c0 = ((long)(K - poz) * Lc.ny + (J - poy)) * Lc.nx + (I - pox);
+    const long sy = Lf.nx, sz = (long)Lf.nx * Lf.ny, f0 = (long)fk * sz + (long)fj * sy + fi;
+    double v[3][8], old[3][8];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const double* g = c + n * Lc.N + c0;
+        const double c000 = g[0], c100 = g[ox], c010 = g[oy], c001 = g[oz], c011 = g[oy + oz], c101 = g[ox + oz],
+                     c110 = g[ox + oy], c111 = g[ox + oy + oz];
+        v[n][0] = c000;
+        v[n][1] = 0.5 * (c000 + c100);
+        v[n][2] = 0.5 * (c000 + c010);
+        v[n][3] = 0.25 * (c000 + c100 + c010 + c110);
+        v[n][4] = 0.5 * (c000 + c001);
+        v[n][5] = 0.25 * (c000 + c100 + c001 + c101);
+        v[n][6] = 0.25 * (c000 + c010 + c001 + c011);
+        v[n][7] = 0.125 * (c000 + c100 + c010 + c110 + c001 + c101 + c011 + c111);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const bool ex = hx[e & 1] && hy[(e >> 1) & 1] && hz[e >> 2];
+            old[n][e] = ex ? f[n * Lf.N + f0 + (e & 1) + ((e >> 1) & 1) * sy + (e >> 2) * sz] : 0.0;
+        }
     }
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (hx[e & 1] && hy[(e >> 1) & 1] && hz[e >> 2])
+                f[n * Lf.N + f0 + (e & 1) + ((e >> 1) & 1) * sy + (e >> 2) * sz] = old[n][e] + v[n][e];
 }
 
 // FillPatchTwoLevels with node_bilinear_interp (src/Integrator/Integrator.cpp:
@@ -163,14 +211,53 @@ __global__ void __launch_bounds__(kBlock) k_patch_inject(const double* __restric
 
 // Operator::reflux (src/Operator/Operator.cpp:526-633): the parent residual
 // at the nodes clo..chi (covered and coarse-fine nodes) is replaced by the
-// full-weighting restriction of the patch residual.  At a domain face the
-// stencil falls back to the face, edge and corner weights of the MG
-// restriction (Operator.cpp:280-353), since no fine node exists outside the
-// domain; inside the domain the fine ghost layer supplies the outer nodes.
-// The same restriction of the ncomp planes of a patch's C onto its parent's
-// is Elastic::averageDownCoeffsDifferentAmrLevels (Elastic.cpp:628-745,
-// whose corner, edge, face and interior weights are these).
+// full-weighting restriction of the patch residual, its ghost layer read as 0.
+// At a domain face the stencil falls back to the face, edge and corner weights
+// of the MG restriction (Operator.cpp:280-353), since no fine node exists
+// outside the domain.  One thread per node and component (blockIdx.y), the loads
+// without branches as in restrict_value; it reads the patch once, 24 B a node.
 __global__ void __launch_bounds__(kBlock) k_patch_reflux(const double* __restrict__ rf, Lvl Lf, Patch P,
+                                                         double* __restrict__ rc, Lvl Lc, int pox, int poy, int poz,
+                                                         int dnx, int dny, int dnz) {
+    const unsigned nx = P.chi[0] - P.clo[0] + 1, ny = P.chi[1] - P.clo[1] + 1, nz = P.chi[2] - P.clo[2] + 1;
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nx * ny * nz) return;
+    const unsigned q = t / nx;
+    const int d[3] = {(int)(t - q * nx), (int)(q % ny), (int)(q / ny)};
+    const int g[3] = {P.clo[0] + d[0], P.clo[1] + d[1], P.clo[2] + d[2]};  // global parent node
+    const int dn[3] = {dnx, dny, dnz};
+    const int st[3] = {1, Lf.nx, Lf.nx * Lf.ny};
+    int off[3][3];
+    bool b[3], keep[3][3];  // keep: false where the position along the axis is in the ghost layer
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        b[a] = g[a] == 0 || g[a] == dn[a];  // a domain face: no fine node beyond it
+        off[a][0] = b[a] ? 0 : -st[a];
+        off[a][1] = 0;
+        off[a][2] = b[a] ? 0 : st[a];
+        keep[a][0] = b[a] || g[a] != P.clo[a];
+        keep[a][1] = true;
+        keep[a][2] = b[a] || g[a] != P.chi[a];
+    }
+    const double* F = rf + blockIdx.y * Lf.N + ((long)(2 * g[2] - P.oz) * Lf.ny + (2 * g[1] - P.oy)) * Lf.nx +
+                      (2 * g[0] - P.ox);
+    double v[3][3][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double f = F[off[2][k] + off[1][j] + off[0][i]];
+                v[k][j][i] = keep[2][k] && keep[1][j] && keep[0][i] ? f : 0.0;
+            }
+    rc[blockIdx.y * Lc.N + ((long)(g[2] - poz) * Lc.ny + (g[1] - poy)) * Lc.nx + (g[0] - pox)] = full_weight<double>(v, b);
+}
+
+// Elastic::averageDownCoeffsDifferentAmrLevels (Elastic.cpp:628-745): the same
+// restriction of the ncomp planes of a patch's C, ghost layer included, onto its
+// parent's, in the order of the reference's sums.
+__global__ void __launch_bounds__(kBlock) k_patch_average(const double* __restrict__ rf, Lvl Lf, Patch P,
                                                          double* __restrict__ rc, Lvl Lc, int pox, int poy, int poz,
                                                          int dnx, int dny, int dnz, int ncomp) {
     const int nx = P.chi[0] - P.clo[0] + 1, ny = P.chi[1] - P.clo[1] + 1, nz = P.chi[2] - P.clo[2] + 1;
@@ -227,18 +314,40 @@ __global__ void __launch_bounds__(kBlock) k_box_copy(double* __restrict__ dst, i
     for (int p = 0; p < ncomp; ++p) dst[p * Nd + di] = src[p * Ns + si];
 }
 
-// out = v with the parent nodes strictly inside the patch (covered by the
-// finer level, excluded from the composite norm) set to 0.
-__global__ void __launch_bounds__(kBlock) k_mask_covered(const double* v, Lvl L, int pox, int poy, int poz, Patch P,
-                                                         double* out) {  // out may be v
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= L.N) return;
-    int i, j, k;
-    node_ijk(id, L, i, j, k);
-    const int I = pox + i, J = poy + j, K = poz + k;
-    const bool covered = I > P.clo[0] && I < P.chi[0] && J > P.clo[1] && J < P.chi[1] && K > P.clo[2] && K < P.chi[2];
+__device__ __forceinline__ double max_nan(double a, double b) { return (isnan(a) || isnan(b)) ? NAN : fmax(a, b); }
+
+// Partial max-norms of one handle's field over the composite grid: its ghost
+// nodes and the nodes strictly inside one of its nkid children (covered by the
+// finer level) excluded; NaN propagates.  part[blockIdx.x] of each launch.
+__global__ void __launch_bounds__(kBlock) k_composite_max(const double* __restrict__ v, Lvl L, Patch P,
+                                                          const Patch* __restrict__ kid, int nkid,
+                                                          double* __restrict__ part) {
+    __shared__ double sh[kBlock / 64];
+    double m = 0.0;
+    const unsigned N = (unsigned)L.N;
+    for (unsigned id = blockIdx.x * blockDim.x + threadIdx.x; id < N; id += gridDim.x * blockDim.x) {
+        int i, j, k;
+        node_ijk(id, L, i, j, k);
+        double a[3];
 #pragma unroll
-    for (int p = 0; p < 3; ++p) out[p * L.N + id] = covered ? 0.0 : v[p * L.N + id];
+        for (int p = 0; p < 3; ++p) a[p] = fabs(v[(size_t)p * N + id]);
+        bool out = ghost_node(L, P, i, j, k);
+        const int I = P.ox + i, J = P.oy + j, K = P.oz + k;
+        for (int c = 0; c < nkid; ++c)
+            out |= I > kid[c].clo[0] && I < kid[c].chi[0] && J > kid[c].clo[1] && J < kid[c].chi[1] &&
+                   K > kid[c].clo[2] && K < kid[c].chi[2];
+        if (out) continue;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) m = max_nan(m, a[p]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = max_nan(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) m = max_nan(m, sh[w]);
+        part[blockIdx.x] = m;
+    }
 }
 
 }  // namespace ael

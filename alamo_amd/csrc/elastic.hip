@@ -177,6 +177,9 @@ struct alamo_el_s {
     // AMR placement (alamo_amr_patch_create); a base handle has no parent
     alamo_el_t amr_parent = nullptr;
     int amr_dom[3] = {0, 0, 0};  // domain cells at this handle's level
+    ael::Patch* amr_kids = nullptr;  // the composite solve's children lists and partial norms (base handle)
+    double* amr_part = nullptr;
+    int amr_cap = 0;                 // handles they are sized for
     ael::Patch amr{};            // origin and covered parent cells (origin 0 for a base handle)
 };
 
@@ -1427,7 +1430,7 @@ int alamo_el_destroy(alamo_el_t h) {
     for (void* p : {(void*)h->bct_dev, (void*)h->bcv_dev, (void*)h->red_partial, (void*)h->red_out,
                     (void*)h->bottom_work, (void*)h->bottom_status, (void*)h->gu9, (void*)h->dw9, (void*)h->csoa,
                     (void*)h->kv, (void*)h->kz, (void*)h->kw, (void*)h->kh, (void*)h->kpart,
-                    (void*)h->dense_I, (void*)h->nn_in, (void*)h->nn_out,
+                    (void*)h->dense_I, (void*)h->amr_kids, (void*)h->amr_part, (void*)h->nn_in, (void*)h->nn_out,
                     (void*)h->nn_bc, (void*)h->nn_t, (void*)h->nn_fmean})
         if (p) (void)hipFree(p);
     if (h->red_host) (void)hipHostFree(h->red_host);
@@ -2385,8 +2388,15 @@ void region_faces(int r, bool f[6]) {
     f[(c & 1) ? 5 : 2] = true;
 }
 
-int amr_reduce_max(alamo_el_t h, const double* v, long n, double* out, hipStream_t s) {
-    return reduce_host<double>(h, v, v, n, 0, out, s);
+// The residual fine_res of a patch (its ghost layer read as 0) into its
+// parent's field.
+void launch_reflux(alamo_el_t patch, const double* fine_res, double* parent_res, hipStream_t s) {
+    const ael::Patch& P = patch->amr;
+    const alamo_el_t par = patch->amr_parent;
+    const long m = (long)(P.chi[0] - P.clo[0] + 1) * (P.chi[1] - P.clo[1] + 1) * (P.chi[2] - P.clo[2] + 1);
+    ael::k_patch_reflux<<<dim3(nblk(m), 3), kBlock, 0, s>>>(fine_res, patch->lv[0].L, P, parent_res, par->lv[0].L,
+                                                            par->amr.ox, par->amr.oy, par->amr.oz, par->amr_dom[0],
+                                                            par->amr_dom[1], par->amr_dom[2]);
 }
 
 // The handles of a composite solve: h[0] is the base, every other handle a
@@ -2430,21 +2440,24 @@ struct AmrCtx {
     Level& L(int i) { return h[i]->lv[0]; }
     const ael::Patch& P(int i) { return h[i]->amr; }
 
-    void reflux(int i, const double* rf, double* rc) {  // patch i into its parent
-        const ael::Patch& Pi = P(i);
+    void reflux(int i, const double* rf, double* rc) { launch_reflux(h[i], rf, rc, s); }  // patch i into its parent
+    // f += P c on patch i, c its parent's field
+    void interp_add(int i, const double* c, double* f) {
         const int q = par[i];
-        const long m = (long)(Pi.chi[0] - Pi.clo[0] + 1) * (Pi.chi[1] - Pi.clo[1] + 1) * (Pi.chi[2] - Pi.clo[2] + 1);
-        const int* dom = h[q]->amr_dom;
-        ael::k_patch_reflux<<<nblk(m), kBlock, 0, s>>>(rf, L(i).L, Pi, rc, L(q).L, P(q).ox, P(q).oy, P(q).oz, dom[0],
-                                                        dom[1], dom[2], 3);
+        const ael::Patch& p = P(i);
+        const Lvl& Lf = L(i).L;
+        const int nb[3] = {((p.ox + Lf.nx - 1) >> 1) - (p.ox >> 1) + 1, ((p.oy + Lf.ny - 1) >> 1) - (p.oy >> 1) + 1,
+                           ((p.oz + Lf.nz - 1) >> 1) - (p.oz >> 1) + 1};
+        ael::k_patch_interp_add<<<nblk((long)nb[0] * nb[1] * nb[2]), kBlock, 0, s>>>(c, L(q).L, P(q).ox, P(q).oy, P(q).oz,
+                                                                                     f, Lf, p, nb[0], nb[1], nb[2]);
     }
-    void interp(int i, const double* c, double* f, int mode) {
+    void interp_ghost(int i, const double* c, double* f) {
         const int q = par[i];
-        ael::k_patch_interp<<<nblk(L(i).L.N), kBlock, 0, s>>>(c, L(q).L, P(q).ox, P(q).oy, P(q).oz, f, L(i).L, P(i),
-                                                               mode);
+        ael::k_patch_interp_ghost<<<nblk(ael::boundary_count(L(i).L)), kBlock, 0, s>>>(c, L(q).L, P(q).ox, P(q).oy,
+                                                                                       P(q).oz, f, L(i).L, P(i));
     }
-    void ghost(int i, double* v, const double* src, int mode) {
-        ael::k_patch_ghost<<<nblk(L(i).L.N), kBlock, 0, s>>>(v, src, L(i).L, P(i), mode);
+    void ghost(int i, double* v, const double* src) {
+        ael::k_patch_ghost<<<nblk(ael::boundary_count(L(i).L)), kBlock, 0, s>>>(v, src, L(i).L, P(i));
     }
     void sync_solution() {  // average down (deepest first), then refresh the ghost layers
         for (int i : order) {
@@ -2455,38 +2468,61 @@ struct AmrCtx {
             ael::k_patch_inject<<<nblk(m), kBlock, 0, s>>>(x[i], L(i).L, Pi, x[q], L(q).L, P(q).ox, P(q).oy, P(q).oz);
         }
         for (int u = n - 1; u >= 0; --u)
-            if (order[u] != 0) interp(order[u], x[par[order[u]]], x[order[u]], 2);
+            if (order[u] != 0) interp_ghost(order[u], x[par[order[u]]], x[order[u]]);
     }
     // Composite residual on every handle (deepest first, each patch refluxed
-    // into its parent) and its masked inf-norm.
+    // into its parent, its ghost layer read as 0) and its norm.
     int residuals(double* norm) {
         for (int i : order) {
             Level& lv = L(i);
             launch_residual<double>(h[i], lv, x[i], b[i], lv.d.C, lv.d.res, s);
-            if (i > 0) ghost(i, lv.d.res, nullptr, 0);
             for (int c : kids[i]) reflux(c, L(c).d.res, lv.d.res);
         }
-        return masked_norm(norm, true);
+        return composite_norm(norm, true);
+    }
+    // Device lists of every handle's children, grouped by parent, and the
+    // partial norms; kept by the base handle, which is the call's own.
+    std::vector<int> kid0;  // first child of handle i in the list
+    int upload_kids() {
+        alamo_el_t base = h[0];
+        if (base->amr_cap < n) {
+            for (void* p : {(void*)base->amr_kids, (void*)base->amr_part})
+                if (p) (void)hipFree(p);
+            base->amr_kids = nullptr;
+            base->amr_part = nullptr;
+            base->amr_cap = 0;
+            ALLOC(base->amr_kids, n);
+            ALLOC(base->amr_part, (long)kRedBlocks * n);
+            base->amr_cap = n;
+        }
+        std::vector<ael::Patch> list;
+        kid0.assign(n, 0);
+        for (int i = 0; i < n; ++i) {
+            kid0[i] = (int)list.size();
+            for (int c : kids[i]) list.push_back(P(c));
+        }
+        HIPCHK(hipMemcpyAsync(base->amr_kids, list.data(), sizeof(ael::Patch) * list.size(), hipMemcpyHostToDevice, s));
+        HIPCHK(hipStreamSynchronize(s));  // the list is this frame's
+        return 0;
     }
     // max |v| over the composite grid: each handle's res (use_res) or b, ghost
-    // nodes excluded, nodes strictly covered by a child excluded.
-    int masked_norm(double* norm, bool use_res) {
-        *norm = 0.0;
-        int rc;
+    // nodes and nodes strictly covered by a child excluded.  One read of each
+    // field and one wait for the host (a copy to scratch, a mask launch per
+    // child, a reduction and a wait a handle before).
+    int composite_norm(double* norm, bool use_res) {
+        long at = 0;
         for (int i = 0; i < n; ++i) {
             Level& lv = L(i);
-            const long M = 3 * lv.L.N;
-            const double* v = use_res ? lv.d.res : b[i];
-            double* t = lv.d.rescor;
-            launch_copy<double>(t, v, M, s);
-            for (int c : kids[i])
-                ael::k_mask_covered<<<nblk(lv.L.N), kBlock, 0, s>>>(t, lv.L, P(i).ox, P(i).oy, P(i).oz, P(c), t);
-            if (i > 0) ghost(i, t, nullptr, 0);
-            double m;
-            if ((rc = amr_reduce_max(h[i], t, M, &m, s))) return rc;
-            if (std::isnan(m)) return fail(ALAMO_EL_ENAN, "NaN in the composite residual");
-            *norm = std::max(*norm, m);
+            const unsigned nb = (unsigned)std::min<long>(kRedBlocks, nblk(lv.L.N));
+            ael::k_composite_max<<<nb, kBlock, 0, s>>>(use_res ? lv.d.res : b[i], lv.L, P(i), h[0]->amr_kids + kid0[i],
+                                                       (int)kids[i].size(), h[0]->amr_part + at);
+            at += nb;
         }
+        ael::k_reduce_final<<<1, kBlock, 0, s>>>(h[0]->amr_part, (int)at, 0, h[0]->red_out);
+        HIPCHK(hipMemcpyAsync(h[0]->red_host, h[0]->red_out, sizeof(double), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        *norm = h[0]->red_host[0];
+        if (std::isnan(*norm)) return fail(ALAMO_EL_ENAN, "NaN in the composite residual");
         return 0;
     }
 };
@@ -2605,16 +2641,7 @@ int alamo_amr_cluster(const unsigned char* tags_host, const int ncell[3], const 
 int alamo_amr_reflux(alamo_el_t patch, const double* fine_res, double* parent_res, hipStream_t s) {
     if (!patch || !fine_res || !parent_res) return fail(ALAMO_EL_EINVAL, "null argument");
     if (!patch->amr_parent) return fail(ALAMO_EL_EINVAL, "reflux needs a patch (alamo_amr_patch_create)");
-    Level& lv = patch->lv[0];
-    const alamo_el_t par = patch->amr_parent;
-    const ael::Patch& P = patch->amr;
-    // the patch residual with its ghost rows zeroed, in the patch's own scratch
-    launch_copy<double>(lv.d.rescor, fine_res, 3 * lv.L.N, s);
-    ael::k_patch_ghost<<<nblk(lv.L.N), kBlock, 0, s>>>(lv.d.rescor, nullptr, lv.L, P, 0);
-    const long m = (long)(P.chi[0] - P.clo[0] + 1) * (P.chi[1] - P.clo[1] + 1) * (P.chi[2] - P.clo[2] + 1);
-    ael::k_patch_reflux<<<nblk(m), kBlock, 0, s>>>(lv.d.rescor, lv.L, P, parent_res, par->lv[0].L, par->amr.ox,
-                                                    par->amr.oy, par->amr.oz, par->amr_dom[0], par->amr_dom[1],
-                                                    par->amr_dom[2], 3);
+    launch_reflux(patch, fine_res, parent_res, s);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -2627,7 +2654,7 @@ int alamo_amr_average_down_coeffs(alamo_el_t patch, const double* patch_C, doubl
     const long m = (long)(P.chi[0] - P.clo[0] + 1) * (P.chi[1] - P.clo[1] + 1) * (P.chi[2] - P.clo[2] + 1);
     // the patch's C planes, ghost layer included, restricted onto the parent's
     // nodes clo..chi with the reflux weights
-    ael::k_patch_reflux<<<nblk(m), kBlock, 0, s>>>(patch_C, patch->lv[0].L, P, parent_C, par->lv[0].L, par->amr.ox,
+    ael::k_patch_average<<<nblk(m), kBlock, 0, s>>>(patch_C, patch->lv[0].L, P, parent_C, par->lv[0].L, par->amr.ox,
                                                     par->amr.oy, par->amr.oz, par->amr_dom[0], par->amr_dom[1],
                                                     par->amr_dom[2], patch->nc);
     HIPCHK(hipGetLastError());
@@ -2714,10 +2741,11 @@ int alamo_amr_solve(int nlev, const alamo_el_t* hs, double* const* x, const doub
     }
     const bool fp32 = o.precision == ALAMO_EL_PREC_FP32_IR;
     if (fp32 && (rc = prepare32(hs[0], s))) return rc;
+    if ((rc = A.upload_kids())) return rc;
     A.sync_solution();
     double r0, bn;
     if ((rc = A.residuals(&r0))) return rc;
-    if ((rc = A.masked_norm(&bn, false))) return rc;
+    if ((rc = A.composite_norm(&bn, false))) return rc;
     const double target = std::max(tol_abs, std::max(tol_rel, 1.e-16) * std::max(r0, bn));
     Cycle<double> c64{hs[0], s, o.nu1, o.nu2, o.final_smooth, o.bottom_max_iter, o.bottom_tol_rel, o.bottom_solver,
                       o.smoother};
@@ -2726,8 +2754,9 @@ int alamo_amr_solve(int nlev, const alamo_el_t* hs, double* const* x, const doub
     double nrm = r0;
     int iters = 0, status = nrm <= target ? 0 : ALAMO_EL_NOT_CONVERGED;
     const long M0 = 3 * A.L(0).L.N;
-    // nu Fsmooth calls of patch i on its correction (ghost rows held)
-    auto smooth_patch = [&](int i, int nu) {
+    // nu Fsmooth calls of patch i on its correction (ghost rows held), from sweep
+    // done of them on (an odd number leaves the iterate in tmp)
+    auto smooth_patch = [&](int i, int nu, int done) {
         Level& lv = A.L(i);
         if (o.smoother == ALAMO_EL_SMOOTH_RBGS) {
             Cycle<double> ci{hs[i], s, o.nu1, o.nu2, o.final_smooth, o.bottom_max_iter, o.bottom_tol_rel,
@@ -2735,7 +2764,7 @@ int alamo_amr_solve(int nlev, const alamo_el_t* hs, double* const* x, const doub
             ci.smooth(0, lv.d.cor, lv.d.res, nu);
             return;
         }
-        for (int q = 0; q < 2 * nu; ++q) {
+        for (int q = done; q < 2 * nu; ++q) {
             double* src = (q % 2 == 0) ? lv.d.cor : lv.d.tmp;
             double* dst = (q % 2 == 0) ? lv.d.tmp : lv.d.cor;
             launch_jacobi<double>(hs[i], lv, src, lv.d.res, lv.d.diag, lv.d.C, dst, s);
@@ -2748,11 +2777,16 @@ int alamo_amr_solve(int nlev, const alamo_el_t* hs, double* const* x, const doub
             if (i == 0) continue;
             Level& lv = A.L(i);
             const long M = 3 * lv.L.N;
-            launch_fill<double>(lv.d.cor, 0.0, M, s);
-            A.ghost(i, lv.d.res, lv.d.cor, 1);
-            smooth_patch(i, o.nu1);
+            A.ghost(i, lv.d.res, nullptr);  // ghost rows hold the correction at 0
+            if (o.smoother == ALAMO_EL_SMOOTH_JACOBI && o.nu1 > 0) {
+                // the first sweep from zero is w res / D
+                ael::k_jacobi_from_zero<double><<<nblk(M), kBlock, 0, s>>>(lv.d.res, lv.d.diag, hs[i]->omega, lv.d.tmp, M);
+                smooth_patch(i, o.nu1, 1);
+            } else {
+                launch_fill<double>(lv.d.cor, 0.0, M, s);
+                smooth_patch(i, o.nu1, 0);
+            }
             launch_residual<double>(hs[i], lv, lv.d.cor, lv.d.res, lv.d.C, lv.d.rescor, s);
-            A.ghost(i, lv.d.rescor, nullptr, 0);
             A.reflux(i, lv.d.rescor, A.L(A.par[i]).d.res);
         }
         // base level: one multigrid cycle on its composite residual
@@ -2768,9 +2802,9 @@ int alamo_amr_solve(int nlev, const alamo_el_t* hs, double* const* x, const doub
             const int i = A.order[u];
             if (i == 0) continue;
             Level& lv = A.L(i);
-            A.interp(i, A.L(A.par[i]).d.cor, lv.d.cor, 1);
-            A.ghost(i, lv.d.res, lv.d.cor, 1);
-            smooth_patch(i, o.nu2);
+            A.interp_add(i, A.L(A.par[i]).d.cor, lv.d.cor);
+            A.ghost(i, lv.d.res, lv.d.cor);
+            smooth_patch(i, o.nu2, 0);
         }
         for (int l = 0; l < nlev; ++l) launch_axpy<double>(x[l], 1.0, A.L(l).d.cor, 3 * A.L(l).L.N, s);
         A.sync_solution();
