@@ -51,7 +51,7 @@ __device__ __forceinline__ bool eta_tagged(const double* __restrict__ eta, int n
 }
 __global__ void __launch_bounds__(kBlock) k_tag_eta(const double* __restrict__ eta, int ncomp, Lvl L, double thr,
                                                     int* __restrict__ bb) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(kBlock) k_tag_eta(const double* __restrict__ e
 // The same tags, one byte per cell of the box ((nx-1)(ny-1)(nz-1), x fastest).
 __global__ void __launch_bounds__(kBlock) k_tag_cells(const double* __restrict__ eta, int ncomp, Lvl L, double thr,
                                                       unsigned char* __restrict__ tags) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(kBlock) k_tag_cells(const double* __restrict__
 // shell took 16 us on average over the patches of a three-level solve, this 6).
 __global__ void __launch_bounds__(kBlock) k_patch_ghost(double* __restrict__ v, const double* __restrict__ src, Lvl L,
                                                         Patch P) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long t = (long)blockIdx.x * kBlock + threadIdx.x;
     if (t >= boundary_count(L)) return;
     int i, j, k;
     boundary_node(L, t, i, j, k);
@@ -113,7 +113,7 @@ __device__ __forceinline__ double parent_trilinear(const double* __restrict__ c,
 // parent field c).  One thread per node on the handle's faces.
 __global__ void __launch_bounds__(kBlock) k_patch_interp_ghost(const double* __restrict__ c, Lvl Lc, int pox, int poy,
                                                                int poz, double* __restrict__ f, Lvl Lf, Patch P) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long t = (long)blockIdx.x * kBlock + threadIdx.x;
     if (t >= boundary_count(Lf)) return;
     int i, j, k;
     boundary_node(Lf, t, i, j, k);
@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(kBlock) k_patch_interp_ghost(const double* __r
 __global__ void __launch_bounds__(kBlock) k_patch_interp_add(const double* __restrict__ c, Lvl Lc, int pox, int poy,
                                                              int poz, double* __restrict__ f, Lvl Lf, Patch P, int nbx,
                                                              int nby, int nbz) {
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= (unsigned)nbx * nby * nbz) return;
     const unsigned q = t / nbx;
     const int I = (P.ox >> 1) + (int)(t - q * nbx), K = (P.oz >> 1) + (int)(q / nby), J = (P.oy >> 1) + (int)(q % nby);
@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(kBlock) k_patch_interp_add(const double* __res
 __global__ void __launch_bounds__(kBlock) k_patch_fill(const double* __restrict__ c, Lvl Lc, int pox, int poy,
                                                        int poz, const double* __restrict__ so, Lvl Ls, Patch Ps,
                                                        double* __restrict__ f, Lvl Lf, Patch P) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= Lf.N) return;
     int i, j, k;
     node_ijk(id, Lf, i, j, k);
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(kBlock) k_patch_fill(const double* __restrict_
 __global__ void __launch_bounds__(kBlock) k_patch_inject(const double* __restrict__ f, Lvl Lf, Patch P,
                                                          double* __restrict__ c, Lvl Lc, int pox, int poy, int poz) {
     const int nx = P.chi[0] - P.clo[0] + 1, ny = P.chi[1] - P.clo[1] + 1, nz = P.chi[2] - P.clo[2] + 1;
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= (long)nx * ny * nz) return;
     const int a = (int)(id % nx), b = (int)((id / nx) % ny), d = (int)(id / ((long)nx * ny));
     const int I = P.clo[0] + a, J = P.clo[1] + b, K = P.clo[2] + d;  // global parent node
@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(kBlock) k_patch_reflux(const double* __restric
                                                          double* __restrict__ rc, Lvl Lc, int pox, int poy, int poz,
                                                          int dnx, int dny, int dnz) {
     const unsigned nx = P.chi[0] - P.clo[0] + 1, ny = P.chi[1] - P.clo[1] + 1, nz = P.chi[2] - P.clo[2] + 1;
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= nx * ny * nz) return;
     const unsigned q = t / nx;
     const int d[3] = {(int)(t - q * nx), (int)(q % ny), (int)(q / ny)};
@@ -261,7 +261,7 @@ __global__ void __launch_bounds__(kBlock) k_patch_average(const double* __restri
                                                          double* __restrict__ rc, Lvl Lc, int pox, int poy, int poz,
                                                          int dnx, int dny, int dnz, int ncomp) {
     const int nx = P.chi[0] - P.clo[0] + 1, ny = P.chi[1] - P.clo[1] + 1, nz = P.chi[2] - P.clo[2] + 1;
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= (long)nx * ny * nz) return;
     const int a = (int)(id % nx), b = (int)((id / nx) % ny), d = (int)(id / ((long)nx * ny));
     const int I = P.clo[0] + a, J = P.clo[1] + b, K = P.clo[2] + d;  // global parent node
@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(kBlock) k_box_copy(double* __restrict__ dst, i
                                                      int doy, int doz, const double* __restrict__ src, int nsx, int nsy,
                                                      int nsz, int sox, int soy, int soz, int lox, int loy, int loz,
                                                      int bx, int by, int bz, int ncomp) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= (long)bx * by * bz) return;
     const int a = (int)(id % bx), b = (int)((id / bx) % by), c = (int)(id / ((long)bx * by));
     const int gx = lox + a, gy = loy + b, gz = loz + c;
@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(kBlock) k_composite_max(const double* __restri
     __shared__ double sh[kBlock / 64];
     double m = 0.0;
     const unsigned N = (unsigned)L.N;
-    for (unsigned id = blockIdx.x * blockDim.x + threadIdx.x; id < N; id += gridDim.x * blockDim.x) {
+    for (unsigned id = blockIdx.x * kBlock + threadIdx.x; id < N; id += gridDim.x * kBlock) {
         int i, j, k;
         node_ijk(id, L, i, j, k);
         double a[3];

@@ -25,7 +25,7 @@ constexpr int kXcd = 8;
 __device__ __forceinline__ long xcd_node() {
     const long per = (long)gridDim.x / kXcd;
     const long lb = (long)(blockIdx.x % kXcd) * per + blockIdx.x / kXcd;
-    return lb * blockDim.x + threadIdx.x;
+    return lb * kBlock + threadIdx.x;
 }
 
 template <int SYM> struct NComp;
@@ -731,7 +731,7 @@ struct MixTable {
 __global__ void __launch_bounds__(kBlock) k_mix_models(const double* __restrict__ eta, int nmodels, MixTable tab,
                                                        int ncomp, long N, double* __restrict__ out) {
 #pragma clang fp contract(off)
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= N) return;
     for (int c = 0; c < ncomp; ++c) {
         double acc = 0.0;
@@ -894,7 +894,7 @@ __global__ void __launch_bounds__(kBlock) k_restrict_fz(const T* __restrict__ fi
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_inject(const T* __restrict__ fine, Lvl Lf, T* __restrict__ crse, Lvl Lc,
                                                    int ncomp) {
-    const long cid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long cid = (long)blockIdx.x * kBlock + threadIdx.x;
     if (cid >= Lc.N) return;
     int I, J, K;
     node_ijk(cid, Lc, I, J, K);
@@ -916,7 +916,7 @@ struct InjectLevels {
 };
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_inject_all(InjectLevels<T> lv, int ncomp) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = (long)blockIdx.x * kBlock + threadIdx.x;
     if (e >= lv.off[lv.n]) return;
     int l = 1;
     while (e >= lv.off[l + 1]) ++l;
@@ -990,7 +990,7 @@ __global__ void __launch_bounds__(kBlock) k_interp_cell(const T* __restrict__ cr
 
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_fill(T* __restrict__ p, T v, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) p[id] = v;
 }
 
@@ -1000,7 +1000,7 @@ __global__ void __launch_bounds__(kBlock) k_fill(T* __restrict__ p, T v, long n)
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_jacobi_from_zero(const T* __restrict__ b, const T* __restrict__ diag,
                                                              T omega, T* __restrict__ out, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) out[id] = omega * b[id] / diag[id];
 }
 
@@ -1014,7 +1014,7 @@ template <typename T>
 __global__ void __launch_bounds__(kBlock) k_rb_update(T* __restrict__ x, const T* __restrict__ r,
                                                       const T* __restrict__ diag, Lvl L, int color, T w_in,
                                                       T w_bd) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -1030,7 +1030,7 @@ __global__ void __launch_bounds__(kBlock) k_rb_update(T* __restrict__ x, const T
 
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_axpy(T* __restrict__ y, T a, const T* __restrict__ x, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) y[id] += a * x[id];
 }
 
@@ -1040,7 +1040,7 @@ __global__ void __launch_bounds__(kBlock) k_dot2_partial(const double* __restric
                                                          long n, double* __restrict__ partial) {
     __shared__ double sh[2][kBlock / 64];
     double rw = 0.0, ww = 0.0;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
+    for (long q = (long)blockIdx.x * kBlock + threadIdx.x; q < n; q += (long)gridDim.x * kBlock) {
         const double wq = w[q];
         rw += r[q] * wq;
         ww += wq * wq;
@@ -1071,7 +1071,7 @@ __global__ void __launch_bounds__(kBlock) k_step_residual(double* __restrict__ w
                                                           double* __restrict__ partial) {
     __shared__ double sh[kBlock];
     double m = 0.0;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
+    for (long q = (long)blockIdx.x * kBlock + threadIdx.x; q < n; q += (long)gridDim.x * kBlock) {
         const double v = (-g) * w[q] + 1.0 * r[q];
         w[q] = v;
         m = (isnan(v) || isnan(m)) ? NAN : fmax(m, fabs(v));
@@ -1091,7 +1091,7 @@ __global__ void __launch_bounds__(kBlock) k_step_residual(double* __restrict__ w
 // x += g e and r = w, one pass (the step taken).
 __global__ void __launch_bounds__(kBlock) k_take_step(double* __restrict__ x, double g, const double* __restrict__ e,
                                                       double* __restrict__ r, const double* __restrict__ w, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) {
         x[id] += g * e[id];
         r[id] = w[id];
@@ -1101,13 +1101,13 @@ __global__ void __launch_bounds__(kBlock) k_take_step(double* __restrict__ x, do
 // y = a * x
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_scale_copy(const T* __restrict__ x, T a, T* __restrict__ y, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) y[id] = a * x[id];
 }
 
 template <typename Tin, typename Tout>
 __global__ void __launch_bounds__(kBlock) k_cast(const Tin* __restrict__ a, Tout* __restrict__ b, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) b[id] = (Tout)a[id];
 }
 
@@ -1123,7 +1123,7 @@ __global__ void __launch_bounds__(kBlock) k_scale_copy_cast(const double* x, dou
                                                             long n, const Tc* __restrict__ diag = nullptr,
                                                             Tc omega = Tc(0), Tc* __restrict__ fz = nullptr,
                                                             const double* __restrict__ nrm2 = nullptr) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (nrm2) {
         const double hn = sqrt(*nrm2);
         a = hn > 0.0 ? 1.0 / hn : 0.0;
@@ -1141,21 +1141,21 @@ __global__ void __launch_bounds__(kBlock) k_scale_copy_cast(const double* x, dou
 template <typename Tin, typename Tout>
 __global__ void __launch_bounds__(kBlock) k_cast_sum(const Tin* __restrict__ a, const Tin* __restrict__ b,
                                                      Tout* __restrict__ out, long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) out[id] = (Tout)(a[id] + Tin(1) * b[id]);
 }
 
 // y += (double) x  (FP64 correction accumulation of an FP32 correction)
 __global__ void __launch_bounds__(kBlock) k_add_f32_to_f64(double* __restrict__ y, const float* __restrict__ x,
                                                            long n) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) y[id] += (double)x[id];
 }
 
 // AoS (BaseFab<Matrix4> order) -> SoA copy of a stiffness field.
 __global__ void __launch_bounds__(kBlock) k_aos_to_soa(const double* __restrict__ a, double* __restrict__ s, long N,
                                                        int nc) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= N) return;
     for (int c = 0; c < nc; ++c) s[c * N + id] = a[id * nc + c];
 }
@@ -1167,7 +1167,7 @@ __global__ void __launch_bounds__(kBlock) k_reduce_partial(const T* __restrict__
                                                            int op, double* __restrict__ partial) {
     __shared__ double sh[kBlock];
     double acc = 0.0;
-    for (long id = (long)blockIdx.x * blockDim.x + threadIdx.x; id < n; id += (long)gridDim.x * blockDim.x) {
+    for (long id = (long)blockIdx.x * kBlock + threadIdx.x; id < n; id += (long)gridDim.x * kBlock) {
         // max |v| propagates NaN (fmax alone would drop it and hide a blow-up)
         if (op == 0) acc = (isnan((double)a[id]) || isnan(acc)) ? NAN : fmax(acc, fabs((double)a[id]));
         else if (op == 1) acc += (double)a[id] * (double)b[id];
@@ -1190,7 +1190,7 @@ __global__ void __launch_bounds__(kBlock) k_reduce_final(const double* __restric
                                                          double* __restrict__ out) {
     __shared__ double sh[kBlock];
     double acc = 0.0;
-    for (int q = threadIdx.x; q < nb; q += blockDim.x)
+    for (int q = threadIdx.x; q < nb; q += kBlock)
         acc = op == 0 ? ((isnan(partial[q]) || isnan(acc)) ? NAN : fmax(acc, partial[q])) : acc + partial[q];
     sh[threadIdx.x] = acc;
     __syncthreads();
@@ -1208,7 +1208,7 @@ __global__ void __launch_bounds__(kBlock) k_reduce_final(const double* __restric
 // BC::Operator::Elastic::Constant::Init (src/BC/Operator/Elastic/Constant.H:197-286).
 __global__ void __launch_bounds__(kBlock) k_bc_init(double* __restrict__ rhs, const int* __restrict__ bct,
                                                     const double* __restrict__ bcv, int homogeneous, Lvl L) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -1244,7 +1244,7 @@ __global__ void __launch_bounds__(kBlock) k_newton_dw(const double* __restrict__
                                                       int np, double* __restrict__ gu9, double* __restrict__ dw9) {
     constexpr int NC = NComp<SYM>::value;
     const long S = (long)np * L.nx * L.ny;
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long q = (long)blockIdx.x * kBlock + threadIdx.x;
     if (q >= S) return;
     const long id = (long)kb * L.nx * L.ny + q;
     int i, j, k;
@@ -1272,7 +1272,7 @@ __global__ void __launch_bounds__(kBlock) k_stress(const double* __restrict__ u,
                                                    const double* __restrict__ F0, Lvl L, double* __restrict__ sigma,
                                                    double* __restrict__ strain) {
     constexpr int NC = NComp<SYM>::value;
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -1351,7 +1351,7 @@ __global__ void __launch_bounds__(kBlock) k_newton_rhs(const double* __restrict_
                                                        int kb, int np, const int* __restrict__ bct, Lvl L, int k0,
                                                        int k1, double* __restrict__ rhs) {
     const long P = (long)L.nx * L.ny, S = (long)np * P;
-    const long id = (long)k0 * P + (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)k0 * P + (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= (long)k1 * P) return;
     const long q = id - (long)kb * P;  // position in the slab of gu9 and dw9
     int i, j, k;
@@ -1395,7 +1395,7 @@ template <int SYM>
 __global__ void __launch_bounds__(kBlock) k_assemble_dense(const double* __restrict__ I, const double* __restrict__ C,
                                                            const int* __restrict__ bct, int uniform, Lvl L,
                                                            double* __restrict__ Acol) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     const long M = 3 * L.N;
     if (id >= L.N) return;
     const long q = blockIdx.y;
@@ -1415,7 +1415,7 @@ constexpr int kDenseMvChunk = 32;
 template <typename T, typename TA>
 __global__ void __launch_bounds__(kBlock) k_dense_mv_partial(const TA* __restrict__ A, const T* __restrict__ x,
                                                              int M, double* __restrict__ part) {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (r >= M) return;
     const int c0 = (int)blockIdx.y * kDenseMvChunk, c1 = min(M, c0 + kDenseMvChunk);
     double acc = 0.0;
@@ -1426,7 +1426,7 @@ __global__ void __launch_bounds__(kBlock) k_dense_mv_partial(const TA* __restric
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_dense_mv_final(const double* __restrict__ part, int nch, int M,
                                                            T* __restrict__ y) {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (r >= M) return;
     double acc = 0.0;
 #pragma unroll 8
@@ -1440,7 +1440,7 @@ __global__ void __launch_bounds__(kBlock) k_dense_mv_final(const double* __restr
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_dense_mv_rows(const double* __restrict__ At, const T* __restrict__ x,
                                                           int M, T* __restrict__ y) {
-    const int r = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), lane = (int)(threadIdx.x & 63);
+    const int r = (int)((blockIdx.x * kBlock + threadIdx.x) >> 6), lane = (int)(threadIdx.x & 63);
     if (r >= M) return;  // whole waves
     const double* __restrict__ row = At + (long)r * M;
     double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
@@ -1489,8 +1489,8 @@ __global__ void __launch_bounds__(kBlock) k_multidot_partial(const TV* __restric
     for (int i = 0; i < kMultiDotMax; ++i) acc[i] = 0.0;
     // four grid strides per step with independent loads (the accumulation
     // order is the plain loop's), then the remainder
-    const long st = (long)gridDim.x * blockDim.x;
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long st = (long)gridDim.x * kBlock;
+    long q = (long)blockIdx.x * kBlock + threadIdx.x;
     for (; q + 3 * st < M; q += 4 * st) {
         double wq[4], vq[kMultiDotMax][4];
 #pragma unroll
@@ -1547,8 +1547,8 @@ __global__ void __launch_bounds__(kBlock) k_multiaxpy_dot(double* __restrict__ w
     double acc[kMultiDotMax], nrm = 0.0;
 #pragma unroll
     for (int i = 0; i < kMultiDotMax; ++i) acc[i] = 0.0;
-    const long st = (long)gridDim.x * blockDim.x;
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long st = (long)gridDim.x * kBlock;
+    long q = (long)blockIdx.x * kBlock + threadIdx.x;
     for (; q + 3 * st < M; q += 4 * st) {
         double wq[4], vq[kMultiDotMax][4];
 #pragma unroll
@@ -1640,8 +1640,8 @@ __global__ void __launch_bounds__(kBlock) k_multidot2_partial(const TV* __restri
     // two grid strides per step with independent loads (four held 256 VGPRs
     // with an FP64 basis, and ran at half speed with an FP32 one)
     constexpr int kU = 2;
-    const long st = (long)gridDim.x * blockDim.x;
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long st = (long)gridDim.x * kBlock;
+    long q = (long)blockIdx.x * kBlock + threadIdx.x;
     for (; q + (kU - 1) * st < M; q += kU * st) {
         double wq[kU], tq[kU], vq[kMultiDotMax - 1][kU];
 #pragma unroll
@@ -1750,8 +1750,8 @@ __global__ void __launch_bounds__(kBlock) k_dcgs2_update(TV* __restrict__ V, int
     double nrm = 0.0;
     // two grid strides per step with independent loads (four held 256 VGPRs)
     constexpr int kU = 2;
-    const long st = (long)gridDim.x * blockDim.x;
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long st = (long)gridDim.x * kBlock;
+    long q = (long)blockIdx.x * kBlock + threadIdx.x;
     for (; q + (kU - 1) * st < M; q += kU * st) {
         double wq[kU], tq[kU], vq[kMultiDotMax - 1][kU];
 #pragma unroll
@@ -1812,7 +1812,7 @@ __global__ void __launch_bounds__(kBlock) k_multidot_final(const double* __restr
                                                            double* __restrict__ h) {
     __shared__ double sh[kBlock];
     double acc = 0.0;
-    for (int q = threadIdx.x; q < nb; q += blockDim.x) acc += partial[(long)blockIdx.x * nb + q];
+    for (int q = threadIdx.x; q < nb; q += kBlock) acc += partial[(long)blockIdx.x * nb + q];
     sh[threadIdx.x] = acc;
     __syncthreads();
     for (int st = kBlock / 2; st > 0; st >>= 1) {
@@ -1827,7 +1827,7 @@ __global__ void __launch_bounds__(kBlock) k_multidot_final(const double* __restr
 template <typename TV>
 __global__ void __launch_bounds__(kBlock) k_multiaxpy(double* __restrict__ w, const TV* __restrict__ V, int k, long M,
                                                       long ld, const double* __restrict__ h, double sign) {
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long q = (long)blockIdx.x * kBlock + threadIdx.x;
     if (q >= M) return;
     double acc = w[q];
     for (int i = 0; i < k; ++i) acc += sign * h[i] * (double)V[(long)i * ld + q];

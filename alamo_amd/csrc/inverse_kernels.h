@@ -196,7 +196,7 @@ inline void launch_inv_panel(double* W, int M, int c0, int nb, int* perm, InvSta
 // untouched).  The caller's threads fill the identity and stage the swaps;
 // thread 0 applies them in order, from LDS.
 __device__ __forceinline__ void swap_map(const int* __restrict__ perm, int M, int k0, int n, int* map, int* ps) {
-    for (int r = (int)threadIdx.x; r < M; r += blockDim.x) map[r] = r;
+    for (int r = (int)threadIdx.x; r < M; r += kBlock) map[r] = r;
     if ((int)threadIdx.x < n) ps[threadIdx.x] = perm[k0 + threadIdx.x];
     __syncthreads();
     if (threadIdx.x == 0)
@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(kBlock) k_inv_rowmap(const int* __restrict__ p
                                                        int* __restrict__ map) {
     __shared__ int sm[kInvMax], ps[kInvBlock];
     swap_map(perm, M, k0, nbk, sm, ps);
-    for (int r = (int)threadIdx.x; r < M; r += blockDim.x) map[r] = sm[r];
+    for (int r = (int)threadIdx.x; r < M; r += kBlock) map[r] = sm[r];
 }
 
 // Out of place, Wo from Wi: the block's columns [k0, k0 + kInvBlock) are
@@ -536,7 +536,7 @@ __device__ __forceinline__ double inv_check_x(int r) {
     return (double)(int)(h >> 8) / 8388608.0 - 1.0;
 }
 __global__ void __launch_bounds__(kBlock) k_inv_check_x(double* __restrict__ x, int M) {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (r < M) x[r] = inv_check_x(r);
 }
 __global__ void __launch_bounds__(kBlock) k_inv_check(const double* __restrict__ z, int M, InvState* __restrict__ st) {
@@ -572,7 +572,7 @@ __global__ void __launch_bounds__(kBlock) k_inv_check(const double* __restrict__
 // Undo the column permutation: inv[:, c] = W[:, src[c]].
 __global__ void __launch_bounds__(kBlock) k_inv_unpermute(const double* __restrict__ W, int M,
                                                           const int* __restrict__ src, double* __restrict__ inv) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = (long)blockIdx.x * kBlock + threadIdx.x;
     if (e >= (long)M * M) return;
     const int c = (int)(e / M), r = (int)(e - (long)c * M);
     inv[e] = W[(long)src[c] * M + r];
@@ -580,7 +580,7 @@ __global__ void __launch_bounds__(kBlock) k_inv_unpermute(const double* __restri
 
 // Identity (column-major M x M): the unit vectors of the dense assemblies.
 __global__ void __launch_bounds__(kBlock) k_eye(double* __restrict__ I, int M) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = (long)blockIdx.x * kBlock + threadIdx.x;
     if (e >= (long)M * M) return;
     const int c = (int)(e / M), r = (int)(e - (long)c * M);
     I[e] = r == c ? 1.0 : 0.0;

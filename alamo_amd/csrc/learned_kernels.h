@@ -28,7 +28,7 @@ __device__ __forceinline__ bool on_boundary(const Lvl& L, int i, int j, int k) {
 // out = b on interior nodes, 0 on boundary nodes (3 components).
 __global__ void __launch_bounds__(kBlock) k_interior_only(const double* __restrict__ b, Lvl L,
                                                           double* __restrict__ out) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(kBlock) k_interior_only(const double* __restri
 // sit on (fine index = factor * coarse index); interior nodes are kept.
 __global__ void __launch_bounds__(kBlock) k_inject_boundary(const double* __restrict__ bf, Lvl Lf, int factor,
                                                             double* __restrict__ bc, Lvl Lc) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= Lc.N) return;
     int I, J, K;
     node_ijk(id, Lc, I, J, K);
@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_boundary(const double* __rest
 // t = b / alpha on interior nodes, b on boundary nodes.
 __global__ void __launch_bounds__(kBlock) k_prescale(const double* __restrict__ b, Lvl L, double inv_alpha,
                                                      double* __restrict__ t) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(kBlock) k_face_means(const double* __restrict_
     const int n1 = ax == 0 ? L.ny : L.nx, n2 = ax == 2 ? L.ny : L.nz;
     const long cnt = (long)n1 * n2;
     double acc = 0.0;
-    for (long q = threadIdx.x; q < cnt; q += blockDim.x) {
+    for (long q = threadIdx.x; q < cnt; q += kBlock) {
         const int a = (int)(q % n1), b = (int)(q / n1);
         int i, j, k;
         if (ax == 0) { i = hi ? L.nx - 1 : 0; j = a; k = b; }
@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(kBlock) k_face_means(const double* __restrict_
 __global__ void __launch_bounds__(kBlock) k_features(const double* __restrict__ C, int nc, const double* __restrict__ t,
                                                      const int* __restrict__ bct, const double* __restrict__ fmean,
                                                      Lvl L, double inv_alpha, double inv_s, float* __restrict__ feat) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kBlock) k_features(const double* __restrict__ 
 // u = s * y (float32 network output -> FP64 level field).
 __global__ void __launch_bounds__(kBlock) k_scale_output(const float* __restrict__ y, long n, double s,
                                                          double* __restrict__ u) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id < n) u[id] = s * (double)y[id];
 }
 

@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(kBlock) k_psi_post(const T* __restrict__ x, co
                                                      const int* __restrict__ bct, const double* __restrict__ psi,
                                                      double small, Lvl L, T w, int mode, T* __restrict__ out) {
     constexpr int NC = NComp<SYM>::value;
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     x += 3 * L.N * (long)blockIdx.y;
     out += 3 * L.N * (long)blockIdx.y;
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(kBlock) k_psi_post(const T* __restrict__ x, co
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_psi_diag(T* __restrict__ diag, const int* __restrict__ bct,
                                                      const double* __restrict__ psi, double small, Lvl L) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);
@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(kBlock) k_psi_restrict(const double* __restric
                                                          double* __restrict__ pc, Lvl Lc) {
     const int cx = Lc.nx - 1, cy = Lc.ny - 1, cz = Lc.nz - 1;
     const int fx = Lf.nx - 1, fy = Lf.ny - 1;
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= (long)cx * cy * cz) return;
     const long t = id / cx;
     const int I = (int)(id - t * cx), K = (int)(t / cy), J = (int)(t - (long)K * cy);

@@ -100,7 +100,7 @@ __device__ __forceinline__ bool slab_interior_node(const Lvl& L, long ib, int& i
     const unsigned x = (unsigned)ib % kXcd, lb = (unsigned)ib / kXcd;
     const unsigned j0 = x * (unsigned)nj / kXcd, j1 = (x + 1) * (unsigned)nj / kXcd;
     const unsigned per_plane = (j1 - j0) * (unsigned)ni;
-    const unsigned t = lb * blockDim.x + threadIdx.x;  // below 2^29 + the padding of the last workgroups
+    const unsigned t = lb * kBlock + threadIdx.x;  // below 2^29 + the padding of the last workgroups
     if (t >= per_plane * (unsigned)nk) return false;
     const unsigned kk = t / per_plane;
     const unsigned r = t - kk * per_plane;
@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(kBlock)
     long id;
     T o[3];
     if (blockIdx.x < nbb) {
-        const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+        const long t = (long)blockIdx.x * kBlock + threadIdx.x;
         if (t >= boundary_count(L)) return;
         boundary_node(L, t, i, j, k);
         id = ((long)k * L.ny + j) * L.nx + i;
@@ -270,7 +270,7 @@ __global__ void __launch_bounds__(kBlock)
 template <int NC>
 __global__ void __launch_bounds__(kBlock) k_grad_mask(const double* __restrict__ C, Lvl L,
                                                       unsigned char* __restrict__ gmask) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= L.N) return;
     int i, j, k;
     node_ijk(id, L, i, j, k);

@@ -95,7 +95,7 @@ struct TileIdx {
 // 64-bit hash of each node's 21 slots (bit patterns).
 __global__ void __launch_bounds__(kBlock) k_c_hash(const double* __restrict__ C, long N,
                                                    unsigned long long* __restrict__ hs) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= N) return;
     unsigned long long h = 0xcbf29ce484222325ull;
     for (int q = 0; q < 21; ++q) {
@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(kBlock) k_c_hash(const double* __restrict__ C,
 __global__ void __launch_bounds__(kBlock) k_run_heads(const unsigned long long* __restrict__ hs, long N, int cap,
                                                       unsigned long long* __restrict__ heads,
                                                       unsigned int* __restrict__ count) {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long id = (long)blockIdx.x * kBlock + threadIdx.x;
     if (id >= N) return;
     const unsigned long long h = hs[id];
     if (id > 0 && hs[id - 1] == h) return;
@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(kBlock) k_run_heads(const unsigned long long* 
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_pal_gather(const double* __restrict__ C, long N, const long* __restrict__ rep,
                                                        int npal, T* __restrict__ pal) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= npal * kPalStride) return;
     const int q = t / kPalStride, s = t % kPalStride;
     pal[t] = s < 21 ? (T)C[s * N + rep[q]] : T(0);
@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(kBlock) k_pal_index_b(const double* __restrict
                                                         const unsigned long long* __restrict__ ph, int npal,
                                                         const double* __restrict__ pal, PalIdx* __restrict__ pidx_b,
                                                         int* __restrict__ bad) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long t = (long)blockIdx.x * kBlock + threadIdx.x;
     if (t >= boundary_count(L)) return;
     int i, j, k;
     boundary_node(L, t, i, j, k);
@@ -214,7 +214,7 @@ __device__ __forceinline__ void pal_row(const T* __restrict__ pr, T cv[21]) {
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_pack_bnd_c(const double* __restrict__ C, Lvl L, int nc,
                                                        T* __restrict__ Cb) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long t = (long)blockIdx.x * kBlock + threadIdx.x;
     const long nb = boundary_count(L);
     if (t >= nb) return;
     int i, j, k;
@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(TS::NT)
     const unsigned ntb = gridDim.x - nbb;  // tile workgroups
     const bool bnd = kBoundaryLast ? blockIdx.x >= ntb : blockIdx.x < nbb;
     if (bnd) {
-        const long t = (long)(kBoundaryLast ? blockIdx.x - ntb : blockIdx.x) * blockDim.x + threadIdx.x;
+        const long t = (long)(kBoundaryLast ? blockIdx.x - ntb : blockIdx.x) * kBlock + threadIdx.x;
         if (t >= boundary_count(L)) return;
         int i, j, k;
         boundary_node(L, t, i, j, k);
@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(TS::NT) __attribute__((amdgpu_waves_per_eu(4))
     __shared__ T sc[3][2 * HP];  // lambda, mu
     const unsigned ntb = gridDim.x - nbb;  // tile workgroups; the boundary ones come after them
     if (blockIdx.x >= ntb) {
-        const long t = (long)(blockIdx.x - ntb) * blockDim.x + threadIdx.x;
+        const long t = (long)(blockIdx.x - ntb) * kBlock + threadIdx.x;
         if (t >= boundary_count(L)) return;
         int i, j, k;
         boundary_node(L, t, i, j, k);

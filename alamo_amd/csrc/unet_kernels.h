@@ -19,6 +19,9 @@ typedef uint16_t bf16_t;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// Threads of the element-wise launches: a constant, as blockDim is read from memory
+constexpr int kThreads = 256;
+
 struct G3 {
     int nx, ny, nz, N;
 };
@@ -252,7 +255,7 @@ __global__ void __launch_bounds__(64) k_conv_wgrad(const bf16_t* __restrict__ X,
 // out[i] = sum_c part[c * M + i]
 __global__ void __launch_bounds__(256) k_sum_chunks(const float* __restrict__ part, int nchunk, long M,
                                                     float* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= M) return;
     float s = 0.f;
     for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * M + i];
@@ -279,7 +282,7 @@ __global__ void __launch_bounds__(256) k_bias_grad(const bf16_t* __restrict__ dZ
 // Wb[ci][t][co] = W[co][26 - t][ci], used by the input gradient.
 __global__ void __launch_bounds__(256) k_pack_weights(const float* __restrict__ W, int Cin, int Cout, int Cinp,
                                                       int Coutp, bf16_t* __restrict__ Wt, bf16_t* __restrict__ Wb) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     const long M = (long)Coutp * 27 * Cinp;
     if (i >= M) return;
     const int ci = (int)(i % Cinp);
@@ -294,7 +297,7 @@ __global__ void __launch_bounds__(256) k_pack_weights(const float* __restrict__ 
 // Padded float32 dW[Coutp][27][Cinp] -> canonical dWc[Cout][27][Cin].
 __global__ void __launch_bounds__(256) k_unpack_grad(const float* __restrict__ dWp, int Cin, int Cout, int Cinp,
                                                      float* __restrict__ dWc) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     const long M = (long)Cout * 27 * Cin;
     if (i >= M) return;
     const int ci = (int)(i % Cin);
@@ -308,7 +311,7 @@ __global__ void __launch_bounds__(256) k_unpack_grad(const float* __restrict__ d
 __global__ void __launch_bounds__(256) k_down(const bf16_t* __restrict__ X, int C, G3 gf, G3 gc, float scale,
                                               bf16_t* __restrict__ Y) {
     const int c8 = C / 8;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)gc.N * c8) return;
     const int q = (int)(i % c8);
     const int I = (int)(i / c8);
@@ -334,7 +337,7 @@ __global__ void __launch_bounds__(256) k_down(const bf16_t* __restrict__ X, int 
 __global__ void __launch_bounds__(256) k_up(const bf16_t* __restrict__ X, int C, G3 gc, G3 gf, float scale,
                                             const bf16_t* __restrict__ add, bf16_t* __restrict__ Y) {
     const int c8 = C / 8;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)gf.N * c8) return;
     const int q = (int)(i % c8);
     const int v = (int)(i / c8);
@@ -362,7 +365,7 @@ __global__ void __launch_bounds__(256) k_up(const bf16_t* __restrict__ X, int C,
 __global__ void __launch_bounds__(256) k_concat(const bf16_t* __restrict__ A, int Ca, const bf16_t* __restrict__ B,
                                                 int Cb, int N, bf16_t* __restrict__ Y) {
     const int c8 = (Ca + Cb) / 8;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)N * c8) return;
     const int q = (int)(i % c8), v = (int)(i / c8);
     const int c = 8 * q;
@@ -373,7 +376,7 @@ __global__ void __launch_bounds__(256) k_concat(const bf16_t* __restrict__ A, in
 __global__ void __launch_bounds__(256) k_split(const bf16_t* __restrict__ Y, int Ca, int Cb, int N,
                                                bf16_t* __restrict__ A, bf16_t* __restrict__ B) {
     const int c8 = (Ca + Cb) / 8;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)N * c8) return;
     const int q = (int)(i % c8), v = (int)(i / c8);
     const int c = 8 * q;
@@ -384,7 +387,7 @@ __global__ void __launch_bounds__(256) k_split(const bf16_t* __restrict__ Y, int
 
 // g = (y > 0) ? g : 0 for the bf16 output y of a ReLU layer, 8 values per thread.
 __global__ void __launch_bounds__(256) k_relu_mask(bf16_t* __restrict__ g, const bf16_t* __restrict__ y, long n8) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n8) return;
     uint4 gq = reinterpret_cast<uint4*>(g)[i];
     const uint4 yq = reinterpret_cast<const uint4*>(y)[i];
@@ -402,7 +405,7 @@ __global__ void __launch_bounds__(256) k_relu_mask(bf16_t* __restrict__ g, const
 // Component-major float32 in[c * N + v] (c < n) -> bf16 X[v * Cp + c] (zero padded).
 __global__ void __launch_bounds__(256) k_pack_soa(const float* __restrict__ in, int n, int Cp, int N,
                                                   bf16_t* __restrict__ X) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)N * Cp) return;
     const int c = (int)(i % Cp), v = (int)(i / Cp);
     X[i] = c < n ? f2bf(in[(size_t)c * N + v]) : (bf16_t)0;
@@ -410,7 +413,7 @@ __global__ void __launch_bounds__(256) k_pack_soa(const float* __restrict__ in, 
 // bf16 X[v * Cp + c] -> float32 out[c * N + v] for c < n.
 __global__ void __launch_bounds__(256) k_unpack_soa(const bf16_t* __restrict__ X, int n, int Cp, int N,
                                                     float* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)N * n) return;
     const int v = (int)(i % N), c = (int)(i / N);
     out[i] = bf2f(X[(size_t)v * Cp + c]);
@@ -421,7 +424,7 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ y, const 
                                              float inv, float* __restrict__ d, float* __restrict__ part) {
     __shared__ float sh[256];
     float s = 0.f;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < M; i += (long)gridDim.x * blockDim.x) {
+    for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < M; i += (long)gridDim.x * kThreads) {
         const float e = y[i] - t[i];
         s += e * e;
         if (d) d[i] = 2.f * e * inv;
@@ -439,7 +442,7 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ y, const 
 __global__ void __launch_bounds__(256) k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                                               float* __restrict__ v, long n, float lr, float b1, float b2, float eps,
                                               float c1, float c2) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
     const float gi = g[i];
     const float mi = b1 * m[i] + (1.f - b1) * gi;
