@@ -33,7 +33,8 @@ namespace {
 constexpr int kLevels = 4;
 constexpr int kCh[kLevels] = {16, 32, 64, 128};
 constexpr int kLossBlocks = 256;
-constexpr int kWgradWaves = 2048;  // target waves of one weight-gradient launch
+constexpr int kWgradBlocks = 256;  // target workgroups of one weight-gradient launch
+constexpr int kBiasBlocks = 256;   // most workgroups (bias partials) of k_wgrad_dz
 
 inline unsigned nb256(long n) { return (unsigned)((n + 255) / 256); }
 inline int pad16(int c) { return (c + 15) / 16 * 16; }
@@ -60,9 +61,9 @@ struct alamo_nn_s {
     int adam_t = 0;
     bool packed = false;    // bf16 weights up to date with p
     bool have_fwd = false;
-    float* dwp = nullptr;   // padded weight gradient of one layer
-    float* part = nullptr;  // per-chunk partial weight gradients
-    long part_cap = 0;
+    float* part = nullptr;  // per-chunk partial weight gradients of one layer
+    float* bpart = nullptr; // and its bias gradient's
+    bf16_t *trx = nullptr, *trz = nullptr;  // its transposed input (three shifts) and output gradient
     float* loss_part = nullptr;
     float* dtmp = nullptr;  // output gradient of train_step [n_out][N0]
     float* otmp = nullptr;  // output of train_step [n_out][N0]
@@ -115,20 +116,42 @@ void launch_conv(const bf16_t* X, int Cin, const bf16_t* W, const float* bias, i
     }
 }
 
-// Chunking of the weight-gradient reduction over N nodes for `tiles` waves per chunk.
-void wgrad_chunks(int N, int tiles, int& chunk, int& nchunk) {
-    const int maxc = (N + 31) / 32;
-    nchunk = std::max(1, std::min(maxc, kWgradWaves / std::max(1, tiles)));
-    chunk = ((N + nchunk - 1) / nchunk + 31) / 32 * 32;
-    nchunk = (N + chunk - 1) / chunk;
+// The weight gradient's node groups: 8 nodes of a row each, n8 a row.  Its steps
+// of 4 groups are cut into nchunk parts of `steps` each, for about kWgradBlocks
+// workgroups with `tiles` a part and no fewer than a step a wave.
+struct WgradGrid {
+    int n8, steps, nchunk;
+    long ngroup;
+};
+WgradGrid wgrad_grid(const G3& g, int tiles) {
+    WgradGrid w;
+    w.n8 = (g.nx + 7) / 8;
+    w.ngroup = (long)g.ny * g.nz * w.n8;
+    const long total = (w.ngroup + 3) / 4;
+    long nchunk = std::max(1, kWgradBlocks / std::max(1, tiles));
+    nchunk = std::max(1L, std::min(nchunk, total / aunet::kWgradWaves));
+    w.steps = (int)((total + nchunk - 1) / nchunk);
+    w.nchunk = (int)((total + w.steps - 1) / w.steps);
+    return w;
 }
 
 int pack_weights(alamo_nn_t nn, hipStream_t s) {
     if (nn->packed) return 0;
-    for (auto& L : nn->cv) {
-        const long M = (long)L.coutp * 27 * L.cinp;
-        aunet::k_pack_weights<<<nb256(M), 256, 0, s>>>(nn->p + L.woff, L.cin, L.cout, L.cinp, L.coutp, L.wt, L.wb);
+    static_assert(aunet::kMaxConv == 2 * kLevels + 2 * (kLevels - 1) + 1, "one entry per convolution");
+    aunet::PackLayers P{};
+    P.n = (int)nn->cv.size();
+    for (int l = 0; l < P.n; ++l) {
+        const ConvL& L = nn->cv[l];
+        P.first[l + 1] = P.first[l] + (long)L.coutp * 27 * L.cinp;
+        P.W[l] = nn->p + L.woff;
+        P.cin[l] = L.cin;
+        P.cout[l] = L.cout;
+        P.cinp[l] = L.cinp;
+        P.coutp[l] = L.coutp;
+        P.wt[l] = L.wt;
+        P.wb[l] = L.wb;
     }
+    aunet::k_pack_weights<<<nb256(P.first[P.n]), 256, 0, s>>>(P);
     NNCHK(hipGetLastError());
     nn->packed = true;
     return 0;
@@ -146,16 +169,16 @@ void conv_back(alamo_nn_t nn, int li, const bf16_t* X, const bf16_t* Y, bf16_t* 
                hipStream_t s) {
     const ConvL& L = nn->cv[li];
     const G3& g = nn->g[L.level];
-    if (L.relu) aunet::k_relu_mask<<<nb256((long)g.N * L.coutp / 8), 256, 0, s>>>(dY, Y, (long)g.N * L.coutp / 8);
     const int tiles = (L.cinp / 16) * (L.coutp / 16);
-    int chunk, nchunk;
-    wgrad_chunks(g.N, tiles, chunk, nchunk);
-    aunet::k_conv_wgrad<<<dim3(tiles, nchunk), 64, 0, s>>>(X, L.cinp, dY, L.coutp, g, chunk, nn->part);
-    const long M = (long)L.coutp * 27 * L.cinp;
-    aunet::k_sum_chunks<<<nb256(M), 256, 0, s>>>(nn->part, nchunk, M, nn->dwp);
-    const long Mc = (long)L.cout * 27 * L.cin;
-    aunet::k_unpack_grad<<<nb256(Mc), 256, 0, s>>>(nn->dwp, L.cin, L.cout, L.cinp, grad + L.woff);
-    aunet::k_bias_grad<<<L.cout, 256, 0, s>>>(dY, L.coutp, g.N, grad + L.boff);
+    const WgradGrid w = wgrad_grid(g, tiles);
+    const int nb = (int)std::min<long>(kBiasBlocks, (w.ngroup * L.coutp + 255) / 256);
+    aunet::k_wgrad_dz<<<nb, 256, 0, s>>>(dY, L.relu ? Y : nullptr, L.coutp, g.nx, w.n8, w.ngroup, nn->trz, nn->bpart);
+    aunet::k_wgrad_x<<<nb256(w.ngroup * L.cinp), 256, 0, s>>>(X, L.cinp, g.nx, w.n8, w.ngroup, nn->trx);
+    aunet::k_conv_wgrad<<<dim3(tiles, w.nchunk), 64 * aunet::kWgradWaves, 0, s>>>(nn->trx, L.cinp, nn->trz, L.coutp, g.ny,
+                                                                                  g.nz, w.n8, w.steps, nn->part);
+    const long ne = 27L * L.cin * L.cout + L.cout;  // the layer's weights and biases are adjacent
+    aunet::k_wgrad_finish<<<(unsigned)((ne + 63) / 64), 256, 0, s>>>(nn->part, w.nchunk, L.cin, L.cout, L.cinp, L.coutp,
+                                                                     nn->bpart, nb, grad + L.woff);
     if (dX) launch_conv(dY, L.coutp, L.wb, nullptr, L.cinp, g, 0, dX, nullptr, 0, s);
 }
 
@@ -302,19 +325,19 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
     NNCHK(hipMemset(nn->p, 0, sizeof(float) * np));
     NNCHK(hipMemset(nn->m, 0, sizeof(float) * np));
     NNCHK(hipMemset(nn->v, 0, sizeof(float) * np));
-    long dwmax = 0, partmax = 0;
+    long partmax = 0, xmax = 0, zmax = 0;
     for (auto& L : nn->cv) {
         const long M = (long)L.coutp * 27 * L.cinp;
         if ((rc = nalloc_t(nn, &L.wt, M)) || (rc = nalloc_t(nn, &L.wb, M))) return cleanup(rc);
-        dwmax = std::max(dwmax, M);
-        int chunk, nchunk;
-        wgrad_chunks(nn->g[L.level].N, (L.cinp / 16) * (L.coutp / 16), chunk, nchunk);
-        partmax = std::max(partmax, M * nchunk);
+        const WgradGrid w = wgrad_grid(nn->g[L.level], (L.cinp / 16) * (L.coutp / 16));
+        partmax = std::max(partmax, M * w.nchunk);
+        xmax = std::max(xmax, 3L * L.cinp * 8 * w.ngroup);
+        zmax = std::max(zmax, (long)L.coutp * 8 * w.ngroup);
     }
-    if ((rc = nalloc_t(nn, &nn->dwp, dwmax)) || (rc = nalloc_t(nn, &nn->part, partmax)) ||
+    if ((rc = nalloc_t(nn, &nn->part, partmax)) || (rc = nalloc_t(nn, &nn->bpart, (long)kBiasBlocks * kCh[kLevels - 1])) ||
+        (rc = nalloc_t(nn, &nn->trx, xmax)) || (rc = nalloc_t(nn, &nn->trz, zmax)) ||
         (rc = nalloc_t(nn, &nn->loss_part, kLossBlocks)))
         return cleanup(rc);
-    nn->part_cap = partmax;
     const G3* g = nn->g;
     const long N0 = g[0].N;
     if ((rc = nalloc_t(nn, &nn->dtmp, (long)n_out * N0)) || (rc = nalloc_t(nn, &nn->otmp, (long)n_out * N0)) ||

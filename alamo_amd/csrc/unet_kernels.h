@@ -194,116 +194,196 @@ __global__ void __launch_bounds__(64 * KS) k_conv_fwd_ks(const bf16_t* __restric
     conv_store<NB>(acc, bias, Cout, g, relu, v0, row, grp, nbase, Y, Yf, yf_ch);
 }
 
-// Partial weight gradient over one chunk of nodes:
-//   part[chunk][co][t][ci] = sum_{v in chunk} dZ[v][co] * X[v + d_t][ci].
-// One wave per (co block of 16, ci block of 16, chunk), all 27 taps; the
-// reduction over nodes is the MFMA K dimension (32 nodes per step).
-__global__ void __launch_bounds__(64) k_conv_wgrad(const bf16_t* __restrict__ X, int Cin, const bf16_t* __restrict__ dZ,
-                                                   int Cout, G3 g, int chunk, float* __restrict__ part) {
-    const int lane = threadIdx.x;
-    const int ncib = Cin / 16;
-    const int cib = blockIdx.x % ncib, cob = blockIdx.x / ncib;
-    const int ch = blockIdx.y;
-    const int vbeg = ch * chunk, vend = min(g.N, vbeg + chunk);
-    const int row = lane & 15, grp = lane >> 4;
-    const int co = cob * 16 + row, ci = cib * 16 + row;
+// --- Weight and bias gradients ---------------------------------------------
+// dW[co][t][ci] = sum_v dZ[v][co] X[v + d_t][ci] reduces over nodes, which are
+// the MFMA K dimension: a lane holds 8 consecutive K of one channel.  The
+// activations are channels-last, where those 8 are strided two-byte loads, so
+// both operands are first transposed into rows of nodes: T[c][row][i], row =
+// z ny + y, i padded to n8 groups of 8 with zeros.  X is kept three times,
+// shifted by -1, 0 and 1 along i, so that every tap is an aligned 16-byte load.
+// At 33^3 nodes, 15 layers: 422 us for the four kernels (wgrad 14.0, finish 5.5,
+// transposes 4.5 and 4.2 us a layer), where gathers of two bytes a lane, up to
+// 1123 partials a weight summed by one thread each, a mask, a bias and an
+// unpacking launch took 2112 us.
+
+// One thread per (group of 8 nodes, channel): the gradient dY of a layer's output
+// masked by its ReLU (Y the output; null: no ReLU), in place, its transpose T, and
+// the block's sums per channel (the bias gradient's partials, bpart[block][C]).
+// C is a power of two, at most 128.
+__global__ void __launch_bounds__(kThreads) k_wgrad_dz(bf16_t* __restrict__ dY, const bf16_t* __restrict__ Y, int C,
+                                                       int nx, int n8, long ngroup, bf16_t* __restrict__ T,
+                                                       float* __restrict__ bpart) {
+    __shared__ float sh[kThreads];
+    const int c = (int)threadIdx.x & (C - 1), sub = (int)threadIdx.x / C, nsub = kThreads / C;
+    const long rows = ngroup / n8;
+    float sum = 0.f;
+    for (long q = (long)blockIdx.x * nsub + sub; q < ngroup; q += (long)gridDim.x * nsub) {
+        const long row = q / n8;
+        const int i0 = (int)(q - row * n8) * 8;
+        const size_t at = ((size_t)row * nx + i0) * C + c;
+        uint32_t v[8], y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const size_t o = at + (size_t)(i0 + e < nx ? e : 0) * C;  // in the row
+            v[e] = dY[o];
+            y[e] = Y ? Y[o] : 1u;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const bool in = i0 + e < nx, pos = (y[e] & 0x7FFFu) != 0 && !(y[e] & 0x8000u);
+            v[e] = in && pos ? v[e] : 0u;
+            if (Y && in) dY[at + (size_t)e * C] = (bf16_t)v[e];
+            sum += bf2f((bf16_t)v[e]);
+        }
+        *reinterpret_cast<uint4*>(T + ((size_t)c * rows + row) * (8 * n8) + i0) =
+            make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+    }
+    sh[threadIdx.x] = sum;
+    __syncthreads();
+    if (sub == 0) {
+        for (int w = 1; w < nsub; ++w) sum += sh[w * C + c];
+        bpart[(size_t)blockIdx.x * C + c] = sum;
+    }
+}
+// The three shifted transposes of X: T[s][c][row][i] = X[row][i + s - 1][c].
+__global__ void __launch_bounds__(kThreads) k_wgrad_x(const bf16_t* __restrict__ X, int C, int nx, int n8, long ngroup,
+                                                      bf16_t* __restrict__ T) {
+    const long t = (long)blockIdx.x * kThreads + threadIdx.x;
+    const long q = t / C;
+    if (q >= ngroup) return;
+    const int c = (int)(t - q * C);
+    const long row = q / n8, rows = ngroup / n8;
+    const int i0 = (int)(q - row * n8) * 8;
+    uint32_t v[10];
+#pragma unroll
+    for (int e = 0; e < 10; ++e) {
+        const int i = i0 + e - 1;
+        const bool in = i >= 0 && i < nx;
+        const uint32_t x = X[((size_t)row * nx + (in ? i : 0)) * C + c];
+        v[e] = in ? x : 0u;
+    }
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+        *reinterpret_cast<uint4*>(T + (((size_t)s * C + c) * rows + row) * (8 * n8) + i0) =
+            make_uint4(v[s] | (v[s + 1] << 16), v[s + 2] | (v[s + 3] << 16), v[s + 4] | (v[s + 5] << 16),
+                       v[s + 6] | (v[s + 7] << 16));
+}
+// Partial weight gradient of one 16 x 16 tile of (co, ci), all 27 taps, over the
+// blockIdx.y-th part of the node groups: part[chunk][co][t][ci].  4 waves share
+// the part's steps of 4 groups (one per 16 lanes), their tiles added in wave
+// order through LDS.
+constexpr int kWgradWaves = 4;
+__global__ void __launch_bounds__(64 * kWgradWaves) k_conv_wgrad(const bf16_t* __restrict__ Tx, int Cin,
+                                                                 const bf16_t* __restrict__ Tz, int Cout, int ny, int nz,
+                                                                 int n8, int steps, float* __restrict__ part) {
+    __shared__ f32x4 red[27][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ncib = Cin / 16, cib = blockIdx.x % ncib, cob = blockIdx.x / ncib, ch = blockIdx.y;
+    const int r16 = lane & 15, grp = lane >> 4;
+    const int co = cob * 16 + r16, ci = cib * 16 + r16;
+    const int rows = ny * nz;
+    const long ngroup = (long)rows * n8;
+    const size_t line = 8 * (size_t)n8, sx = (size_t)Cin * rows * line;  // a row; a shift of Tx
+    const bf16_t* zc = Tz + (size_t)co * rows * line;
+    const bf16_t* xc = Tx + (size_t)ci * rows * line;
     f32x4 acc[27];
 #pragma unroll
     for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int vb = vbeg; vb < vend; vb += 32) {
-        int xs[8], ys[8], zs[8];
-        bool ok[8];
-        uint16_t av[8];
+    auto keep = [](bool ok, const uint4& v) {  // zeros where the position is outside the grid
+        return make_uint4(ok ? v.x : 0u, ok ? v.y : 0u, ok ? v.z : 0u, ok ? v.w : 0u);
+    };
+    for (int st = wave; st < steps; st += kWgradWaves) {
+        const long q = ((long)ch * steps + st) * 4 + grp;
+        const bool in = q < ngroup;
+        const int row = in ? (int)(q / n8) : 0, g8 = in ? (int)(q - (long)row * n8) : 0;
+        const int z = row / ny, y = row - z * ny;
+        const bf16x8 A =
+            __builtin_bit_cast(bf16x8, keep(in, *reinterpret_cast<const uint4*>(zc + row * line + 8 * g8)));
+        uint4 bq[3][9];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int v = vb + grp * 8 + e;
-            ok[e] = v < vend;
-            const int vv = ok[e] ? v : 0;
-            xs[e] = vv % g.nx;
-            const int t = vv / g.nx;
-            ys[e] = t % g.ny;
-            zs[e] = t / g.ny;
-            av[e] = ok[e] ? dZ[(size_t)vv * Cout + co] : (uint16_t)0;
-        }
-        const uint4 aq = make_uint4(av[0] | ((uint32_t)av[1] << 16), av[2] | ((uint32_t)av[3] << 16),
-                                    av[4] | ((uint32_t)av[5] << 16), av[6] | ((uint32_t)av[7] << 16));
-        const bf16x8 A = __builtin_bit_cast(bf16x8, aq);
+        for (int dz = 0; dz < 3; ++dz)
 #pragma unroll
-        for (int t = 0; t < 27; ++t) {
-            uint16_t bv[8];
+            for (int dy = 0; dy < 3; ++dy) {
+                const int zz = z + dz - 1, yy = y + dy - 1;
+                const bool ok = in && zz >= 0 && zz < nz && yy >= 0 && yy < ny;
+                const bf16_t* xr = xc + (ok ? zz * ny + yy : row) * line + 8 * g8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                int nbr;
-                const bool in = ok[e] && tap_node(g, xs[e], ys[e], zs[e], t, nbr);
-                bv[e] = in ? X[(size_t)nbr * Cin + ci] : (uint16_t)0;
+                for (int s = 0; s < 3; ++s) bq[dz][3 * dy + s] = keep(ok, *reinterpret_cast<const uint4*>(xr + s * sx));
             }
-            const uint4 bq = make_uint4(bv[0] | ((uint32_t)bv[1] << 16), bv[2] | ((uint32_t)bv[3] << 16),
-                                        bv[4] | ((uint32_t)bv[5] << 16), bv[6] | ((uint32_t)bv[7] << 16));
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, bq), acc[t], 0, 0, 0);
-        }
+#pragma unroll
+        for (int t = 0; t < 27; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, bq[t / 9][t % 9]), acc[t], 0,
+                                                             0, 0);
     }
-    // acc[t][e] = D[co_local = 4 grp + e][ci_local = row]
+    for (int w = 1; w < kWgradWaves; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int t = 0; t < 27; ++t) red[t][lane] = acc[t];
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int t = 0; t < 27; ++t) acc[t] += red[t][lane];
+        }
+        __syncthreads();
+    }
+    if (wave > 0) return;
+    // acc[t][e] = D[co_local = 4 grp + e][ci_local = r16]
 #pragma unroll
     for (int t = 0; t < 27; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int o = cob * 16 + grp * 4 + e;
-            part[(((size_t)ch * Cout + o) * 27 + t) * Cin + ci] = acc[t][e];
-        }
+        for (int e = 0; e < 4; ++e)
+            part[(((size_t)ch * Cout + cob * 16 + grp * 4 + e) * 27 + t) * Cin + ci] = acc[t][e];
 }
-
-// out[i] = sum_c part[c * M + i]
-__global__ void __launch_bounds__(256) k_sum_chunks(const float* __restrict__ part, int nchunk, long M,
-                                                    float* __restrict__ out) {
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= M) return;
+// The layer's gradient from the partials, in the canonical parameter order:
+// grad[0 .. 27 cin cout) the weights from part[nchunk][coutp][27][cinp], then the
+// cout biases from bpart[nb][coutp].  64 entries a workgroup, 4 threads an entry,
+// each every 4th partial, added in order.
+__global__ void __launch_bounds__(kThreads) k_wgrad_finish(const float* __restrict__ part, int nchunk, int cin, int cout,
+                                                           int cinp, int coutp, const float* __restrict__ bpart, int nb,
+                                                           float* __restrict__ grad) {
+    __shared__ float sh[4][64];
+    const long nw = 27L * cin * cout, e = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int sl = threadIdx.x >> 6;
     float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * M + i];
-    out[i] = s;
-}
-
-// db[n] = sum_v dZ[v][n]; one workgroup per channel.
-__global__ void __launch_bounds__(256) k_bias_grad(const bf16_t* __restrict__ dZ, int C, int N, float* __restrict__ db) {
-    __shared__ float sh[256];
-    const int n = blockIdx.x;
-    float s = 0.f;
-    for (int v = threadIdx.x; v < N; v += 256) s += bf2f(dZ[(size_t)v * C + n]);
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
+    if (e < nw) {
+        const long q = e / cin;
+        const float* p = part + q * cinp + (e - q * cin);  // q = co 27 + t
+        const long M = 27L * cinp * coutp;
+#pragma unroll 4
+        for (int c = sl; c < nchunk; c += 4) s += p[c * M];
+    } else if (e < nw + cout) {
+#pragma unroll 4
+        for (int c = sl; c < nb; c += 4) s += bpart[(size_t)c * coutp + (e - nw)];
     }
-    if (threadIdx.x == 0) db[n] = sh[0];
+    sh[sl][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (sl == 0 && e < nw + cout) grad[e] = ((s + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
 }
 
 // Canonical float32 W[Cout][27][Cin] -> bf16 Wt[Coutp][27 * Cinp] (zero
 // padded) and the flipped transpose Wb[Cinp][27 * Coutp],
-// Wb[ci][t][co] = W[co][26 - t][ci], used by the input gradient.
-__global__ void __launch_bounds__(256) k_pack_weights(const float* __restrict__ W, int Cin, int Cout, int Cinp,
-                                                      int Coutp, bf16_t* __restrict__ Wt, bf16_t* __restrict__ Wb) {
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    const long M = (long)Coutp * 27 * Cinp;
-    if (i >= M) return;
-    const int ci = (int)(i % Cinp);
-    const int t = (int)((i / Cinp) % 27);
-    const int co = (int)(i / ((long)27 * Cinp));
-    const float w = (ci < Cin && co < Cout) ? W[((size_t)co * 27 + t) * Cin + ci] : 0.f;
+// Wb[ci][t][co] = W[co][26 - t][ci], used by the input gradient.  Every layer in
+// one launch: layer l takes the threads from first[l] on.
+constexpr int kMaxConv = 15;
+struct PackLayers {
+    int n;
+    long first[kMaxConv + 1];
+    const float* W[kMaxConv];
+    int cin[kMaxConv], cout[kMaxConv], cinp[kMaxConv], coutp[kMaxConv];
+    bf16_t *wt[kMaxConv], *wb[kMaxConv];
+};
+__global__ void __launch_bounds__(kThreads) k_pack_weights(PackLayers P) {
+    const long e = (long)blockIdx.x * kThreads + threadIdx.x;
+    if (e >= P.first[P.n]) return;
+    int l = 0;
+    while (e >= P.first[l + 1]) ++l;
+    const unsigned i = (unsigned)(e - P.first[l]), cinp = P.cinp[l];
+    const unsigned q = i / cinp, ci = i - q * cinp, co = q / 27, t = q - co * 27;
+    const float w = ((int)ci < P.cin[l] && (int)co < P.cout[l]) ? P.W[l][((size_t)co * 27 + t) * P.cin[l] + ci] : 0.f;
     const bf16_t b = f2bf(w);
-    Wt[i] = b;
-    Wb[((size_t)ci * 27 + (26 - t)) * Coutp + co] = b;
-}
-
-// Padded float32 dW[Coutp][27][Cinp] -> canonical dWc[Cout][27][Cin].
-__global__ void __launch_bounds__(256) k_unpack_grad(const float* __restrict__ dWp, int Cin, int Cout, int Cinp,
-                                                     float* __restrict__ dWc) {
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    const long M = (long)Cout * 27 * Cin;
-    if (i >= M) return;
-    const int ci = (int)(i % Cin);
-    const int t = (int)((i / Cin) % 27);
-    const int co = (int)(i / ((long)27 * Cin));
-    dWc[i] = dWp[((size_t)co * 27 + t) * Cinp + ci];
+    P.wt[l][i] = b;
+    P.wb[l][((size_t)ci * 27 + (26 - t)) * P.coutp[l] + co] = b;
 }
 
 // Full weighting with scale: Y[I][c] = scale * sum_d w(d) X[2I + d][c],
@@ -383,23 +463,6 @@ __global__ void __launch_bounds__(256) k_split(const bf16_t* __restrict__ Y, int
     const uint4 val = *reinterpret_cast<const uint4*>(Y + (size_t)v * (Ca + Cb) + c);
     if (c < Ca) *reinterpret_cast<uint4*>(A + (size_t)v * Ca + c) = val;
     else *reinterpret_cast<uint4*>(B + (size_t)v * Cb + (c - Ca)) = val;
-}
-
-// g = (y > 0) ? g : 0 for the bf16 output y of a ReLU layer, 8 values per thread.
-__global__ void __launch_bounds__(256) k_relu_mask(bf16_t* __restrict__ g, const bf16_t* __restrict__ y, long n8) {
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n8) return;
-    uint4 gq = reinterpret_cast<uint4*>(g)[i];
-    const uint4 yq = reinterpret_cast<const uint4*>(y)[i];
-    uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
-    const uint32_t yw[4] = {yq.x, yq.y, yq.z, yq.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = yw[k] & 0xFFFFu, hi = yw[k] >> 16;
-        const bool plo = (lo & 0x7FFFu) != 0 && !(lo & 0x8000u), phi = (hi & 0x7FFFu) != 0 && !(hi & 0x8000u);
-        gw[k] = (plo ? (gw[k] & 0xFFFFu) : 0u) | (phi ? (gw[k] & 0xFFFF0000u) : 0u);
-    }
-    reinterpret_cast<uint4*>(g)[i] = make_uint4(gw[0], gw[1], gw[2], gw[3]);
 }
 
 // Component-major float32 in[c * N + v] (c < n) -> bf16 X[v * Cp + c] (zero padded).
