@@ -10,6 +10,7 @@
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/alamo_elastic.h"
@@ -70,12 +71,11 @@ struct alamo_nn_s {
     // activations (bf16, channels last)
     bf16_t* X0 = nullptr;
     bf16_t *A[kLevels] = {}, *E[kLevels] = {}, *D[kLevels] = {};
-    bf16_t *U[kLevels - 1] = {}, *K[kLevels - 1] = {}, *B[kLevels - 1] = {}, *G[kLevels - 1] = {};
+    bf16_t *K[kLevels - 1] = {}, *B[kLevels - 1] = {}, *G[kLevels - 1] = {};
     // gradients of the activations
     bf16_t *gX0 = nullptr, *gY = nullptr;
     bf16_t *gA[kLevels] = {}, *gE[kLevels] = {}, *gD[kLevels] = {};
-    bf16_t *gU[kLevels - 1] = {}, *gK[kLevels - 1] = {}, *gB[kLevels - 1] = {}, *gG[kLevels - 1] = {},
-           *gEs[kLevels - 1] = {};
+    bf16_t *gK[kLevels - 1] = {}, *gB[kLevels - 1] = {}, *gG[kLevels - 1] = {};
     std::vector<void*> allocs;
 };
 
@@ -102,17 +102,28 @@ void launch_conv(const bf16_t* X, int Cin, const bf16_t* W, const float* bias, i
     const char* ks_env = std::getenv("ALAMO_NN_KSPLIT");
     const int ksplit = ks_env ? std::atoi(ks_env) : 1;
     const long plain_wg = (long)grid.x * (Cout % 64 == 0 ? Cout / 64 : Cout % 32 == 0 ? Cout / 32 : Cout / 16);
-    if (ksplit == 2 || (ksplit == 1 && plain_wg < 256)) {
-        aunet::k_conv_fwd_ks<1, 4><<<dim3((unsigned)((g.N + 15) / 16), Cout / 16), 256, 0, s>>>(X, Cin, W, bias, Cout, g,
-                                                                                                relu, Y, Yf, yf_ch);
-        return;
-    }
-    if (Cout % 64 == 0) {
-        aunet::k_conv_fwd<4><<<dim3(grid.x, Cout / 64), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
-    } else if (Cout % 32 == 0) {
-        aunet::k_conv_fwd<2><<<dim3(grid.x, Cout / 32), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
-    } else {
-        aunet::k_conv_fwd<1><<<dim3(grid.x, Cout / 16), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+    const bool ks = ksplit == 2 || (ksplit == 1 && plain_wg < 256);
+    auto go = [&](auto cin_tag) {
+        constexpr int CIN = decltype(cin_tag)::value;
+        if (ks)
+            aunet::k_conv_fwd_ks<1, 4, CIN><<<dim3((unsigned)((g.N + 15) / 16), Cout / 16), 256, 0, s>>>(
+                X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+        else if (Cout % 64 == 0)
+            aunet::k_conv_fwd<4, CIN><<<dim3(grid.x, Cout / 64), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+        else if (Cout % 32 == 0)
+            aunet::k_conv_fwd<2, CIN><<<dim3(grid.x, Cout / 32), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+        else
+            aunet::k_conv_fwd<1, CIN><<<dim3(grid.x, Cout / 16), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+    };
+    switch (Cin) {  // the network's own channel counts; an input padded to another takes the general form
+        case 16: go(std::integral_constant<int, 16>{}); break;
+        case 32: go(std::integral_constant<int, 32>{}); break;
+        case 48: go(std::integral_constant<int, 48>{}); break;
+        case 64: go(std::integral_constant<int, 64>{}); break;
+        case 96: go(std::integral_constant<int, 96>{}); break;
+        case 128: go(std::integral_constant<int, 128>{}); break;
+        case 192: go(std::integral_constant<int, 192>{}); break;
+        default: go(std::integral_constant<int, 0>{}); break;
     }
 }
 
@@ -186,23 +197,22 @@ int forward(alamo_nn_t nn, const float* in, float* out, hipStream_t s) {
     int rc = pack_weights(nn, s);
     if (rc) return rc;
     const G3* g = nn->g;
-    aunet::k_pack_soa<<<nb256((long)g[0].N * nn->cin0p), 256, 0, s>>>(in, nn->n_in, nn->cin0p, g[0].N, nn->X0);
+    aunet::k_pack_soa<<<dim3((unsigned)((g[0].N + 63) / 64), nn->cin0p / 16), 256, 0, s>>>(in, nn->n_in, nn->cin0p, g[0].N, nn->X0);
     const bf16_t* h = nn->X0;
     for (int l = 0; l < kLevels; ++l) {
         conv_fwd(nn, 2 * l, h, nn->A[l], nullptr, s);
         conv_fwd(nn, 2 * l + 1, nn->A[l], nn->E[l], nullptr, s);
         if (l + 1 < kLevels) {
             const long n = (long)g[l + 1].N * kCh[l] / 8;
-            aunet::k_down<<<nb256(n), 256, 0, s>>>(nn->E[l], kCh[l], g[l], g[l + 1], 0.125f, nn->D[l + 1]);
+            aunet::k_down<<<nb256(n), 256, 0, s>>>(nn->E[l], kCh[l], kCh[l], g[l], g[l + 1], 0.125f, nn->D[l + 1]);
             h = nn->D[l + 1];
         }
     }
     const bf16_t* up_in = nn->E[kLevels - 1];
     for (int l = kLevels - 2; l >= 0; --l) {
         const int cu = kCh[l + 1], ce = kCh[l];
-        aunet::k_up<<<nb256((long)g[l].N * cu / 8), 256, 0, s>>>(up_in, cu, g[l + 1], g[l], 1.f, nullptr, nn->U[l]);
-        aunet::k_concat<<<nb256((long)g[l].N * (cu + ce) / 8), 256, 0, s>>>(nn->U[l], cu, nn->E[l], ce, g[l].N,
-                                                                            nn->K[l]);
+        aunet::k_up_concat<<<nb256((long)g[l].N * (cu + ce) / 8), 256, 0, s>>>(up_in, cu, g[l + 1], g[l], nn->E[l], ce,
+                                                                               nn->K[l]);
         const int li = 2 * kLevels + 2 * (kLevels - 2 - l);
         conv_fwd(nn, li, nn->K[l], nn->B[l], nullptr, s);
         conv_fwd(nn, li + 1, nn->B[l], nn->G[l], nullptr, s);
@@ -218,7 +228,7 @@ int backward(alamo_nn_t nn, const float* dout, float* grad, float* din, hipStrea
     if (!nn->have_fwd) return fail(ALAMO_EL_ESTATE, "alamo_nn_backward needs a preceding alamo_nn_forward");
     const G3* g = nn->g;
     const int last = (int)nn->cv.size() - 1;
-    aunet::k_pack_soa<<<nb256((long)g[0].N * nn->coutp_out), 256, 0, s>>>(dout, nn->n_out, nn->coutp_out, g[0].N,
+    aunet::k_pack_soa<<<dim3((unsigned)((g[0].N + 63) / 64), nn->coutp_out / 16), 256, 0, s>>>(dout, nn->n_out, nn->coutp_out, g[0].N,
                                                                           nn->gY);
     conv_back(nn, last, nn->G[0], nullptr, nn->gY, nn->gG[0], grad, s);
     for (int l = 0; l <= kLevels - 2; ++l) {
@@ -226,17 +236,17 @@ int backward(alamo_nn_t nn, const float* dout, float* grad, float* din, hipStrea
         const int cu = kCh[l + 1], ce = kCh[l];
         conv_back(nn, li + 1, nn->B[l], nn->G[l], nn->gG[l], nn->gB[l], grad, s);
         conv_back(nn, li, nn->K[l], nn->B[l], nn->gB[l], nn->gK[l], grad, s);
-        aunet::k_split<<<nb256((long)g[l].N * (cu + ce) / 8), 256, 0, s>>>(nn->gK[l], cu, ce, g[l].N, nn->gU[l],
-                                                                           nn->gEs[l]);
-        // adjoint of trilinear up: 8 x full weighting
+        // adjoint of trilinear up: 8 x full weighting, of the decoder input's first cu channels
         bf16_t* dst = (l + 1 < kLevels - 1) ? nn->gG[l + 1] : nn->gE[kLevels - 1];
-        aunet::k_down<<<nb256((long)g[l + 1].N * cu / 8), 256, 0, s>>>(nn->gU[l], cu, g[l], g[l + 1], 1.f, dst);
+        aunet::k_down<<<nb256((long)g[l + 1].N * cu / 8), 256, 0, s>>>(nn->gK[l], cu + ce, cu, g[l], g[l + 1], 1.f, dst);
     }
     for (int l = kLevels - 1; l >= 0; --l) {
         if (l < kLevels - 1) {
-            // adjoint of down (full weighting / 8): up / 8, plus the skip-path gradient
-            aunet::k_up<<<nb256((long)g[l].N * kCh[l] / 8), 256, 0, s>>>(nn->gD[l + 1], kCh[l], g[l + 1], g[l],
-                                                                         0.125f, nn->gEs[l], nn->gE[l]);
+            // adjoint of down (full weighting / 8): up / 8, plus the skip-path
+            // gradient, the last channels of the decoder input's
+            aunet::k_up_add<<<nb256((long)g[l].N * kCh[l] / 8), 256, 0, s>>>(nn->gD[l + 1], kCh[l], g[l + 1], g[l], 0.125f,
+                                                                             nn->gK[l], kCh[l + 1] + kCh[l], kCh[l + 1],
+                                                                             nn->gE[l]);
         }
         conv_back(nn, 2 * l + 1, nn->A[l], nn->E[l], nn->gE[l], nn->gA[l], grad, s);
         const bf16_t* Xl = l == 0 ? nn->X0 : nn->D[l];
@@ -353,11 +363,10 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
             return cleanup(rc);
         if (l < kLevels - 1) {
             const int cu = kCh[l + 1], ce = kCh[l];
-            if ((rc = nalloc_t(nn, &nn->U[l], N * cu)) || (rc = nalloc_t(nn, &nn->K[l], N * (cu + ce))) ||
+            if ((rc = nalloc_t(nn, &nn->K[l], N * (cu + ce))) ||
                 (rc = nalloc_t(nn, &nn->B[l], N * ce)) || (rc = nalloc_t(nn, &nn->G[l], N * ce)) ||
-                (rc = nalloc_t(nn, &nn->gU[l], N * cu)) || (rc = nalloc_t(nn, &nn->gK[l], N * (cu + ce))) ||
-                (rc = nalloc_t(nn, &nn->gB[l], N * ce)) || (rc = nalloc_t(nn, &nn->gG[l], N * ce)) ||
-                (rc = nalloc_t(nn, &nn->gEs[l], N * ce)))
+                (rc = nalloc_t(nn, &nn->gK[l], N * (cu + ce))) || (rc = nalloc_t(nn, &nn->gB[l], N * ce)) ||
+                (rc = nalloc_t(nn, &nn->gG[l], N * ce)))
                 return cleanup(rc);
         }
     }

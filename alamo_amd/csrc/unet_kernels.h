@@ -57,21 +57,24 @@ __device__ __forceinline__ bool tap_node(const G3& g, int x, int y, int z, int t
 
 // The K rounds of one wave's 16 nodes x 16*NB output channels, starting at
 // k = kfirst and stepping by kstep (a multiple of 32 * KU): KU steps of 32
-// along K per round, every A and B load of the round issued before its MFMAs
-// (one wait per round instead of one per step; the small levels have few
-// waves to hide it), the MFMAs in step order.
+// along K per round, the A and B loads of LA rounds issued before their MFMAs
+// (a wave waits for memory once per LA rounds; the small levels have few waves
+// to hide it), the MFMAs in step order whatever LA is.  CIN > 0 fixes the input
+// channels at compile time (0: the argument), so that a step's tap and channel
+// need no division.
 constexpr int kConvKU = 4;
-template <int NB>
-__device__ __forceinline__ void conv_rounds(const bf16_t* __restrict__ X, int Cin, const bf16_t* __restrict__ Wt,
+template <int NB, int CIN>
+__device__ __forceinline__ void conv_rounds(const bf16_t* __restrict__ X, int cin, const bf16_t* __restrict__ Wt,
                                             const G3& g, bool vin, int x, int y, int z, int row, int grp, int nbase,
                                             int kfirst, int kstep, f32x4 acc[NB]) {
-    constexpr int KU = kConvKU;
+    constexpr int KU = kConvKU, LA = NB == 1 ? 3 : NB == 2 ? 2 : 1;
+    const int Cin = CIN > 0 ? CIN : cin;
     const int K = 27 * Cin;
-    for (int k0 = kfirst; k0 < K; k0 += kstep) {
-        uint4 a[KU], b[KU][NB];
+    for (int k0 = kfirst; k0 < K; k0 += LA * kstep) {
+        uint4 a[LA * KU], b[LA * KU][NB];
 #pragma unroll
-        for (int u = 0; u < KU; ++u) {
-            const int k = k0 + 32 * u + grp * 8;
+        for (int u = 0; u < LA * KU; ++u) {
+            const int k = k0 + (u / KU) * kstep + 32 * (u % KU) + grp * 8;
             a[u] = make_uint4(0, 0, 0, 0);
             if (vin && k < K) {
                 const int t = k / Cin, c = k - t * Cin;
@@ -86,8 +89,8 @@ __device__ __forceinline__ void conv_rounds(const bf16_t* __restrict__ X, int Ci
             }
         }
 #pragma unroll
-        for (int u = 0; u < KU; ++u) {
-            if (k0 + 32 * u >= K) break;
+        for (int u = 0; u < LA * KU; ++u) {
+            if (k0 + (u / KU) * kstep + 32 * (u % KU) >= K) break;
             const bf16x8 A = __builtin_bit_cast(bf16x8, a[u]);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
@@ -138,7 +141,7 @@ __device__ __forceinline__ void conv_node(const G3& g, int vox, bool vin, int& x
 // selects 16*NB output channels.  Wt[n][27 * Cin] (bf16).  bias may be null.
 // Yf != null: write float32 component-major Yf[n * N + v] for n < yf_ch
 // instead of the bf16 Y (the network output).
-template <int NB>
+template <int NB, int CIN>
 __global__ void __launch_bounds__(256) k_conv_fwd(const bf16_t* __restrict__ X, int Cin, const bf16_t* __restrict__ Wt,
                                                   const float* __restrict__ bias, int Cout, G3 g, int relu,
                                                   bf16_t* __restrict__ Y, float* __restrict__ Yf, int yf_ch) {
@@ -154,7 +157,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const bf16_t* __restrict__ X, 
     f32x4 acc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    conv_rounds<NB>(X, Cin, Wt, g, vin, x, y, z, row, grp, nbase, 0, 32 * kConvKU, acc);
+    conv_rounds<NB, CIN>(X, Cin, Wt, g, vin, x, y, z, row, grp, nbase, 0, 32 * kConvKU, acc);
     conv_store<NB>(acc, bias, Cout, g, relu, v0, row, grp, nbase, Y, Yf, yf_ch);
 }
 
@@ -163,7 +166,7 @@ __global__ void __launch_bounds__(256) k_conv_fwd(const bf16_t* __restrict__ X, 
 // of K = 27 Cin one round after another).  Every wave of the workgroup takes
 // the same 16 nodes and 16*NB channels and every KS-th round of K; wave 0
 // adds the others' float32 tiles in wave order through LDS and stores.
-template <int NB, int KS>
+template <int NB, int KS, int CIN>
 __global__ void __launch_bounds__(64 * KS) k_conv_fwd_ks(const bf16_t* __restrict__ X, int Cin,
                                                          const bf16_t* __restrict__ Wt, const float* __restrict__ bias,
                                                          int Cout, G3 g, int relu, bf16_t* __restrict__ Y,
@@ -180,7 +183,7 @@ __global__ void __launch_bounds__(64 * KS) k_conv_fwd_ks(const bf16_t* __restric
     f32x4 acc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    conv_rounds<NB>(X, Cin, Wt, g, vin, x, y, z, row, grp, nbase, wave * 32 * kConvKU, 32 * kConvKU * KS, acc);
+    conv_rounds<NB, CIN>(X, Cin, Wt, g, vin, x, y, z, row, grp, nbase, wave * 32 * kConvKU, 32 * kConvKU * KS, acc);
     if (wave > 0) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) part[wave - 1][nb][lane] = acc[nb];
@@ -387,91 +390,119 @@ __global__ void __launch_bounds__(kThreads) k_pack_weights(PackLayers P) {
 }
 
 // Full weighting with scale: Y[I][c] = scale * sum_d w(d) X[2I + d][c],
-// w(d) = prod_a (1 - |d_a| / 2), zero outside the fine grid.  8 channels per thread.
-__global__ void __launch_bounds__(256) k_down(const bf16_t* __restrict__ X, int C, G3 gf, G3 gc, float scale,
-                                              bf16_t* __restrict__ Y) {
+// w(d) = prod_a (1 - |d_a| / 2), zero outside the fine grid.  8 channels per
+// thread; X has ld channels a node, the first C of them are taken.  All 27 loads
+// leave before the sums (in tap order; a position outside the grid reads the
+// node itself with weight 0): one at a time they took 12.7 us at 33^3 nodes.
+__global__ void __launch_bounds__(kThreads) k_down(const bf16_t* __restrict__ X, int ld, int C, G3 gf, G3 gc, float scale,
+                                                   bf16_t* __restrict__ Y) {
     const int c8 = C / 8;
     const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)gc.N * c8) return;
-    const int q = (int)(i % c8);
-    const int I = (int)(i / c8);
-    const int X0 = I % gc.nx, Y0 = (I / gc.nx) % gc.ny, Z0 = I / (gc.nx * gc.ny);
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int t = 0; t < 27; ++t) {
-        const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-        const int xx = 2 * X0 + dx, yy = 2 * Y0 + dy, zz = 2 * Z0 + dz;
-        if (xx < 0 || xx >= gf.nx || yy < 0 || yy >= gf.ny || zz < 0 || zz >= gf.nz) continue;
-        const float w = (dx ? 0.5f : 1.f) * (dy ? 0.5f : 1.f) * (dz ? 0.5f : 1.f);
-        float f[8];
-        unpack8(*reinterpret_cast<const uint4*>(X + ((size_t)(zz * gf.ny + yy) * gf.nx + xx) * C + 8 * q), f);
+    const int I = (int)(i / c8), q = (int)(i - (long)I * c8);
+    const int Z0 = I / (gc.nx * gc.ny), r = I - Z0 * gc.nx * gc.ny, Y0 = r / gc.nx, X0 = r - Y0 * gc.nx;
+    uint4 v[27];
+    unsigned in = 0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += w * f[e];
+    for (int t = 0; t < 27; ++t) {
+        const int xx = 2 * X0 + t % 3 - 1, yy = 2 * Y0 + t / 3 % 3 - 1, zz = 2 * Z0 + t / 9 - 1;
+        const bool ok = xx >= 0 && xx < gf.nx && yy >= 0 && yy < gf.ny && zz >= 0 && zz < gf.nz;
+        in |= ok ? 1u << t : 0u;
+        const size_t n = ok ? (size_t)(zz * gf.ny + yy) * gf.nx + xx : (size_t)(2 * Z0 * gf.ny + 2 * Y0) * gf.nx + 2 * X0;
+        v[t] = *reinterpret_cast<const uint4*>(X + n * ld + 8 * q);
+    }
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 27; ++t) {
+        const float w = (t % 3 != 1 ? 0.5f : 1.f) * (t / 3 % 3 != 1 ? 0.5f : 1.f) * (t / 9 != 1 ? 0.5f : 1.f);
+        float f[8];
+        unpack8(v[t], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = (in >> t) & 1u ? acc[e] + w * f[e] : acc[e];
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] *= scale;
     *reinterpret_cast<uint4*>(Y + (size_t)I * C + 8 * q) = pack8(acc);
 }
 
-// Trilinear nodal interpolation with scale and optional addend:
-// Y[i][c] = scale * (P X)[i][c] + (add ? add[i][c] : 0).
-__global__ void __launch_bounds__(256) k_up(const bf16_t* __restrict__ X, int C, G3 gc, G3 gf, float scale,
-                                            const bf16_t* __restrict__ add, bf16_t* __restrict__ Y) {
+// The trilinear value of 8 channels at fine node v (x, y, z): w times the sum of
+// the 1 to 8 coarse nodes around it, in (z, y, x) order.  All 8 are loaded (those
+// of an even coordinate twice) and the repeats left out of the sum.
+__device__ __forceinline__ void up_value(const bf16_t* __restrict__ X, int C, const G3& gc, const G3& gf, int v, int q,
+                                         float acc[8]) {
+    const int z = v / (gf.nx * gf.ny), r = v - z * gf.nx * gf.ny, y = r / gf.nx, x = r - y * gf.nx;
+    uint4 u[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int xs = (x + (e & 1)) >> 1, ys = (y + ((e >> 1) & 1)) >> 1, zs = (z + (e >> 2)) >> 1;
+        u[e] = *reinterpret_cast<const uint4*>(X + ((size_t)(zs * gc.ny + ys) * gc.nx + xs) * C + 8 * q);
+    }
+    const int n = ((x & 1) + 1) * ((y & 1) + 1) * ((z & 1) + 1);
+    const float w = 1.f / (float)n;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k] = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const bool use = (!(e & 1) || (x & 1)) && (!(e & 2) || (y & 1)) && (!(e & 4) || (z & 1));
+        float f[8];
+        unpack8(u[e], f);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] = use ? acc[k] + w * f[k] : acc[k];
+    }
+}
+// Interpolation with scale and addend: Y[i][c] = scale * (P X)[i][c] + add[i][c],
+// add with ld channels a node, its C from channel off on.
+__global__ void __launch_bounds__(kThreads) k_up_add(const bf16_t* __restrict__ X, int C, G3 gc, G3 gf, float scale,
+                                                     const bf16_t* __restrict__ add, int ld, int off,
+                                                     bf16_t* __restrict__ Y) {
     const int c8 = C / 8;
     const long i = (long)blockIdx.x * kThreads + threadIdx.x;
     if (i >= (long)gf.N * c8) return;
-    const int q = (int)(i % c8);
-    const int v = (int)(i / c8);
-    const int x = v % gf.nx, y = (v / gf.nx) % gf.ny, z = v / (gf.nx * gf.ny);
-    const int xs[2] = {x >> 1, (x + 1) >> 1}, ys[2] = {y >> 1, (y + 1) >> 1}, zs[2] = {z >> 1, (z + 1) >> 1};
-    const int nx_ = (x & 1) ? 2 : 1, ny_ = (y & 1) ? 2 : 1, nz_ = (z & 1) ? 2 : 1;
-    const float w = 1.f / (float)(nx_ * ny_ * nz_);
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int a = 0; a < nz_; ++a)
-        for (int b = 0; b < ny_; ++b)
-            for (int c = 0; c < nx_; ++c) {
-                float f[8];
-                unpack8(*reinterpret_cast<const uint4*>(X + ((size_t)(zs[a] * gc.ny + ys[b]) * gc.nx + xs[c]) * C + 8 * q), f);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] += w * f[e];
-            }
-    float ad[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (add) unpack8(*reinterpret_cast<const uint4*>(add + (size_t)v * C + 8 * q), ad);
+    const int v = (int)(i / c8), q = (int)(i - (long)v * c8);
+    float ad[8], acc[8];
+    const uint4 a = *reinterpret_cast<const uint4*>(add + (size_t)v * ld + off + 8 * q);
+    up_value(X, C, gc, gf, v, q, acc);
+    unpack8(a, ad);
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = scale * acc[e] + ad[e];
     *reinterpret_cast<uint4*>(Y + (size_t)v * C + 8 * q) = pack8(acc);
 }
-
-// Y[v] = [A[v] (Ca channels), B[v] (Cb channels)]; split is the inverse.
-__global__ void __launch_bounds__(256) k_concat(const bf16_t* __restrict__ A, int Ca, const bf16_t* __restrict__ B,
-                                                int Cb, int N, bf16_t* __restrict__ Y) {
-    const int c8 = (Ca + Cb) / 8;
+// The decoder's input Y[v] = [(P X)[v] (C channels), E[v] (Ce channels)].
+__global__ void __launch_bounds__(kThreads) k_up_concat(const bf16_t* __restrict__ X, int C, G3 gc, G3 gf,
+                                                        const bf16_t* __restrict__ E, int Ce, bf16_t* __restrict__ Y) {
+    const int c8 = (C + Ce) / 8;
     const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= (long)N * c8) return;
-    const int q = (int)(i % c8), v = (int)(i / c8);
-    const int c = 8 * q;
-    const uint4 val = c < Ca ? *reinterpret_cast<const uint4*>(A + (size_t)v * Ca + c)
-                             : *reinterpret_cast<const uint4*>(B + (size_t)v * Cb + (c - Ca));
-    *reinterpret_cast<uint4*>(Y + (size_t)v * (Ca + Cb) + c) = val;
-}
-__global__ void __launch_bounds__(256) k_split(const bf16_t* __restrict__ Y, int Ca, int Cb, int N,
-                                               bf16_t* __restrict__ A, bf16_t* __restrict__ B) {
-    const int c8 = (Ca + Cb) / 8;
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= (long)N * c8) return;
-    const int q = (int)(i % c8), v = (int)(i / c8);
-    const int c = 8 * q;
-    const uint4 val = *reinterpret_cast<const uint4*>(Y + (size_t)v * (Ca + Cb) + c);
-    if (c < Ca) *reinterpret_cast<uint4*>(A + (size_t)v * Ca + c) = val;
-    else *reinterpret_cast<uint4*>(B + (size_t)v * Cb + (c - Ca)) = val;
+    if (i >= (long)gf.N * c8) return;
+    const int v = (int)(i / c8), q = (int)(i - (long)v * c8);
+    uint4 val;
+    if (8 * q < C) {
+        float acc[8];
+        up_value(X, C, gc, gf, v, q, acc);
+        val = pack8(acc);
+    } else {
+        val = *reinterpret_cast<const uint4*>(E + (size_t)v * Ce + 8 * q - C);
+    }
+    *reinterpret_cast<uint4*>(Y + (size_t)v * (C + Ce) + 8 * q) = val;
 }
 
-// Component-major float32 in[c * N + v] (c < n) -> bf16 X[v * Cp + c] (zero padded).
-__global__ void __launch_bounds__(256) k_pack_soa(const float* __restrict__ in, int n, int Cp, int N,
-                                                  bf16_t* __restrict__ X) {
-    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= (long)N * Cp) return;
-    const int c = (int)(i % Cp), v = (int)(i / Cp);
-    X[i] = c < n ? f2bf(in[(size_t)c * N + v]) : (bf16_t)0;
+// Component-major float32 in[c * N + v] (c < n) -> bf16 X[v * Cp + c] (zero
+// padded), 64 nodes x 16 channels a workgroup (blockIdx.y: the channels) through
+// LDS: nodes fastest on the way in, channels on the way out.
+__global__ void __launch_bounds__(kThreads) k_pack_soa(const float* __restrict__ in, int n, int Cp, int N,
+                                                       bf16_t* __restrict__ X) {
+    __shared__ bf16_t sh[64][16 + 2];
+    const int v0 = blockIdx.x * 64, c0 = blockIdx.y * 16, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int c = c0 + 4 * k + w, v = v0 + lane;
+        sh[lane][4 * k + w] = c < n && v < N ? f2bf(in[(size_t)c * N + v]) : (bf16_t)0;
+    }
+    __syncthreads();
+    const int v = threadIdx.x >> 2, q = (threadIdx.x & 3) * 4;
+    if (v0 + v >= N) return;
+    const bf16_t* p = &sh[v][q];
+    *reinterpret_cast<uint2*>(X + (size_t)(v0 + v) * Cp + c0 + q) =
+        make_uint2(p[0] | ((uint32_t)p[1] << 16), p[2] | ((uint32_t)p[3] << 16));
 }
 // bf16 X[v * Cp + c] -> float32 out[c * N + v] for c < n.
 __global__ void __launch_bounds__(256) k_unpack_soa(const bf16_t* __restrict__ X, int n, int Cp, int N,
