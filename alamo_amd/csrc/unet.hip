@@ -38,13 +38,14 @@ constexpr int kWgradBlocks = 256;  // target workgroups of one weight-gradient l
 constexpr int kBiasBlocks = 256;   // most workgroups (bias partials) of k_wgrad_dz
 
 inline unsigned nb256(long n) { return (unsigned)((n + 255) / 256); }
+inline unsigned nb64(long n) { return (unsigned)((n + 63) / 64); }
 inline int pad16(int c) { return (c + 15) / 16 * 16; }
 
 struct ConvL {
     int cin, cout, cinp, coutp, level;
     bool relu;
     long woff, boff;  // offsets of W and b in the canonical parameter vector
-    bf16_t* wt = nullptr;  // [coutp][27 cinp]
+    bf16_t* wt = nullptr;  // [coutp][27 cinp] (aunet::frag_index)
     bf16_t* wb = nullptr;  // [cinp][27 coutp], taps flipped
 };
 
@@ -95,25 +96,33 @@ int nalloc_t(alamo_nn_t nn, T** p, size_t count) {
 
 void launch_conv(const bf16_t* X, int Cin, const bf16_t* W, const float* bias, int Cout, const G3& g, int relu,
                  bf16_t* Y, float* Yf, int yf_ch, hipStream_t s) {
-    const dim3 grid((unsigned)((g.N + 63) / 64), 1);
     // Levels whose one-wave-per-16-nodes grid leaves most of the 256 CUs
     // idle split K over 4 waves a workgroup, 16 channels a workgroup
     // (ALAMO_NN_KSPLIT=0 never, 2 on every level; read at every launch).
     const char* ks_env = std::getenv("ALAMO_NN_KSPLIT");
     const int ksplit = ks_env ? std::atoi(ks_env) : 1;
-    const long plain_wg = (long)grid.x * (Cout % 64 == 0 ? Cout / 64 : Cout % 32 == 0 ? Cout / 32 : Cout / 16);
+    const long wg4 = (g.N + 63) / 64;
+    const long plain_wg = wg4 * (Cout % 64 == 0 ? Cout / 64 : Cout % 32 == 0 ? Cout / 32 : Cout / 16);
     const bool ks = ksplit == 2 || (ksplit == 1 && plain_wg < 256);
+    const unsigned wg = (unsigned)((g.N + 15) / 16);
+    // 32 nodes a wave read the weights half as often, 16 nodes make twice the
+    // waves: even at 49 x 41 x 33 nodes, 2 waves of 32 a SIMD (174.0 us the
+    // network's pass, 175.9 with 32), 383 us with 32 against 389 at 65^3 (8 a
+    // SIMD), 1043 against 1183 at 97^3.
+    const bool two = wg / 2 >= 8 * 4 * 256;
     auto go = [&](auto cin_tag) {
         constexpr int CIN = decltype(cin_tag)::value;
         if (ks)
-            aunet::k_conv_fwd_ks<1, 4, CIN><<<dim3((unsigned)((g.N + 15) / 16), Cout / 16), 256, 0, s>>>(
-                X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+            aunet::k_conv_fwd_ks<1, 4, CIN><<<dim3(wg, Cout / 16), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
         else if (Cout % 64 == 0)
-            aunet::k_conv_fwd<4, CIN><<<dim3(grid.x, Cout / 64), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+            aunet::k_conv_fwd<1, 4, CIN><<<dim3(wg, Cout / 64), 64, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
         else if (Cout % 32 == 0)
-            aunet::k_conv_fwd<2, CIN><<<dim3(grid.x, Cout / 32), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+            aunet::k_conv_fwd<1, 2, CIN><<<dim3(wg, Cout / 32), 64, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+        else if (two)
+            aunet::k_conv_fwd<2, 1, CIN><<<dim3((wg + 1) / 2, Cout / 16), 64, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf,
+                                                                                      yf_ch);
         else
-            aunet::k_conv_fwd<1, CIN><<<dim3(grid.x, Cout / 16), 256, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
+            aunet::k_conv_fwd<1, 1, CIN><<<dim3(wg, Cout / 16), 64, 0, s>>>(X, Cin, W, bias, Cout, g, relu, Y, Yf, yf_ch);
     };
     switch (Cin) {  // the network's own channel counts; an input padded to another takes the general form
         case 16: go(std::integral_constant<int, 16>{}); break;
@@ -203,15 +212,15 @@ int forward(alamo_nn_t nn, const float* in, float* out, hipStream_t s) {
         conv_fwd(nn, 2 * l, h, nn->A[l], nullptr, s);
         conv_fwd(nn, 2 * l + 1, nn->A[l], nn->E[l], nullptr, s);
         if (l + 1 < kLevels) {
-            const long n = (long)g[l + 1].N * kCh[l] / 8;
-            aunet::k_down<<<nb256(n), 256, 0, s>>>(nn->E[l], kCh[l], kCh[l], g[l], g[l + 1], 0.125f, nn->D[l + 1]);
+            const long n = (long)g[l + 1].N * kCh[l] / 2;
+            aunet::k_down<<<nb64(n), aunet::kWave, 0, s>>>(nn->E[l], kCh[l], kCh[l], g[l], g[l + 1], 0.125f, nn->D[l + 1]);
             h = nn->D[l + 1];
         }
     }
     const bf16_t* up_in = nn->E[kLevels - 1];
     for (int l = kLevels - 2; l >= 0; --l) {
         const int cu = kCh[l + 1], ce = kCh[l];
-        aunet::k_up_concat<<<nb256((long)g[l].N * (cu + ce) / 8), 256, 0, s>>>(up_in, cu, g[l + 1], g[l], nn->E[l], ce,
+        aunet::k_up_concat<<<nb64((long)g[l].N * (cu + ce) / 8), aunet::kWave, 0, s>>>(up_in, cu, g[l + 1], g[l], nn->E[l], ce,
                                                                                nn->K[l]);
         const int li = 2 * kLevels + 2 * (kLevels - 2 - l);
         conv_fwd(nn, li, nn->K[l], nn->B[l], nullptr, s);
@@ -238,13 +247,13 @@ int backward(alamo_nn_t nn, const float* dout, float* grad, float* din, hipStrea
         conv_back(nn, li, nn->K[l], nn->B[l], nn->gB[l], nn->gK[l], grad, s);
         // adjoint of trilinear up: 8 x full weighting, of the decoder input's first cu channels
         bf16_t* dst = (l + 1 < kLevels - 1) ? nn->gG[l + 1] : nn->gE[kLevels - 1];
-        aunet::k_down<<<nb256((long)g[l + 1].N * cu / 8), 256, 0, s>>>(nn->gK[l], cu + ce, cu, g[l], g[l + 1], 1.f, dst);
+        aunet::k_down<<<nb64((long)g[l + 1].N * cu / 2), aunet::kWave, 0, s>>>(nn->gK[l], cu + ce, cu, g[l], g[l + 1], 1.f, dst);
     }
     for (int l = kLevels - 1; l >= 0; --l) {
         if (l < kLevels - 1) {
             // adjoint of down (full weighting / 8): up / 8, plus the skip-path
             // gradient, the last channels of the decoder input's
-            aunet::k_up_add<<<nb256((long)g[l].N * kCh[l] / 8), 256, 0, s>>>(nn->gD[l + 1], kCh[l], g[l + 1], g[l], 0.125f,
+            aunet::k_up_add<<<nb64((long)g[l].N * kCh[l] / 8), aunet::kWave, 0, s>>>(nn->gD[l + 1], kCh[l], g[l + 1], g[l], 0.125f,
                                                                              nn->gK[l], kCh[l + 1] + kCh[l], kCh[l + 1],
                                                                              nn->gE[l]);
         }
@@ -338,7 +347,10 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
     long partmax = 0, xmax = 0, zmax = 0;
     for (auto& L : nn->cv) {
         const long M = (long)L.coutp * 27 * L.cinp;
-        if ((rc = nalloc_t(nn, &L.wt, M)) || (rc = nalloc_t(nn, &L.wb, M))) return cleanup(rc);
+        const size_t nwt = aunet::frag_size(27 * L.cinp, L.coutp), nwb = aunet::frag_size(27 * L.coutp, L.cinp);
+        if ((rc = nalloc_t(nn, &L.wt, nwt)) || (rc = nalloc_t(nn, &L.wb, nwb))) return cleanup(rc);
+        NNCHK(hipMemset(L.wt, 0, sizeof(bf16_t) * nwt));
+        NNCHK(hipMemset(L.wb, 0, sizeof(bf16_t) * nwb));
         const WgradGrid w = wgrad_grid(nn->g[L.level], (L.cinp / 16) * (L.coutp / 16));
         partmax = std::max(partmax, M * w.nchunk);
         xmax = std::max(xmax, 3L * L.cinp * 8 * w.ngroup);
