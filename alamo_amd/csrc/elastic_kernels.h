@@ -448,8 +448,7 @@ __device__ __forceinline__ void gradc_matrix_mm(const double* __restrict__ C, co
 
 // sigma = C : A for MajorMinor C, streamed over the slots (contract2).
 template <typename T>
-__device__ __forceinline__ void contract2_mm_stream(const T* __restrict__ C, long N, long id, const T A[3][3],
-                                                    T sg[3][3]) {
+__device__ __forceinline__ void contract2_mm(const T C[21], const T A[3][3], T sg[3][3]) {
     T e1[6], sp[6];
 #pragma unroll
     for (int Q = 0; Q < 6; ++Q) {
@@ -460,9 +459,8 @@ __device__ __forceinline__ void contract2_mm_stream(const T* __restrict__ C, lon
 #pragma unroll
     for (int s = 0; s < 21; ++s) {
         const int P = slot_p(s), Q = slot_q(s);
-        const T c = C[s * N + id];
-        sp[P] += c * e1[Q];
-        if (Q != P) sp[Q] += c * e1[P];
+        sp[P] += C[s] * e1[Q];
+        if (Q != P) sp[Q] += C[s] * e1[P];
     }
 #pragma unroll
     for (int P = 0; P < 6; ++P) sg[pair_a(P)][pair_b(P)] = sg[pair_b(P)][pair_a(P)] = sp[P];
@@ -471,38 +469,62 @@ __device__ __forceinline__ void contract2_mm_stream(const T* __restrict__ C, lon
 // Boundary row of Fapply at node (i, j, k) of region reg with normal nrm:
 // one-sided gradients, sigma = C : grad u, and the Constant BC row.  u may be
 // narrower than T (widened exactly).  PER false: no axis of L is periodic.
+// C slot s of the node at C[s * cN + cid] (a separate layout of C), or at
+// C[s * N + id] by default.  Every load leaves before the arithmetic and the
+// spacings enter as reciprocals: on the small levels these rows are the longest
+// path of a launch (an FP64 sweep at 8 x 6 x 7 nodes 4.31 -> 4.06 us, isotropic at
+// 5^3 4.36 -> 3.85, against a wait per group of loads and nine divisions).
 template <typename T, int SYM, typename TU = T, bool PER = true>
 __device__ __forceinline__ void apply_boundary(const TU* __restrict__ u, const T* __restrict__ C,
-                                               const int* __restrict__ bct, const Lvl& L, int i, int j, int k,
-                                               long id, int reg, const T nrm[3], T out[3], long cN = -1,
+                                               const int* __restrict__ bct, const Lvl& L, const Spc<T>& H, int i, int j,
+                                               int k, long id, int reg, const T nrm[3], T out[3], long cN = -1,
                                                long cid = -1) {
-    // C slot s of the node at C[s * cN + cid] (a separate layout of C), or at
-    // C[s * N + id] by default
-    const long N = L.N, sy = L.nx, sz = (long)L.nx * L.ny;
+    constexpr int NC = NComp<SYM>::value;
     if (cN < 0) {
-        cN = N;
+        cN = L.N;
         cid = id;
     }
-    const T hx = T(L.dx), hy = T(L.dy), hz = T(L.dz);
+    int t3[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) t3[c] = bct[3 * reg + c];
+    // the gradient along an axis, as d1's: (u[id + o[0]] - u[id + o[1]]) * w, one-sided on a face
+    long o[3][2];
+    T w[3];
+    const int pos[3] = {i, j, k}, n[3] = {L.nx, L.ny, L.nz};
+    const long stride[3] = {1, L.nx, (long)L.nx * L.ny};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool lo = pos[a] == 0, hi = pos[a] == n[a] - 1, per = PER && ((L.per >> a) & 1);
+        const long wrap = per ? (long)(n[a] - 2) * stride[a] : 0;
+        o[a][0] = hi ? -wrap : stride[a];
+        o[a][1] = lo ? wrap : -stride[a];
+        w[a] = (lo || hi) && !per ? T(2) * H.h2[a] : H.h2[a];
+    }
+    TU v[3][7];
+    T c[NC];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        const TU* f = u + p * L.N + id;
+        v[p][0] = f[0];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            v[p][1 + 2 * a] = f[o[a][0]];
+            v[p][2 + 2 * a] = f[o[a][1]];
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < NC; ++s) c[s] = C[s * cN + cid];
+    __builtin_amdgcn_sched_barrier(0);
     T uu[3], gu[3][3], sg[3][3];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-        const TU* f = u + p * N;
-        uu[p] = (T)f[id];
-        gu[p][0] = d1(f, id, 1, i, L.nx, hx, PER && (L.per & 1));
-        gu[p][1] = d1(f, id, sy, j, L.ny, hy, PER && ((L.per >> 1) & 1));
-        gu[p][2] = d1(f, id, sz, k, L.nz, hz, PER && ((L.per >> 2) & 1));
-    }
-    if constexpr (SYM == 1) {
-        contract2_mm_stream<T>(C, cN, cid, gu, sg);
-    } else {
-        constexpr int NC = NComp<SYM>::value;
-        T c[NC];
+        uu[p] = (T)v[p][0];
 #pragma unroll
-        for (int s = 0; s < NC; ++s) c[s] = C[s * cN + cid];
-        contract2<T, SYM>(c, gu, sg);
+        for (int a = 0; a < 3; ++a) gu[p][a] = ((T)v[p][1 + 2 * a] - (T)v[p][2 + 2 * a]) * w[a];
     }
-    bc_set<T>(bct + 3 * reg, uu, gu, sg, nrm, out);
+    if constexpr (SYM == 1) contract2_mm<T>(c, gu, sg);
+    else contract2<T, SYM>(c, gu, sg);
+    bc_set<T>(t3, uu, gu, sg, nrm, out);
 }
 
 // Interior row of Fapply for an isotropic C = (lambda, mu), the sums of contract3
@@ -715,7 +737,7 @@ __device__ __forceinline__ void apply_node(const T* __restrict__ u, const T* __r
                                            int k, long id, T out[3], unsigned gmask = 7u) {
     T nrm[3];
     const int reg = region_of<T>(i, j, k, L, nrm);
-    if (reg >= 0) apply_boundary<T, SYM>(u, C, bct, L, i, j, k, id, reg, nrm, out);
+    if (reg >= 0) apply_boundary<T, SYM>(u, C, bct, L, Spc<T>(L), i, j, k, id, reg, nrm, out);
     else if (L.per && on_face(L, i, j, k)) apply_interior_wrap<T, SYM>(u, C, uniform, L, i, j, k, id, out);
     else apply_interior<T, SYM>(u, C, uniform, L, id, out, gmask);
 }

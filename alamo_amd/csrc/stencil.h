@@ -21,6 +21,28 @@ __device__ __forceinline__ T finish_op(T Ax, T xv, T bv, T dv, T omega) {
     else return (T(1) - omega) * xv + omega * (bv - (Ax - xv * dv)) / dv;
 }
 
+// The operands of finish_op at node n32, and its results' stores.  The boundary
+// rows load them ahead of the row's own loads, so that they wait once.
+template <typename T, int OP, typename TX>
+__device__ __forceinline__ void load_operands(const TX* __restrict__ x, const T* __restrict__ b,
+                                              const T* __restrict__ diag, const Lvl& L, unsigned n32, T xv[3], T bv[3],
+                                              T dv[3]) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        const size_t off = (size_t)p * L.N;
+        xv[p] = (OP == 2) ? (T)ld32(x + off, n32) : T(0);
+        bv[p] = (OP >= 1) ? ld32(b + off, n32) : T(0);
+        dv[p] = (OP == 2) ? ld32(diag + off, n32) : T(1);
+    }
+}
+template <typename T, int OP>
+__device__ __forceinline__ void store_row(T* __restrict__ out, const Lvl& L, unsigned n32, const T o[3], const T xv[3],
+                                          const T bv[3], const T dv[3], T omega) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+        st32(out + (size_t)p * L.N, n32, finish_op<T, OP>(o[p], xv[p], bv[p], dv[p], omega));
+}
+
 // One thread per node over the whole box (XCD-remapped), any OP.
 template <typename T, int SYM, int OP>
 __global__ void __launch_bounds__(kBlock)
@@ -183,19 +205,20 @@ __global__ void __launch_bounds__(kBlock)
                    const T* __restrict__ Dc, int nflag, T* __restrict__ out, Spc<T> H) {
     int i, j, k;
     long id;
-    T o[3];
+    T o[3], xv[3], bv[3], dv[3];
     if (blockIdx.x < nbb) {
         const long t = (long)blockIdx.x * kBlock + threadIdx.x;
         if (t >= boundary_count(L)) return;
         boundary_node(L, t, i, j, k);
         id = ((long)k * L.ny + j) * L.nx + i;
+        load_operands<T, OP>(x, b, diag, L, (unsigned)id, xv, bv, dv);
         T nrm[3];
         const int reg = region_of<T, PER>(i, j, k, L, nrm);
         if constexpr (PER) {
-            if (reg >= 0) apply_boundary<T, SYM, T, true>(x, C, bct, L, i, j, k, id, reg, nrm, o);
+            if (reg >= 0) apply_boundary<T, SYM, T, true>(x, C, bct, L, H, i, j, k, id, reg, nrm, o);
             else apply_interior_wrap<T, SYM>(x, C, uniform, L, i, j, k, id, o);  // a periodic face
         } else {
-            apply_boundary<T, SYM, T, false>(x, C, bct, L, i, j, k, id, reg, nrm, o);
+            apply_boundary<T, SYM, T, false>(x, C, bct, L, H, i, j, k, id, reg, nrm, o);
         }
     } else {
         const long ib = (long)(blockIdx.x - nbb);
@@ -203,15 +226,15 @@ __global__ void __launch_bounds__(kBlock)
         if constexpr (SYM == 1 && DC) {
             // Every load of the node leaves first (the 19-point u neighbourhood,
             // C, the mask, the wave's first D position and the OP operands),
-            // ahead of the arithmetic: on the latency-bound small levels the
-            // kernel then waits on memory twice (these, then D), not once per
-            // group of loads the compiler would otherwise interleave.
+            // ahead of the arithmetic, and D as soon as the mask is there: on the
+            // latency-bound small levels the kernel then waits on memory once, not
+            // once per group of loads the compiler would otherwise interleave.
             const unsigned o32 = (unsigned)id;
             // wave-uniform; readfirstlane (convergent) keeps the load ahead of
             // the flagged-lanes branch, where the compiler would otherwise sink it
             const int dwb = __builtin_amdgcn_readfirstlane(dwbase[ib * kWavesPerBlock + threadIdx.x / 64]);
             const unsigned gm = gmask[id];  // the compact-D launch always passes the mask
-            T uv[3][19], cv[21], xv[3], bv[3], dv[3];
+            T uv[3][19], cv[21];
             mm_load<T>(x, C, L, o32, uv, cv);
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
@@ -221,15 +244,22 @@ __global__ void __launch_bounds__(kBlock)
                 dv[p] = (OP == 2) ? ld32(diag + off, o32) : T(1);
             }
             __builtin_amdgcn_sched_barrier(0);
+            const bool flagged = !uniform && gm != 0u;
+            const unsigned long long bal = __ballot(gm != 0u);
+            T D[18];
+            if (flagged) {
+                const unsigned p = (unsigned)dwb + (unsigned)__popcll(bal & lanes_below());
+#pragma unroll
+                for (int q = 0; q < 18; ++q) D[q] = ld32(Dc + (size_t)q * nflag, p);
+            }
+            __builtin_amdgcn_sched_barrier(0);
             T e1[6];
             mm_compute<T>(uv, cv, H, o, e1);
-            const unsigned long long bal = __ballot(gm != 0u);
-            if (!uniform && gm != 0u) {
-                const unsigned p = (unsigned)dwb + (unsigned)__popcll(bal & lanes_below());
+            if (flagged) {
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
 #pragma unroll
-                    for (int Q = 0; Q < 6; ++Q) o[r] += ld32(Dc + (size_t)(6 * r + Q) * nflag, p) * e1[Q];
+                    for (int Q = 0; Q < 6; ++Q) o[r] += D[6 * r + Q] * e1[Q];
             }
 #pragma unroll
             for (int p = 0; p < 3; ++p)
@@ -239,7 +269,7 @@ __global__ void __launch_bounds__(kBlock)
             // Every load of the node first, as for MajorMinor; the Jacobi
             // diagonal from the lambda and mu already there instead of a load.
             const unsigned o32 = (unsigned)id;
-            T uv[3][15], cv[2][7], bv[3], dg[3];
+            T uv[3][15], cv[2][7], dg[3];
             iso_load<T>(x, C, L, o32, uv, cv);
 #pragma unroll
             for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1) ? ld32(b + (size_t)p * L.N, o32) : T(0);
@@ -251,17 +281,10 @@ __global__ void __launch_bounds__(kBlock)
             return;
         } else {
             apply_interior<T, SYM>(x, C, uniform, L, id, o, gmask ? (unsigned)gmask[id] : 7u);
+            load_operands<T, OP>(x, b, diag, L, (unsigned)id, xv, bv, dv);
         }
     }
-    const unsigned n32 = (unsigned)id;
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-        const size_t off = (size_t)p * L.N;
-        const T xv = (OP == 2) ? ld32(x + off, n32) : T(0);
-        const T bv = (OP >= 1) ? ld32(b + off, n32) : T(0);
-        const T dv = (OP == 2) ? ld32(diag + off, n32) : T(1);
-        st32(out + off, n32, finish_op<T, OP>(o[p], xv, bv, dv, omega));
-    }
+    store_row<T, OP>(out, L, (unsigned)id, o, xv, bv, dv, omega);
 }
 
 // gmask of every interior node: bit a set iff some slot of C differs between

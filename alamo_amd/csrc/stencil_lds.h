@@ -366,28 +366,21 @@ __global__ void __launch_bounds__(TS::NT)
         int i, j, k;
         boundary_node(L, t, i, j, k);
         const long id = ((long)k * L.ny + j) * L.nx + i;
-        T nrm[3], o[3];
+        T nrm[3], o[3], xv[3], bv[3], dv[3];
         const int reg = region_of<T, PER>(i, j, k, L, nrm);
         if constexpr (PER) {
-            if (reg >= 0) apply_boundary<T, 1, TX, true>(x, Cb, bct, L, i, j, k, id, reg, nrm, o, boundary_count(L), t);
+            if (reg >= 0) apply_boundary<T, 1, TX, true>(x, Cb, bct, L, H, i, j, k, id, reg, nrm, o, boundary_count(L), t);
             else apply_interior_wrap<T, 1, TX>(x, Cf, uniform, L, i, j, k, id, o);  // a periodic face: the level's C
         } else if constexpr (CM == 2) {
             // the node's tensor from the palette (Ct is the table): the values
             // of the compact copy, so the same bits, from a row in the caches
-            apply_boundary<T, 1, TX, false>(x, Ct + (size_t)pidx_b[t] * kPalStride, bct, L, i, j, k, id, reg, nrm, o,
+            apply_boundary<T, 1, TX, false>(x, Ct + (size_t)pidx_b[t] * kPalStride, bct, L, H, i, j, k, id, reg, nrm, o,
                                             1, 0);
         } else {
-            apply_boundary<T, 1, TX, false>(x, Cb, bct, L, i, j, k, id, reg, nrm, o, boundary_count(L), t);
+            apply_boundary<T, 1, TX, false>(x, Cb, bct, L, H, i, j, k, id, reg, nrm, o, boundary_count(L), t);
         }
-        const unsigned n32 = (unsigned)id;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            const size_t off = (size_t)p * L.N;
-            const T xv = (OP == 2) ? (T)ld32(x + off, n32) : T(0);
-            const T bv = (OP >= 1) ? ld32(b + off, n32) : T(0);
-            const T dv = (OP == 2) ? ld32(diag + off, n32) : T(1);
-            st32(out + off, n32, finish_op<T, OP>(o[p], xv, bv, dv, omega));
-        }
+        load_operands<T, OP>(x, b, diag, L, (unsigned)id, xv, bv, dv);
+        store_row<T, OP>(out, L, (unsigned)id, o, xv, bv, dv, omega);
         return;
     }
     const long ib = (long)(kBoundaryLast ? blockIdx.x : blockIdx.x - nbb);
@@ -615,19 +608,12 @@ __global__ void __launch_bounds__(TS::NT) __attribute__((amdgpu_waves_per_eu(4))
         int i, j, k;
         boundary_node(L, t, i, j, k);
         const long id = ((long)k * L.ny + j) * L.nx + i;
-        T nrm[3], o[3];
+        T nrm[3], o[3], xv[3], bv[3], dv[3];
+        load_operands<T, OP>(x, b, diag, L, (unsigned)id, xv, bv, dv);
         const int reg = region_of<T, PER>(i, j, k, L, nrm);
-        if (!PER || reg >= 0) apply_boundary<T, 0, T, PER>(x, C, bct, L, i, j, k, id, reg, nrm, o);
+        if (!PER || reg >= 0) apply_boundary<T, 0, T, PER>(x, C, bct, L, H, i, j, k, id, reg, nrm, o);
         else apply_interior_wrap<T, 0>(x, C, uniform, L, i, j, k, id, o);  // a periodic face
-        const unsigned n32 = (unsigned)id;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            const size_t off = (size_t)p * L.N;
-            const T xv = (OP == 2) ? ld32(x + off, n32) : T(0);
-            const T bv = (OP >= 1) ? ld32(b + off, n32) : T(0);
-            const T dv = (OP == 2) ? ld32(diag + off, n32) : T(1);
-            st32(out + off, n32, finish_op<T, OP>(o[p], xv, bv, dv, omega));
-        }
+        store_row<T, OP>(out, L, (unsigned)id, o, xv, bv, dv, omega);
         return;
     }
     int it, jt, kc;
