@@ -345,16 +345,22 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
     NNCHK(hipMemset(nn->m, 0, sizeof(float) * np));
     NNCHK(hipMemset(nn->v, 0, sizeof(float) * np));
     long partmax = 0, xmax = 0, zmax = 0;
+    size_t nweights = 0;
     for (auto& L : nn->cv) {
         const long M = (long)L.coutp * 27 * L.cinp;
-        const size_t nwt = aunet::frag_size(27 * L.cinp, L.coutp), nwb = aunet::frag_size(27 * L.coutp, L.cinp);
-        if ((rc = nalloc_t(nn, &L.wt, nwt)) || (rc = nalloc_t(nn, &L.wb, nwb))) return cleanup(rc);
-        NNCHK(hipMemset(L.wt, 0, sizeof(bf16_t) * nwt));
-        NNCHK(hipMemset(L.wb, 0, sizeof(bf16_t) * nwb));
+        nweights += aunet::frag_size(27 * L.cinp, L.coutp) + aunet::frag_size(27 * L.coutp, L.cinp);
         const WgradGrid w = wgrad_grid(nn->g[L.level], (L.cinp / 16) * (L.coutp / 16));
         partmax = std::max(partmax, M * w.nchunk);
         xmax = std::max(xmax, 3L * L.cinp * 8 * w.ngroup);
         zmax = std::max(zmax, (long)L.coutp * 8 * w.ngroup);
+    }
+    bf16_t* w = nullptr;  // every layer's packed weights
+    if ((rc = nalloc_t(nn, &w, nweights))) return cleanup(rc);
+    NNCHK(hipMemset(w, 0, sizeof(bf16_t) * nweights));
+    for (auto& L : nn->cv) {
+        L.wt = w;
+        L.wb = L.wt + aunet::frag_size(27 * L.cinp, L.coutp);
+        w = L.wb + aunet::frag_size(27 * L.coutp, L.cinp);
     }
     if ((rc = nalloc_t(nn, &nn->part, partmax)) || (rc = nalloc_t(nn, &nn->bpart, (long)kBiasBlocks * kCh[kLevels - 1])) ||
         (rc = nalloc_t(nn, &nn->trx, xmax)) || (rc = nalloc_t(nn, &nn->trz, zmax)) ||
