@@ -150,16 +150,25 @@ def _check(rc: int, what: str) -> int:
     return rc
 
 
+_torch_mod = None
+
+
 def _torch():
-    import torch
-    if not torch.cuda.is_available():
-        raise AlamoError("no GPU: the elastic operator runs on the HIP device only")
-    return torch
+    """The torch module, once a GPU was found: the question costs 1.4 us, and the
+    wrappers ask it several times a call."""
+    global _torch_mod
+    if _torch_mod is None:
+        import torch
+        if not torch.cuda.is_available():
+            raise AlamoError("no GPU: the elastic operator runs on the HIP device only")
+        _torch_mod = torch
+    return _torch_mod
 
 
 def _stream():
     torch = _torch()
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the device by number: asked for without it, the stream takes 1.3 us longer
+    return ctypes.c_void_p(torch.cuda.current_stream(torch.cuda.current_device()).cuda_stream)
 
 
 def _ptr(t):
@@ -194,6 +203,11 @@ class ElasticOperator:
         nl = ctypes.c_int()
         _check(lib().alamo_el_num_levels(h, ctypes.byref(nl)), "alamo_el_num_levels")
         self.num_levels = nl.value
+        self._shapes = []             # (nz, ny, nx) of each level, fixed at creation
+        for lev in range(self.num_levels):
+            n = (ctypes.c_int * 3)()
+            _check(lib().alamo_el_level_nodes(h, lev, n), "alamo_el_level_nodes")
+            self._shapes.append((n[2], n[1], n[0]))
         self._bc = _bc.Constant()
         self.periodic = (0, 0, 0)
         self.parent = None
@@ -233,9 +247,9 @@ class ElasticOperator:
 
     # -- set-up ---------------------------------------------------------------
     def level_shape(self, mglev: int = 0):
-        n = (ctypes.c_int * 3)()
-        _check(lib().alamo_el_level_nodes(self._h, mglev, n), "alamo_el_level_nodes")
-        return (n[2], n[1], n[0])
+        if not 0 <= mglev < self.num_levels:
+            raise AlamoError(f"alamo_el_level_nodes: level {mglev} out of range [0, {self.num_levels})")
+        return self._shapes[mglev]
 
     def SetBC(self, bc: _bc.Constant):
         t = np.ascontiguousarray(bc.type, dtype=np.int32)
