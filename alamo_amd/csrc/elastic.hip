@@ -2199,24 +2199,42 @@ int fgmres_solve(alamo_el_t h, double* x, const double* b, double target, const 
         // DCGS2's two passes over V for step jj, then |w|^2, and the copy of
         // the coefficients into the host buffer of jj's parity; the event of
         // that parity marks the copy done.
-        auto dcgs2_passes = [&](auto* V, long ld, int jj) {
+        // Returns the partials of |w|^2.
+        auto dcgs2_passes = [&](auto* V, long ld, int jj) -> int {
             using TV = std::remove_pointer_t<decltype(V)>;
-            const int n = jj + 1;
             if (jj == 0) {
                 ael::k_multidot_partial<TV><<<kDotBlocks, kBlock, 0, s>>>(V, 1, M0, ld, h->kw, h->kpart);
                 ael::k_multidot_final<<<1, kBlock, 0, s>>>(h->kpart, kDotBlocks, h->kh);
                 ael::k_multiaxpy_dot<false, TV><<<kDotBlocks, kBlock, 0, s>>>(h->kw, V, 1, M0, ld, h->kh, h->kpart);
-            } else {
-                double* sums = h->kh + 2 * (m + 1) + 2;  // the 2n sums of pass 1
-                ael::k_multidot2_partial<TV><<<kDotBlocks, kBlock, 0, s>>>(V, n, M0, ld, h->kw, h->kpart);
-                ael::k_multidot_final<<<2 * n, kBlock, 0, s>>>(h->kpart, kDotBlocks, sums);
-                ael::k_dcgs2_update<TV><<<kDotBlocks, kBlock, 0, s>>>(V, n, M0, ld, h->kw, sums, h->kh, h->kpart);
+                return kDotBlocks;
             }
+            double* sums = h->kh + 2 * (m + 1) + 2;  // the 2n sums of pass 1
+            const int nb = (int)std::min<long>(kDotBlocks, std::max<long>(1, nblk(M0 / 4)));
+            auto go = [&](auto k_tag) {
+                constexpr int K = decltype(k_tag)::value;
+                ael::k_multidot2_partial<K, TV><<<nb, kBlock, 0, s>>>(V, M0, ld, h->kw, h->kpart);
+                ael::k_multidot_final<<<2 * (K + 1), kBlock, 0, s>>>(h->kpart, nb, sums);
+                ael::k_dcgs2_update<K, TV><<<nb, kBlock, 0, s>>>(V, M0, ld, h->kw, sums, h->kh, h->kpart);
+            };
+            static_assert(ael::kMultiDotMax == 12, "a case for every number of vectors before the last");
+            switch (jj) {
+                case 1: go(std::integral_constant<int, 1>{}); break;
+                case 2: go(std::integral_constant<int, 2>{}); break;
+                case 3: go(std::integral_constant<int, 3>{}); break;
+                case 4: go(std::integral_constant<int, 4>{}); break;
+                case 5: go(std::integral_constant<int, 5>{}); break;
+                case 6: go(std::integral_constant<int, 6>{}); break;
+                case 7: go(std::integral_constant<int, 7>{}); break;
+                case 8: go(std::integral_constant<int, 8>{}); break;
+                case 9: go(std::integral_constant<int, 9>{}); break;
+                case 10: go(std::integral_constant<int, 10>{}); break;
+                default: go(std::integral_constant<int, 11>{}); break;
+            }
+            return nb;
         };
         auto launch_dcgs2 = [&](int jj) -> int {
-            if (v32) dcgs2_passes(reinterpret_cast<float*>(h->kv), MPf, jj);
-            else dcgs2_passes(h->kv, MP, jj);
-            ael::k_multidot_final<<<1, kBlock, 0, s>>>(h->kpart, kDotBlocks, nrm_slot);
+            const int nb = v32 ? dcgs2_passes(reinterpret_cast<float*>(h->kv), MPf, jj) : dcgs2_passes(h->kv, MP, jj);
+            ael::k_multidot_final<<<1, kBlock, 0, s>>>(h->kpart, nb, nrm_slot);
             const long nv = 2 * (m + 1) + 2;
             HIPCHK(hipMemcpyAsync(h->red_host_vec + (jj & 1) * nv, h->kh, sizeof(double) * nv, hipMemcpyDeviceToHost,
                                   s));

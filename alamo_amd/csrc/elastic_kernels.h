@@ -1648,58 +1648,54 @@ __global__ void __launch_bounds__(kBlock) k_multiaxpy_dot(double* __restrict__ w
 // V may hold FP32 vectors (TV = float): they are widened exactly, and every
 // sum is formed in FP64.
 //
+// Both passes are bound by memory.  K = n - 1 is a constant, so that a thread's
+// loads of 4 consecutive entries of every vector leave together, 16 bytes each
+// (the vectors start on 128-byte lines); entries past the last whole group of 4
+// go to the first workgroup.  129^3 nodes, FP32 vectors, restart 10: the two passes
+// 144 -> 80 us a step on average (a branch per vector and 4-byte loads before); at
+// 257^3 with K = 6 pass 2 takes 533 us, 4.6 TB/s, the rate of a copy.
+template <typename T>
+struct alignas(16) Quad {
+    T v[4];
+};
+template <typename T>
+__device__ __forceinline__ Quad<T> load_quad(const T* __restrict__ p, long q) {
+    return *reinterpret_cast<const Quad<T>*>(p + 4 * q);
+}
+
 // Pass 1: slot i < n of the partials holds Q_i, slot n + i holds R_i.
-template <typename TV = double>
-__global__ void __launch_bounds__(kBlock) k_multidot2_partial(const TV* __restrict__ V, int n, long M, long ld,
+template <int K, typename TV>
+__global__ void __launch_bounds__(kBlock) k_multidot2_partial(const TV* __restrict__ V, long M, long ld,
                                                               const double* __restrict__ w,
                                                               double* __restrict__ partial) {
-    __shared__ double sh[kBlock / 64][2 * kMultiDotMax];
-    const TV* __restrict__ t = V + (long)(n - 1) * ld;
-    const int k = n - 1;  // vectors before t
-    double aw[kMultiDotMax - 1], at[kMultiDotMax - 1], awl = 0.0, atl = 0.0;
+    constexpr int n = K + 1;
+    __shared__ double sh[kBlock / 64][2 * n];
+    double aw[n], at[n];
 #pragma unroll
-    for (int i = 0; i < kMultiDotMax - 1; ++i) aw[i] = at[i] = 0.0;
-    // two grid strides per step with independent loads (four held 256 VGPRs
-    // with an FP64 basis, and ran at half speed with an FP32 one)
-    constexpr int kU = 2;
-    const long st = (long)gridDim.x * kBlock;
-    long q = (long)blockIdx.x * kBlock + threadIdx.x;
-    for (; q + (kU - 1) * st < M; q += kU * st) {
-        double wq[kU], tq[kU], vq[kMultiDotMax - 1][kU];
+    for (int i = 0; i < n; ++i) aw[i] = at[i] = 0.0;
+    const long G = M / 4, st = (long)gridDim.x * kBlock;
+    for (long q = (long)blockIdx.x * kBlock + threadIdx.x; q < G; q += st) {
+        const Quad<double> wq = load_quad(w, q);
+        Quad<TV> vq[n];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            wq[u] = w[q + u * st];
-            tq[u] = (double)t[q + u * st];
-        }
+        for (int i = 0; i < n; ++i) vq[i] = load_quad(V + (long)i * ld, q);
 #pragma unroll
-        for (int i = 0; i < kMultiDotMax - 1; ++i)
+        for (int i = 0; i < n; ++i)
 #pragma unroll
-            for (int u = 0; u < kU; ++u) vq[i][u] = i < k ? (double)V[(long)i * ld + q + u * st] : 0.0;
-#pragma unroll
-        for (int i = 0; i < kMultiDotMax - 1; ++i)
-#pragma unroll
-            for (int u = 0; u < kU; ++u)
-                if (i < k) {
-                    aw[i] += vq[i][u] * wq[u];
-                    at[i] += vq[i][u] * tq[u];
-                }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            awl += tq[u] * wq[u];
-            atl += tq[u] * tq[u];
-        }
-    }
-    for (; q < M; q += st) {
-        const double wq = w[q], tq = (double)t[q];
-#pragma unroll
-        for (int i = 0; i < kMultiDotMax - 1; ++i)
-            if (i < k) {
-                const double v = (double)V[(long)i * ld + q];
-                aw[i] += v * wq;
-                at[i] += v * tq;
+            for (int u = 0; u < 4; ++u) {
+                aw[i] += (double)vq[i].v[u] * wq.v[u];
+                at[i] += (double)vq[i].v[u] * (double)vq[K].v[u];
             }
-        awl += tq * wq;
-        atl += tq * tq;
+    }
+    if (blockIdx.x == 0 && 4 * G + threadIdx.x < M) {
+        const long q = 4 * G + threadIdx.x;
+        const double wq = w[q], tq = (double)V[(long)K * ld + q];
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const double v = (double)V[(long)i * ld + q];
+            aw[i] += v * wq;
+            at[i] += v * tq;
+        }
     }
     const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
     auto wave_sum = [](double v) {
@@ -1708,20 +1704,11 @@ __global__ void __launch_bounds__(kBlock) k_multidot2_partial(const TV* __restri
         return v;
     };
 #pragma unroll
-    for (int i = 0; i < kMultiDotMax - 1; ++i) {
-        if (i < k) {
-            const double a = wave_sum(aw[i]), b = wave_sum(at[i]);
-            if (lane == 0) {
-                sh[wave][i] = a;
-                sh[wave][n + i] = b;
-            }
-        }
-    }
-    {
-        const double a = wave_sum(awl), b = wave_sum(atl);
+    for (int i = 0; i < n; ++i) {
+        const double a = wave_sum(aw[i]), b = wave_sum(at[i]);
         if (lane == 0) {
-            sh[wave][k] = a;
-            sh[wave][n + k] = b;
+            sh[wave][i] = a;
+            sh[wave][n + i] = b;
         }
     }
     __syncthreads();
@@ -1740,81 +1727,72 @@ __global__ void __launch_bounds__(kBlock) k_multidot2_partial(const TV* __restri
 // the span of the other vectors).  With FP32 vectors the rewritten V_{n-1}
 // is rounded to FP32 and w is projected on the rounded vector, the one the
 // later passes read.
-template <typename TV = double>
-__global__ void __launch_bounds__(kBlock) k_dcgs2_update(TV* __restrict__ V, int n, long M, long ld,
-                                                         double* __restrict__ w, const double* __restrict__ d,
-                                                         double* __restrict__ coef, double* __restrict__ partial) {
+template <int K, typename TV>
+__global__ void __launch_bounds__(kBlock) k_dcgs2_update(TV* __restrict__ V, long M, long ld, double* __restrict__ w,
+                                                         const double* __restrict__ d, double* __restrict__ coef,
+                                                         double* __restrict__ partial) {
+    constexpr int n = K + 1;
     __shared__ double sh[kBlock / 64];
-    TV* __restrict__ t = V + (long)(n - 1) * ld;
-    const int k = n - 1;
-    double p[kMultiDotMax - 1], c[kMultiDotMax - 1];
+    TV* __restrict__ t = V + (long)K * ld;
+    double p[K], c[K];
     double pp = 0.0, pq = 0.0;
 #pragma unroll
-    for (int i = 0; i < kMultiDotMax - 1; ++i) {
-        p[i] = i < k ? d[n + i] : 0.0;
-        c[i] = i < k ? d[i] : 0.0;
+    for (int i = 0; i < K; ++i) {
+        p[i] = d[n + i];
+        c[i] = d[i];
         pp += p[i] * p[i];
         pq += p[i] * c[i];
     }
-    const double a2 = d[n + k] - pp;
+    const double a2 = d[n + K] - pp;
     const double alpha = a2 > 0.0 ? sqrt(a2) : 0.0;
     const double inv = alpha > 0.0 ? 1.0 / alpha : 0.0;
-    const double cl = (d[k] - pq) * inv;
+    const double cl = (d[K] - pq) * inv;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        for (int i = 0; i < k; ++i) {
-            coef[i] = d[n + i];
-            coef[n + i] = d[i];
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            coef[i] = p[i];
+            coef[n + i] = c[i];
         }
-        coef[k] = inv;
-        coef[n + k] = cl;
+        coef[K] = inv;
+        coef[n + K] = cl;
         coef[2 * n] = alpha;
     }
     double nrm = 0.0;
-    // two grid strides per step with independent loads (four held 256 VGPRs)
-    constexpr int kU = 2;
-    const long st = (long)gridDim.x * kBlock;
-    long q = (long)blockIdx.x * kBlock + threadIdx.x;
-    for (; q + (kU - 1) * st < M; q += kU * st) {
-        double wq[kU], tq[kU], vq[kMultiDotMax - 1][kU];
+    // the entry of t and of w from those of the vectors before t
+    auto update = [&](const double v[K], TV& tq, double& wq) {
+        double b = (double)tq, a = wq;
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            wq[u] = w[q + u * st];
-            tq[u] = (double)t[q + u * st];
+        for (int i = 0; i < K; ++i) {
+            b += -p[i] * v[i];
+            a += -c[i] * v[i];
         }
-#pragma unroll
-        for (int i = 0; i < kMultiDotMax - 1; ++i)
-#pragma unroll
-            for (int u = 0; u < kU; ++u) vq[i][u] = i < k ? (double)V[(long)i * ld + q + u * st] : 0.0;
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            double v = tq[u], a = wq[u];
-#pragma unroll
-            for (int i = 0; i < kMultiDotMax - 1; ++i)
-                if (i < k) {
-                    v += -p[i] * vq[i][u];
-                    a += -c[i] * vq[i][u];
-                }
-            const TV vs = (TV)(v * inv);
-            a += -cl * (double)vs;
-            t[q + u * st] = vs;
-            w[q + u * st] = a;
-            nrm += a * a;
-        }
-    }
-    for (; q < M; q += st) {
-        double v = (double)t[q], a = w[q];
-#pragma unroll
-        for (int i = 0; i < kMultiDotMax - 1; ++i)
-            if (i < k) {
-                const double vi = (double)V[(long)i * ld + q];
-                v += -p[i] * vi;
-                a += -c[i] * vi;
-            }
-        const TV vs = (TV)(v * inv);
-        a += -cl * (double)vs;
-        t[q] = vs;
-        w[q] = a;
+        tq = (TV)(b * inv);
+        a += -cl * (double)tq;
+        wq = a;
         nrm += a * a;
+    };
+    const long G = M / 4, st = (long)gridDim.x * kBlock;
+    for (long q = (long)blockIdx.x * kBlock + threadIdx.x; q < G; q += st) {
+        Quad<double> wq = load_quad(w, q);
+        Quad<TV> tq = load_quad(t, q), vq[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) vq[i] = load_quad(V + (long)i * ld, q);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            double v[K];
+#pragma unroll
+            for (int i = 0; i < K; ++i) v[i] = (double)vq[i].v[u];
+            update(v, tq.v[u], wq.v[u]);
+        }
+        *reinterpret_cast<Quad<TV>*>(t + 4 * q) = tq;
+        *reinterpret_cast<Quad<double>*>(w + 4 * q) = wq;
+    }
+    if (blockIdx.x == 0 && 4 * G + threadIdx.x < M) {
+        const long q = 4 * G + threadIdx.x;
+        double v[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) v[i] = (double)V[(long)i * ld + q];
+        update(v, t[q], w[q]);
     }
     const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
 #pragma unroll
