@@ -35,7 +35,7 @@ constexpr int kLevels = 4;
 constexpr int kCh[kLevels] = {16, 32, 64, 128};
 constexpr int kLossBlocks = 256;
 constexpr int kWgradBlocks = 256;  // target workgroups of one weight-gradient launch
-constexpr int kBiasBlocks = 256;   // most workgroups (bias partials) of k_wgrad_dz
+constexpr int kBiasBlocks = 256;   // most workgroups (bias partials) of k_wgrad_rows on dZ
 
 inline unsigned nb256(long n) { return (unsigned)((n + 255) / 256); }
 inline unsigned nb64(long n) { return (unsigned)((n + 63) / 64); }
@@ -45,6 +45,7 @@ struct ConvL {
     int cin, cout, cinp, coutp, level;
     bool relu;
     long woff, boff;  // offsets of W and b in the canonical parameter vector
+    long poff = 0;    // of its partial weight gradients
     bf16_t* wt = nullptr;  // [coutp][27 cinp] (aunet::frag_index)
     bf16_t* wb = nullptr;  // [cinp][27 coutp], taps flipped
 };
@@ -63,8 +64,8 @@ struct alamo_nn_s {
     int adam_t = 0;
     bool packed = false;    // bf16 weights up to date with p
     bool have_fwd = false;
-    float* part = nullptr;  // per-chunk partial weight gradients of one layer
-    float* bpart = nullptr; // and its bias gradient's
+    float* part = nullptr;  // per-chunk partial weight gradients, every layer's (ConvL::poff)
+    float* bpart = nullptr; // and the bias gradients' (kBiasBlocks * 128 a layer)
     bf16_t *trx = nullptr, *trz = nullptr;  // its transposed input (three shifts) and output gradient
     float* loss_part = nullptr;
     float* dtmp = nullptr;  // output gradient of train_step [n_out][N0]
@@ -182,24 +183,47 @@ void conv_fwd(alamo_nn_t nn, int li, const bf16_t* X, bf16_t* Y, float* Yf, hipS
     launch_conv(X, L.cinp, L.wt, nn->p + L.boff, L.coutp, nn->g[L.level], L.relu ? 1 : 0, Y, Yf, nn->n_out, s);
 }
 
+int bias_blocks(const ConvL& L, const WgradGrid& w) {
+    return (int)std::min<long>(kBiasBlocks, (w.ngroup * L.coutp + 255) / 256);
+}
+float* bias_part(alamo_nn_t nn, int li) { return nn->bpart + (long)li * kBiasBlocks * kCh[kLevels - 1]; }
+
 // Backward of conv li: dY (bf16, masked in place for ReLU layers), X its
-// input, Y its output.  Writes the weight and bias gradients into grad and,
-// when dX is given, the input gradient.
-void conv_back(alamo_nn_t nn, int li, const bf16_t* X, const bf16_t* Y, bf16_t* dY, bf16_t* dX, float* grad,
-               hipStream_t s) {
+// input, Y its output.  Leaves the weight and bias gradients' partials for
+// finish_gradients and, when dX is given, the input gradient.
+void conv_back(alamo_nn_t nn, int li, const bf16_t* X, const bf16_t* Y, bf16_t* dY, bf16_t* dX, hipStream_t s) {
     const ConvL& L = nn->cv[li];
     const G3& g = nn->g[L.level];
     const int tiles = (L.cinp / 16) * (L.coutp / 16);
     const WgradGrid w = wgrad_grid(g, tiles);
-    const int nb = (int)std::min<long>(kBiasBlocks, (w.ngroup * L.coutp + 255) / 256);
-    aunet::k_wgrad_dz<<<nb, 256, 0, s>>>(dY, L.relu ? Y : nullptr, L.coutp, g.nx, w.n8, w.ngroup, nn->trz, nn->bpart);
-    aunet::k_wgrad_x<<<nb256(w.ngroup * L.cinp), 256, 0, s>>>(X, L.cinp, g.nx, w.n8, w.ngroup, nn->trx);
-    aunet::k_conv_wgrad<<<dim3(tiles, w.nchunk), 64 * aunet::kWgradWaves, 0, s>>>(nn->trx, L.cinp, nn->trz, L.coutp, g.ny,
-                                                                                  g.nz, w.n8, w.steps, nn->part);
-    const long ne = 27L * L.cin * L.cout + L.cout;  // the layer's weights and biases are adjacent
-    aunet::k_wgrad_finish<<<(unsigned)((ne + 63) / 64), 256, 0, s>>>(nn->part, w.nchunk, L.cin, L.cout, L.cinp, L.coutp,
-                                                                     nn->bpart, nb, grad + L.woff);
+    const int nb = bias_blocks(L, w);
+    aunet::k_wgrad_rows<<<nb + nb256(w.ngroup * L.cinp), 256, 0, s>>>(
+        dY, L.relu ? Y : nullptr, L.coutp, X, L.cinp, g.nx, w.n8, w.ngroup, nb, nn->trz, nn->trx, bias_part(nn, li));
+    aunet::k_conv_wgrad<<<dim3(tiles, w.nchunk), 64 * aunet::kWgradWaves, 0, s>>>(
+        nn->trx, L.cinp, nn->trz, L.coutp, g.ny, g.nz, w.n8, w.steps, nn->part + L.poff);
     if (dX) launch_conv(dY, L.coutp, L.wb, nullptr, L.cinp, g, 0, dX, nullptr, 0, s);
+}
+
+// Every layer's weight and bias gradients into grad, from conv_back's partials.
+void finish_gradients(alamo_nn_t nn, float* grad, hipStream_t s) {
+    aunet::FinishLayers F{};
+    F.n = (int)nn->cv.size();
+    for (int l = 0; l < F.n; ++l) {
+        const ConvL& L = nn->cv[l];
+        const WgradGrid w = wgrad_grid(nn->g[L.level], (L.cinp / 16) * (L.coutp / 16));
+        const long ne = 27L * L.cin * L.cout + L.cout;  // the layer's weights and biases are adjacent
+        F.first[l + 1] = F.first[l] + (unsigned)((ne + 63) / 64);
+        F.part[l] = nn->part + L.poff;
+        F.bpart[l] = bias_part(nn, l);
+        F.grad[l] = grad + L.woff;
+        F.nchunk[l] = w.nchunk;
+        F.cin[l] = L.cin;
+        F.cout[l] = L.cout;
+        F.cinp[l] = L.cinp;
+        F.coutp[l] = L.coutp;
+        F.nb[l] = bias_blocks(L, w);
+    }
+    aunet::k_wgrad_finish<<<F.first[F.n], 256, 0, s>>>(F);
 }
 
 int forward(alamo_nn_t nn, const float* in, float* out, hipStream_t s) {
@@ -239,12 +263,12 @@ int backward(alamo_nn_t nn, const float* dout, float* grad, float* din, hipStrea
     const int last = (int)nn->cv.size() - 1;
     aunet::k_pack_soa<<<dim3((unsigned)((g[0].N + 63) / 64), nn->coutp_out / 16), 256, 0, s>>>(dout, nn->n_out, nn->coutp_out, g[0].N,
                                                                           nn->gY);
-    conv_back(nn, last, nn->G[0], nullptr, nn->gY, nn->gG[0], grad, s);
+    conv_back(nn, last, nn->G[0], nullptr, nn->gY, nn->gG[0], s);
     for (int l = 0; l <= kLevels - 2; ++l) {
         const int li = 2 * kLevels + 2 * (kLevels - 2 - l);
         const int cu = kCh[l + 1], ce = kCh[l];
-        conv_back(nn, li + 1, nn->B[l], nn->G[l], nn->gG[l], nn->gB[l], grad, s);
-        conv_back(nn, li, nn->K[l], nn->B[l], nn->gB[l], nn->gK[l], grad, s);
+        conv_back(nn, li + 1, nn->B[l], nn->G[l], nn->gG[l], nn->gB[l], s);
+        conv_back(nn, li, nn->K[l], nn->B[l], nn->gB[l], nn->gK[l], s);
         // adjoint of trilinear up: 8 x full weighting, of the decoder input's first cu channels
         bf16_t* dst = (l + 1 < kLevels - 1) ? nn->gG[l + 1] : nn->gE[kLevels - 1];
         aunet::k_down<<<nb64((long)g[l + 1].N * cu / 2), aunet::kWave, 0, s>>>(nn->gK[l], cu + ce, cu, g[l], g[l + 1], 1.f, dst);
@@ -257,11 +281,12 @@ int backward(alamo_nn_t nn, const float* dout, float* grad, float* din, hipStrea
                                                                              nn->gK[l], kCh[l + 1] + kCh[l], kCh[l + 1],
                                                                              nn->gE[l]);
         }
-        conv_back(nn, 2 * l + 1, nn->A[l], nn->E[l], nn->gE[l], nn->gA[l], grad, s);
+        conv_back(nn, 2 * l + 1, nn->A[l], nn->E[l], nn->gE[l], nn->gA[l], s);
         const bf16_t* Xl = l == 0 ? nn->X0 : nn->D[l];
         bf16_t* dXl = l == 0 ? (din ? nn->gX0 : nullptr) : nn->gD[l];
-        conv_back(nn, 2 * l, Xl, nn->A[l], nn->gA[l], dXl, grad, s);
+        conv_back(nn, 2 * l, Xl, nn->A[l], nn->gA[l], dXl, s);
     }
+    finish_gradients(nn, grad, s);
     if (din)
         aunet::k_unpack_soa<<<nb256((long)g[0].N * nn->n_in), 256, 0, s>>>(nn->gX0, nn->n_in, nn->cin0p, g[0].N, din);
     NNCHK(hipGetLastError());
@@ -344,13 +369,14 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
     NNCHK(hipMemset(nn->p, 0, sizeof(float) * np));
     NNCHK(hipMemset(nn->m, 0, sizeof(float) * np));
     NNCHK(hipMemset(nn->v, 0, sizeof(float) * np));
-    long partmax = 0, xmax = 0, zmax = 0;
+    long parts = 0, xmax = 0, zmax = 0;
     size_t nweights = 0;
     for (auto& L : nn->cv) {
         const long M = (long)L.coutp * 27 * L.cinp;
         nweights += aunet::frag_size(27 * L.cinp, L.coutp) + aunet::frag_size(27 * L.coutp, L.cinp);
         const WgradGrid w = wgrad_grid(nn->g[L.level], (L.cinp / 16) * (L.coutp / 16));
-        partmax = std::max(partmax, M * w.nchunk);
+        L.poff = parts;
+        parts += M * w.nchunk;
         xmax = std::max(xmax, 3L * L.cinp * 8 * w.ngroup);
         zmax = std::max(zmax, (long)L.coutp * 8 * w.ngroup);
     }
@@ -362,7 +388,8 @@ int alamo_nn_create(const int nodes[3], int n_in, int n_out, alamo_nn_t* out) {
         L.wb = L.wt + aunet::frag_size(27 * L.cinp, L.coutp);
         w = L.wb + aunet::frag_size(27 * L.coutp, L.cinp);
     }
-    if ((rc = nalloc_t(nn, &nn->part, partmax)) || (rc = nalloc_t(nn, &nn->bpart, (long)kBiasBlocks * kCh[kLevels - 1])) ||
+    if ((rc = nalloc_t(nn, &nn->part, parts)) ||
+        (rc = nalloc_t(nn, &nn->bpart, (long)nn->cv.size() * kBiasBlocks * kCh[kLevels - 1])) ||
         (rc = nalloc_t(nn, &nn->trx, xmax)) || (rc = nalloc_t(nn, &nn->trz, zmax)) ||
         (rc = nalloc_t(nn, &nn->loss_part, kLossBlocks)))
         return cleanup(rc);

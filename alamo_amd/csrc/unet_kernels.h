@@ -237,26 +237,57 @@ __global__ void __launch_bounds__(64 * KS) k_conv_fwd_ks(const bf16_t* __restric
 // dW[co][t][ci] = sum_v dZ[v][co] X[v + d_t][ci] reduces over nodes, which are
 // the MFMA K dimension: a lane holds 8 consecutive K of one channel.  The
 // activations are channels-last, where those 8 are strided two-byte loads, so
-// both operands are first transposed into rows of nodes: T[c][row][i], row =
-// z ny + y, i padded to n8 groups of 8 with zeros.  X is kept three times,
+// both operands are first transposed into groups of 8 nodes of a row (the last one
+// filled up with zeros): group q = row n8 + i / 8, row = z ny + y, of 16 channels
+// in a run of 256 bytes (row_group), so that a wave's load of 4 groups of 16
+// channels is 1 KB in a row whichever tap it is for; as T[c][row][i] the 16 lanes
+// took 16 bytes from 16 places, which bound the kernel.  X is kept three times,
 // shifted by -1, 0 and 1 along i, so that every tap is an aligned 16-byte load.
-// At 33^3 nodes, 15 layers: 422 us for the four kernels (wgrad 14.0, finish 5.5,
-// transposes 4.5 and 4.2 us a layer), where gathers of two bytes a lane, up to
-// 1123 partials a weight summed by one thread each, a mask, a bias and an
+// At 33^3 nodes, 15 layers: 231 us for the three kernels (wgrad 8.3 us and the
+// transposes 5.1 us a layer, finish 30.5 us), where gathers of two bytes a lane, up
+// to 1123 partials a weight summed by one thread each, a mask, a bias and an
 // unpacking launch took 2112 us.
+__host__ __device__ inline size_t row_group(size_t c, long q, long ngroup) {
+    return (((c >> 4) * ngroup + q) * 16 + (c & 15)) * 8;
+}
 
-// One thread per (group of 8 nodes, channel): the gradient dY of a layer's output
-// masked by its ReLU (Y the output; null: no ReLU), in place, its transpose T, and
-// the block's sums per channel (the bias gradient's partials, bpart[block][C]).
-// C is a power of two, at most 128.
-__global__ void __launch_bounds__(kThreads) k_wgrad_dz(bf16_t* __restrict__ dY, const bf16_t* __restrict__ Y, int C,
-                                                       int nx, int n8, long ngroup, bf16_t* __restrict__ T,
-                                                       float* __restrict__ bpart) {
+// Both transposes of a layer, one thread per (group of 8 nodes, channel); the first
+// nbz workgroups take dZ, the others X (4.1 and 4.5 us a layer as two launches,
+// 5.1 us as one).
+// dZ: the gradient dY of the layer's output masked by its ReLU (Y the output; null:
+// no ReLU), in place, its transpose Tz, and the block's sums per channel (the bias
+// gradient's partials, bpart[block][C]).  C is a power of two, at most 128.
+// X: its three shifted transposes, Tx[s][c][row][i] = X[row][i + s - 1][c] (channel s Cin + c).
+__global__ void __launch_bounds__(kThreads) k_wgrad_rows(bf16_t* __restrict__ dY, const bf16_t* __restrict__ Y, int C,
+                                                         const bf16_t* __restrict__ X, int Cin, int nx, int n8,
+                                                         long ngroup, unsigned nbz, bf16_t* __restrict__ Tz,
+                                                         bf16_t* __restrict__ Tx, float* __restrict__ bpart) {
     __shared__ float sh[kThreads];
+    if (blockIdx.x >= nbz) {
+        const long t = (long)(blockIdx.x - nbz) * kThreads + threadIdx.x;
+        const long q = t / Cin;
+        if (q >= ngroup) return;
+        const int c = (int)(t - q * Cin);
+        const long row = q / n8;
+        const int i0 = (int)(q - row * n8) * 8;
+        uint32_t v[10];
+#pragma unroll
+        for (int e = 0; e < 10; ++e) {
+            const int i = i0 + e - 1;
+            const bool in = i >= 0 && i < nx;
+            const uint32_t x = X[((size_t)row * nx + (in ? i : 0)) * Cin + c];
+            v[e] = in ? x : 0u;
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+            *reinterpret_cast<uint4*>(Tx + row_group((size_t)s * Cin + c, q, ngroup)) =
+                make_uint4(v[s] | (v[s + 1] << 16), v[s + 2] | (v[s + 3] << 16), v[s + 4] | (v[s + 5] << 16),
+                           v[s + 6] | (v[s + 7] << 16));
+        return;
+    }
     const int c = (int)threadIdx.x & (C - 1), sub = (int)threadIdx.x / C, nsub = kThreads / C;
-    const long rows = ngroup / n8;
     float sum = 0.f;
-    for (long q = (long)blockIdx.x * nsub + sub; q < ngroup; q += (long)gridDim.x * nsub) {
+    for (long q = (long)blockIdx.x * nsub + sub; q < ngroup; q += (long)nbz * nsub) {
         const long row = q / n8;
         const int i0 = (int)(q - row * n8) * 8;
         const size_t at = ((size_t)row * nx + i0) * C + c;
@@ -274,7 +305,7 @@ __global__ void __launch_bounds__(kThreads) k_wgrad_dz(bf16_t* __restrict__ dY, 
             if (Y && in) dY[at + (size_t)e * C] = (bf16_t)v[e];
             sum += bf2f((bf16_t)v[e]);
         }
-        *reinterpret_cast<uint4*>(T + ((size_t)c * rows + row) * (8 * n8) + i0) =
+        *reinterpret_cast<uint4*>(Tz + row_group(c, q, ngroup)) =
             make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
     }
     sh[threadIdx.x] = sum;
@@ -284,47 +315,24 @@ __global__ void __launch_bounds__(kThreads) k_wgrad_dz(bf16_t* __restrict__ dY, 
         bpart[(size_t)blockIdx.x * C + c] = sum;
     }
 }
-// The three shifted transposes of X: T[s][c][row][i] = X[row][i + s - 1][c].
-__global__ void __launch_bounds__(kThreads) k_wgrad_x(const bf16_t* __restrict__ X, int C, int nx, int n8, long ngroup,
-                                                      bf16_t* __restrict__ T) {
-    const long t = (long)blockIdx.x * kThreads + threadIdx.x;
-    const long q = t / C;
-    if (q >= ngroup) return;
-    const int c = (int)(t - q * C);
-    const long row = q / n8, rows = ngroup / n8;
-    const int i0 = (int)(q - row * n8) * 8;
-    uint32_t v[10];
-#pragma unroll
-    for (int e = 0; e < 10; ++e) {
-        const int i = i0 + e - 1;
-        const bool in = i >= 0 && i < nx;
-        const uint32_t x = X[((size_t)row * nx + (in ? i : 0)) * C + c];
-        v[e] = in ? x : 0u;
-    }
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-        *reinterpret_cast<uint4*>(T + (((size_t)s * C + c) * rows + row) * (8 * n8) + i0) =
-            make_uint4(v[s] | (v[s + 1] << 16), v[s + 2] | (v[s + 3] << 16), v[s + 4] | (v[s + 5] << 16),
-                       v[s + 6] | (v[s + 7] << 16));
-}
 // Partial weight gradient of one 16 x 16 tile of (co, ci), all 27 taps, over the
 // blockIdx.y-th part of the node groups: part[chunk][co][t][ci].  4 waves share
-// the part's steps of 4 groups (one per 16 lanes), their tiles added in wave
-// order through LDS.
+// the part's steps of 4 groups (one per 16 lanes); their tiles are added in wave
+// order through LDS, each wave a quarter of the taps
+// (one wave after the other, wave 0 storing all: 12.0 us a layer, 8.3 so).
 constexpr int kWgradWaves = 4;
 __global__ void __launch_bounds__(64 * kWgradWaves) k_conv_wgrad(const bf16_t* __restrict__ Tx, int Cin,
                                                                  const bf16_t* __restrict__ Tz, int Cout, int ny, int nz,
                                                                  int n8, int steps, float* __restrict__ part) {
-    __shared__ f32x4 red[27][64];
+    __shared__ f32x4 red[kWgradWaves][27][64];  // 108 KB: a workgroup has a CU to itself
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ncib = Cin / 16, cib = blockIdx.x % ncib, cob = blockIdx.x / ncib, ch = blockIdx.y;
     const int r16 = lane & 15, grp = lane >> 4;
     const int co = cob * 16 + r16, ci = cib * 16 + r16;
-    const int rows = ny * nz;
-    const long ngroup = (long)rows * n8;
-    const size_t line = 8 * (size_t)n8, sx = (size_t)Cin * rows * line;  // a row; a shift of Tx
-    const bf16_t* zc = Tz + (size_t)co * rows * line;
-    const bf16_t* xc = Tx + (size_t)ci * rows * line;
+    const long ngroup = (long)ny * nz * n8;
+    const bf16_t* zc = Tz + row_group(co, 0, ngroup);
+    const bf16_t* xc = Tx + row_group(ci, 0, ngroup);
+    const size_t sx = (size_t)Cin * ngroup * 8;  // a shift of Tx
     f32x4 acc[27];
 #pragma unroll
     for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -334,10 +342,10 @@ __global__ void __launch_bounds__(64 * kWgradWaves) k_conv_wgrad(const bf16_t* _
     for (int st = wave; st < steps; st += kWgradWaves) {
         const long q = ((long)ch * steps + st) * 4 + grp;
         const bool in = q < ngroup;
-        const int row = in ? (int)(q / n8) : 0, g8 = in ? (int)(q - (long)row * n8) : 0;
+        const long qi = in ? q : 0;
+        const int row = (int)(qi / n8);
         const int z = row / ny, y = row - z * ny;
-        const bf16x8 A =
-            __builtin_bit_cast(bf16x8, keep(in, *reinterpret_cast<const uint4*>(zc + row * line + 8 * g8)));
+        const bf16x8 A = __builtin_bit_cast(bf16x8, keep(in, *reinterpret_cast<const uint4*>(zc + qi * 128)));
         uint4 bq[3][9];
 #pragma unroll
         for (int dz = 0; dz < 3; ++dz)
@@ -345,7 +353,7 @@ __global__ void __launch_bounds__(64 * kWgradWaves) k_conv_wgrad(const bf16_t* _
             for (int dy = 0; dy < 3; ++dy) {
                 const int zz = z + dz - 1, yy = y + dy - 1;
                 const bool ok = in && zz >= 0 && zz < nz && yy >= 0 && yy < ny;
-                const bf16_t* xr = xc + (ok ? zz * ny + yy : row) * line + 8 * g8;
+                const bf16_t* xr = xc + (qi + (ok ? ((dz - 1) * ny + dy - 1) * n8 : 0)) * 128;
 #pragma unroll
                 for (int s = 0; s < 3; ++s) bq[dz][3 * dy + s] = keep(ok, *reinterpret_cast<const uint4*>(xr + s * sx));
             }
@@ -354,57 +362,60 @@ __global__ void __launch_bounds__(64 * kWgradWaves) k_conv_wgrad(const bf16_t* _
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, bq[t / 9][t % 9]), acc[t], 0,
                                                              0, 0);
     }
-    for (int w = 1; w < kWgradWaves; ++w) {
-        if (wave == w) {
 #pragma unroll
-            for (int t = 0; t < 27; ++t) red[t][lane] = acc[t];
-        }
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int t = 0; t < 27; ++t) acc[t] += red[t][lane];
-        }
-        __syncthreads();
-    }
-    if (wave > 0) return;
+    for (int t = 0; t < 27; ++t) red[wave][t][lane] = acc[t];
+    __syncthreads();
     // acc[t][e] = D[co_local = 4 grp + e][ci_local = r16]
+    for (int t = wave; t < 27; t += kWgradWaves) {
+        f32x4 sum = red[0][t][lane];
 #pragma unroll
-    for (int t = 0; t < 27; ++t)
+        for (int w = 1; w < kWgradWaves; ++w) sum += red[w][t][lane];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            part[(((size_t)ch * Cout + cob * 16 + grp * 4 + e) * 27 + t) * Cin + ci] = acc[t][e];
+            part[(((size_t)ch * Cout + cob * 16 + grp * 4 + e) * 27 + t) * Cin + ci] = sum[e];
+    }
 }
-// The layer's gradient from the partials, in the canonical parameter order:
+// Every layer's gradient from its partials, in the canonical parameter order:
 // grad[0 .. 27 cin cout) the weights from part[nchunk][coutp][27][cinp], then the
 // cout biases from bpart[nb][coutp].  64 entries a workgroup, 4 threads an entry,
-// each every 4th partial, added in order.
-__global__ void __launch_bounds__(kThreads) k_wgrad_finish(const float* __restrict__ part, int nchunk, int cin, int cout,
-                                                           int cinp, int coutp, const float* __restrict__ bpart, int nb,
-                                                           float* __restrict__ grad) {
+// each every 4th partial, added in order.  One launch, layer l from workgroup
+// first[l] on (5.3 us a layer as 15 launches, 30.5 us for all).
+constexpr int kMaxConv = 15;
+struct FinishLayers {
+    int n;
+    unsigned first[kMaxConv + 1];
+    const float *part[kMaxConv], *bpart[kMaxConv];
+    float* grad[kMaxConv];
+    int nchunk[kMaxConv], cin[kMaxConv], cout[kMaxConv], cinp[kMaxConv], coutp[kMaxConv], nb[kMaxConv];
+};
+__global__ void __launch_bounds__(kThreads) k_wgrad_finish(FinishLayers F) {
     __shared__ float sh[4][64];
-    const long nw = 27L * cin * cout, e = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+    int l = 0;
+    while (blockIdx.x >= F.first[l + 1]) ++l;  // the grid has first[n] workgroups
+    const int cin = F.cin[l], cout = F.cout[l], cinp = F.cinp[l], coutp = F.coutp[l], nchunk = F.nchunk[l], nb = F.nb[l];
+    const long nw = 27L * cin * cout, e = (long)(blockIdx.x - F.first[l]) * 64 + (threadIdx.x & 63);
     const int sl = threadIdx.x >> 6;
     float s = 0.f;
     if (e < nw) {
         const long q = e / cin;
-        const float* p = part + q * cinp + (e - q * cin);  // q = co 27 + t
+        const float* p = F.part[l] + q * cinp + (e - q * cin);  // q = co 27 + t
         const long M = 27L * cinp * coutp;
 #pragma unroll 4
         for (int c = sl; c < nchunk; c += 4) s += p[c * M];
     } else if (e < nw + cout) {
+        const float* p = F.bpart[l] + (e - nw);
 #pragma unroll 4
-        for (int c = sl; c < nb; c += 4) s += bpart[(size_t)c * coutp + (e - nw)];
+        for (int c = sl; c < nb; c += 4) s += p[(size_t)c * coutp];
     }
     sh[sl][threadIdx.x & 63] = s;
     __syncthreads();
-    if (sl == 0 && e < nw + cout) grad[e] = ((s + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
+    if (sl == 0 && e < nw + cout) F.grad[l][e] = ((s + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
 }
 
 // Canonical float32 W[Cout][27][Cin] -> bf16 Wt[Coutp][27 * Cinp] (zero
 // padded) and the flipped transpose Wb[Cinp][27 * Coutp],
 // Wb[ci][t][co] = W[co][26 - t][ci], used by the input gradient, both in the order
 // of frag_index.  Every layer in one launch: layer l takes the threads from first[l] on.
-constexpr int kMaxConv = 15;
 struct PackLayers {
     int n;
     long first[kMaxConv + 1];

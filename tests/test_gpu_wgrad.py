@@ -1,4 +1,4 @@
-"""The weight and bias gradients (k_wgrad_dz, k_wgrad_x, k_conv_wgrad,
+"""The weight and bias gradients (k_wgrad_rows, k_conv_wgrad,
 k_wgrad_finish) of the output convolution against sums in float64 of the same
 bfloat16 operands: its output gradient is the caller's, rounded, and its input
 the forward tape, so nothing but the float32 sums differs.  Each sum has at most
