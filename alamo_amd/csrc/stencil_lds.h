@@ -341,7 +341,7 @@ __device__ __forceinline__ void tile_store(T* __restrict__ s, const T pre[TS::PR
 // periodic axes (their face nodes, in the boundary workgroups, take the
 // wrapped interior row from the level's C, Cf).
 template <class TS, typename T, int OP, bool DC, int CM, typename TX = T, bool PER = false>
-__global__ void __launch_bounds__(TS::NT)
+__global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : 3)
     k_stencil_lds(const TX* __restrict__ x, const T* __restrict__ b, const T* __restrict__ diag,
                   const T* __restrict__ Ct, const T* __restrict__ Cb, const T* __restrict__ Cf,
                   const int* __restrict__ bct, int uniform,
@@ -358,6 +358,11 @@ __global__ void __launch_bounds__(TS::NT)
     // FP32 runs 4 per CU: placed last they form a trailing round of their own
     // (65^3 sweep 12.9 us vs 11.9 first; 129^3 residual 63.5 vs 61.8 us).
     constexpr bool kBoundaryLast = sizeof(T) == 8;
+    // D with the plane's other loads, or after C's part of the row: in FP64 its 36
+    // registers then take C's place and a SIMD holds 3 waves instead of 2 (97 x 81 x
+    // 113 sweep @@S64@@); in FP32 a fifth wave
+    // does not fit without spills and the later wait costs (129^3 solve 21.6 -> 22.0 ms).
+    constexpr bool kDFirst = sizeof(T) == 4;
     const unsigned ntb = gridDim.x - nbb;  // tile workgroups
     const bool bnd = kBoundaryLast ? blockIdx.x >= ntb : blockIdx.x < nbb;
     if (bnd) {
@@ -463,17 +468,19 @@ __global__ void __launch_bounds__(TS::NT)
             for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1) ? ld32(b + (size_t)p * N, o) : T(0);
         }
         bool flagged = false;
+        unsigned dpos = 0;  // this node's place among the compact D
+        auto load_d = [&](T dv[18]) {
+#pragma unroll
+            for (int q = 0; q < 18; ++q) dv[q] = ld32(Dc + (size_t)q * nflag, dpos);
+        };
         if constexpr (DC) {
             const unsigned gm = (unsigned)(gpk & 0xfu);
             gpk >>= 4;
             flagged = !uniform && gm != 0u;
             const unsigned long long bal = __ballot(flagged);
             const int base = __builtin_amdgcn_readlane(dwb_lane, kk);
-            if (flagged) {
-                const unsigned pidx = (unsigned)base + (unsigned)__popcll(bal & lanes_below());
-#pragma unroll
-                for (int q = 0; q < 18; ++q) dv[q] = ld32(Dc + (size_t)q * nflag, pidx);
-            }
+            dpos = (unsigned)base + (unsigned)__popcll(bal & lanes_below());
+            if (kDFirst && flagged) load_d(dv);
         }
         if (more) tile_fetch<TS, T, TX>(x, L, it, jt, k + 2 * d, pre);
         __builtin_amdgcn_sched_barrier(0);
@@ -538,6 +545,7 @@ __global__ void __launch_bounds__(TS::NT)
                 }
             }
             if (DC && flagged) {
+                if (!kDFirst) load_d(dv);
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
 #pragma unroll
