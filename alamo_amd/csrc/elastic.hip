@@ -888,16 +888,11 @@ int assemble_direct(alamo_el_t h, hipStream_t s) {
 // Compact grad-C matrices of one level (MajorMinor): per-wave counts of the
 // flagged interior nodes, their exclusive prefix (on the host, once per
 // model), then D of each flagged node at its position.
-// Levels whose interior is at least kTiledMin nodes along every axis use the
-// LDS-tiled MajorMinor kernel (unless ALAMO_EL_STENCIL=slab-only).
-constexpr int kTiledMin = 32;
 // Isotropic levels also need this many interior nodes: FP64 sweeps of 41^3 and
 // 49^3 nodes take 6.8 and 8.3 us in tiles (2 x 6 of them a plane, many lanes past
 // the box) and 7.0 and 7.8 us by node, of 65^3 nodes 9.2 and 12.1.
 constexpr long kTiledMinIso = 128l << 10;
-bool tiled_level(const Lvl& L) {
-    return stencil_variant() == kVariantSlab && L.nx - 2 >= kTiledMin && L.ny - 2 >= kTiledMin && L.nz - 2 >= kTiledMin;
-}
+bool tiled_level(const Lvl& L) { return stencil_variant() == kVariantSlab && ael::tiles_serve(L); }
 
 // The palette of a tiled level (ael::k_pal_index): the distinct 21-slot
 // tensors of its nodes when there are at most ael::kPalMax of them and at most

@@ -273,7 +273,8 @@ __host__ __device__ constexpr bool slot_in_col(int s, int a) {
 
 // Load base[idx] with a 32-bit element index: with base uniform, the address
 // is a scalar base plus a 32-bit byte offset (no 64-bit vector address math).
-// Every array indexed this way holds fewer than 2^32 bytes (checked at create).
+// Every array indexed this way holds fewer than 2^32 bytes: a field's component
+// (checked at create), on the tiled levels the whole field (tiles_serve).
 template <typename T>
 __device__ __forceinline__ T ld32(const T* __restrict__ base, unsigned idx) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (size_t)(idx * (unsigned)sizeof(T)));

@@ -49,6 +49,18 @@ struct TileGrid {
 // a plane in one 64-bit register.
 constexpr int kMaxChunk = 16;
 
+// Levels that tiles may serve (unless ALAMO_EL_STENCIL=slab-only): at least
+// kTiledMin interior nodes along every axis, and an FP64 field below 2^32 bytes.
+// The lanes of a halo load take different components through one base with a
+// 32-bit byte offset (tile_fetch, plane_fetch), which wraps from 178,956,971
+// nodes on; the per-node kernels add a component's offset in 64 bits and take
+// the larger boxes.
+constexpr int kTiledMin = 32;
+inline bool tiles_serve(const Lvl& L) {
+    return L.nx - 2 >= kTiledMin && L.ny - 2 >= kTiledMin && L.nz - 2 >= kTiledMin &&
+           3 * L.N * (long)sizeof(double) < (1L << 32);
+}
+
 // Interior copy of C in tile blocks: the 21 slots of the TX x TY nodes of
 // one (tile, plane) are contiguous, slot-major, so that the workgroup's 21
 // loads of a plane read one block (21 NT values) and each wave's load of a
