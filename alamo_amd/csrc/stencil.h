@@ -43,6 +43,17 @@ __device__ __forceinline__ void store_row(T* __restrict__ out, const Lvl& L, uns
         st32(out + (size_t)p * L.N, n32, finish_op<T, OP>(o[p], xv[p], bv[p], dv[p], omega));
 }
 
+// Whether an isotropic sweep reads its diagonal: in FP32 the stored one, the FP64
+// diagonal rounded once.  Formed in FP32 from lambda, mu and the spacings it would
+// carry the rounding of each of them and of every sum (a sweep of x = 0 off by 4.2
+// 2^-24 of itself against 2.5, at 21 x 19 x 23 nodes).  The read costs an FP32 sweep
+// of 129^3 nodes 3 us of 34, of 201^3 24 us of 142; solves in FP32 cycles nothing
+// that the runs resolve (97^3: 12.6 ms either way).
+template <typename T, int OP>
+__host__ __device__ constexpr bool iso_reads_diag() {
+    return OP == 2 && sizeof(T) == 4;
+}
+
 // One thread per node over the whole box (XCD-remapped), any OP.
 template <typename T, int SYM, int OP>
 __global__ void __launch_bounds__(kBlock)
@@ -266,18 +277,24 @@ __global__ void __launch_bounds__(kBlock)
                 st32(out + (size_t)p * L.N, o32, finish_op<T, OP>(o[p], xv[p], bv[p], dv[p], omega));
             return;
         } else if constexpr (SYM == 0) {
-            // Every load of the node first, as for MajorMinor; the Jacobi
+            // Every load of the node first, as for MajorMinor; the FP64 Jacobi
             // diagonal from the lambda and mu already there instead of a load.
             const unsigned o32 = (unsigned)id;
             T uv[3][15], cv[2][7], dg[3];
             iso_load<T>(x, C, L, o32, uv, cv);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1) ? ld32(b + (size_t)p * L.N, o32) : T(0);
+            for (int p = 0; p < 3; ++p) {
+                const size_t off = (size_t)p * L.N;
+                bv[p] = (OP >= 1) ? ld32(b + off, o32) : T(0);
+                if constexpr (iso_reads_diag<T, OP>()) dv[p] = ld32(diag + off, o32);
+            }
             __builtin_amdgcn_sched_barrier(0);
             iso_compute<T>(uv, cv, H, uniform != 0, o, dg);
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-                st32(out + (size_t)p * L.N, o32, finish_op<T, OP>(o[p], uv[p][0], bv[p], dg[p], omega));
+            for (int p = 0; p < 3; ++p) {
+                const T d = iso_reads_diag<T, OP>() ? dv[p] : dg[p];
+                st32(out + (size_t)p * L.N, o32, finish_op<T, OP>(o[p], uv[p][0], bv[p], d, omega));
+            }
             return;
         } else {
             apply_interior<T, SYM>(x, C, uniform, L, id, o, gmask ? (unsigned)gmask[id] : 7u);

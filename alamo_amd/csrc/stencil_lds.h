@@ -584,8 +584,8 @@ __global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : 3)
 // 59 neighbour values a node through L1; a workgroup of it covers two rows, so
 // the rows and planes around them come from L2 about six times.  Here a plane
 // of a tile is read once per march (1.33 times with the halo), 40.8 KB of LDS
-// and at most 128 registers leave 4 workgroups a CU in FP64.  A Jacobi sweep
-// takes its interior diagonal from lambda and mu.  Boundary nodes as in
+// and at most 128 registers leave 4 workgroups a CU in FP64.  An FP64 Jacobi
+// sweep takes its interior diagonal from lambda and mu.  Boundary nodes as in
 // k_stencil_lds.  FP64 sweep: 31.7 us at 129 x 113 x 97 nodes (45.2 by node;
 // 88 B a node: 3.9 TB/s), 211 us at 201^3 (322; 3.4 TB/s, 4.2 with the halos).
 template <class TS, int NF>
@@ -669,9 +669,12 @@ __global__ void __launch_bounds__(TS::NT) __attribute__((amdgpu_waves_per_eu(4))
         const bool more = kk + 1 < nstep;
         const unsigned o = (unsigned)k * sxy + col;
         // every global load of the plane leaves here, before the LDS work
-        T bv[3];
+        T bv[3], dv[3];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) bv[p] = (OP >= 1 && valid) ? ld32(b + (size_t)p * N, o) : T(0);
+        for (int p = 0; p < 3; ++p) {
+            bv[p] = (OP >= 1 && valid) ? ld32(b + (size_t)p * N, o) : T(0);
+            if constexpr (iso_reads_diag<T, OP>()) dv[p] = valid ? ld32(diag + (size_t)p * N, o) : T(1);
+        }
         if (more) {
             plane_fetch<TS, 3>(x, L, it, jt, k + 2 * d, pu);
             plane_fetch<TS, 2>(C, L, it, jt, k + 2 * d, pc);
@@ -723,8 +726,10 @@ __global__ void __launch_bounds__(TS::NT) __attribute__((amdgpu_waves_per_eu(4))
             }
             iso_row<T>(D, cv, H, uniform != 0, ov, dg);
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-                st32(out + (size_t)p * N, o, finish_op<T, OP>(ov[p], su[sn][p * HP + c0], bv[p], dg[p], omega));
+            for (int p = 0; p < 3; ++p) {
+                const T dp = iso_reads_diag<T, OP>() ? dv[p] : dg[p];
+                st32(out + (size_t)p * N, o, finish_op<T, OP>(ov[p], su[sn][p * HP + c0], bv[p], dp, omega));
+            }
         }
         if (more) {
             __syncthreads();  // every read of slot sb (the plane behind) is done
