@@ -353,7 +353,7 @@ __device__ __forceinline__ void tile_store(T* __restrict__ s, const T pre[TS::PR
 // periodic axes (their face nodes, in the boundary workgroups, take the
 // wrapped interior row from the level's C, Cf).
 template <class TS, typename T, int OP, bool DC, int CM, typename TX = T, bool PER = false>
-__global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : 3)
+__global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : PER && OP == 2 ? 2 : 3)
     k_stencil_lds(const TX* __restrict__ x, const T* __restrict__ b, const T* __restrict__ diag,
                   const T* __restrict__ Ct, const T* __restrict__ Cb, const T* __restrict__ Cf,
                   const int* __restrict__ bct, int uniform,
@@ -364,17 +364,22 @@ __global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : 3)
     __shared__ T su[3][TS::RING];  // [ring slot][component][hy][hx], padded to RING
     // The nbb boundary workgroups (a multiple of kXcd, so that tile ib keeps
     // ib % kXcd == XCD) come after the tile ones in FP64 and before them in
-    // FP32.  FP64 runs 2 workgroups per CU and 2 rounds of tiles: the latency-
-    // bound boundary workgroups fill the slots the second round frees (Fapply
-    // at 129^3: 101.5 us, vs 106.3 first and 110.4 spread among the tiles).
-    // FP32 runs 4 per CU: placed last they form a trailing round of their own
-    // (65^3 sweep 12.9 us vs 11.9 first; 129^3 residual 63.5 vs 61.8 us).
+    // FP32.  FP64 tiles take more than one round: the latency-bound boundary
+    // workgroups fill the slots that the last round frees (Fapply at 129^3, with
+    // 2 workgroups a CU: 101.5 us, vs 106.3 first and 110.4 spread among the tiles).
+    // FP32 runs 4 per CU in one round: placed last they form a trailing round of
+    // their own (65^3 sweep 12.9 us vs 11.9 first; 129^3 residual 63.5 vs 61.8 us).
     constexpr bool kBoundaryLast = sizeof(T) == 8;
     // D with the plane's other loads, or after C's part of the row: in FP64 its 36
-    // registers then take C's place and a SIMD holds 3 waves instead of 2 (97 x 81 x
-    // 113 sweep @@S64@@); in FP32 a fifth wave
-    // does not fit without spills and the later wait costs (129^3 solve 21.6 -> 22.0 ms).
-    constexpr bool kDFirst = sizeof(T) == 4;
+    // registers then take C's place and a SIMD holds 3 waves instead of 2.  FP64
+    // sweeps by palette / by C copy, 2 waves and 3: 97 x 81 x 113 nodes 42.2 / 44.6
+    // and 37.1 / 40.3 us, 129^3 63.9 / 85.1 and 62.1 / 86.0, 193^3 251 / 279 and
+    // 237 / 268.  A periodic sweep holds more, for the wrapped rows, and would spill
+    // 10 registers at 3 waves: it keeps 2 (129^3: 139 and 135 us; periodic Fapply and
+    // residual spill 2 at 3 waves and are still faster, 97 x 81 x 113 nodes 50.0 -> 47.8
+    // and 51.6 -> 48.2).  In FP32 a fifth wave does not fit without spills and the
+    // later wait costs (129^3 solve 21.6 -> 22.0 ms).
+    constexpr bool kDFirst = sizeof(T) == 4 || (PER && OP == 2);
     const unsigned ntb = gridDim.x - nbb;  // tile workgroups
     const bool bnd = kBoundaryLast ? blockIdx.x >= ntb : blockIdx.x < nbb;
     if (bnd) {
