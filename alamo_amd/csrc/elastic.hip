@@ -94,10 +94,10 @@ struct Level {
     Lvl L{};  // L.per: periodic axes, the handle's on every MG level
     Vecs<double> d;
     Vecs<float> f;
-    unsigned char* gmask = nullptr;  // per node: axes along which C varies (k_grad_mask)
+    unsigned char* gmask = nullptr;  // per node: axes along which C varies (k_grad_mask; null: isotropic)
     int* dwbase = nullptr;           // per interior wave of the launch: first compact D position
     int nflag = 0;                   // interior nodes with a nonzero gmask
-    bool tiled = false;              // MajorMinor level served by k_stencil_lds (else k_stencil_slab)
+    bool tiled = false;              // served by k_stencil_lds or, isotropic, k_stencil_iso (else k_stencil_slab)
     double* psi = nullptr;           // SetPsi weight on this level's cells (null until set)
     ael::PalIdx* pidx = nullptr;     // palette row of every interior node, tile-blocked (null: no palette)
     ael::PalIdx* pidx_b = nullptr;   // palette row of every boundary node, in boundary_node order
@@ -1382,7 +1382,7 @@ int alamo_el_create(const int n_cell[3], const double dx[3], int sym, int max_co
         const long N = l.L.N;
         int rc;
         if ((rc = alloc((void**)&l.d.C, sizeof(double) * h->nc * N))) return cleanup(rc);
-        if ((rc = alloc((void**)&l.gmask, N))) return cleanup(rc);
+        if (sym != 0 && (rc = alloc((void**)&l.gmask, N))) return cleanup(rc);
         for (double** p : {&l.d.diag, &l.d.cor, &l.d.cor_hold, &l.d.res, &l.d.rescor, &l.d.tmp})
             if ((rc = alloc((void**)p, sizeof(double) * 3 * N))) return cleanup(rc);
     }
