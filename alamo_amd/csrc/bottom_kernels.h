@@ -180,7 +180,6 @@ __global__ void __launch_bounds__(64) k_bottom_rows(const double* __restrict__ A
         for (int r = 0; r < 3; ++r) vals[at + r * plane] = a[r];
     };
     int n = 0;
-#pragma unroll 4
     for (int c0 = 0; c0 < M; c0 += 64) {
         const int c = c0 + lane;
         double a[3];

@@ -216,20 +216,26 @@ enum { kVariantSlab = 0, kVariantSlabNoMask = 1, kVariantNode = 2, kVariantSlabO
 // no faster).
 using TileT = ael::Tile<32, 8>;
 constexpr long kNtMinBytes = 64l << 20;
-// Chunks of k planes sized for the resident tile workgroups: two rounds of
-// 2 per CU in FP64 (200-220 VGPRs), one round of 4 per CU in FP32 (110-120
-// VGPRs).  At 129^3: FP64 chunks of 8 planes (1024 workgroups; Fapply
-// 104.4 us vs 108.4 with 3 planes, 107.0 with 4, 108.8 with 16), FP32 chunks
-// of 8 (sweep 37.2 us vs 39.2 with chunks of 4, 41.4 with 16; the FP32
-// solve 0.15 ms faster).  ALAMO_EL_TILE_TARGET (read when a level's C is
-// set) replaces both targets: the tests use it to reach every chunk length
-// on small boxes.
+// Chunks of k planes sized for the resident tile workgroups.  FP64: two rounds of
+// 2 per CU, from when the kernel held 2 waves a SIMD (Fapply at 129^3 by C copy
+// 104.4 us, vs 108.4 with chunks of 3 planes, 107.0 with 4, 108.8 with 16); a
+// periodic sweep still holds 2, the others 3 now.  Fapply / sweep by palette with
+// targets of 512, 768, 1024 and 1536 workgroups: 129^3 nodes 57.7 / 61.8, 52.1 /
+// 57.8, 56.6 / 62.1, 54.7 / 60.2 us, 97 x 81 x 113 33.5 / 36.0, 35.0 / 36.7, 35.5 /
+// 37.1, 35.4 / 38.2.  FP32: one round of 4 per CU (sweep at 129^3 in chunks of 8
+// planes 37.2 us vs 39.2 with chunks of 4, 41.4 with 16; the FP32 solve 0.15 ms
+// faster).  ALAMO_EL_TILE_TARGET (read when a level's C is set) replaces every
+// target: the tests use it to reach every chunk length on small boxes.
 constexpr long kTileTarget64 = 2 * 2 * 256, kTileTarget32 = 4 * 256;
-// The isotropic tiled kernel: at most 3 workgroups a CU in FP64, 7 in FP32.
-// FP64 sweeps with 512, 640, 768, 1024 and 2048 workgroups as the target:
-// 129 x 113 x 97 nodes 37.2, 34.1, 31.1, 31.7, 32.8 us; 65^3 nodes, in chunks of
-// 2 planes (which read 4) 9.2 us, in chunks of 1 (which read 3) 10.7; 201^3
-// nodes take the longest chunk for all, 211 us.
+// The isotropic tiled kernel, whose chunks read two planes more than they write: at
+// most 3 workgroups a CU in FP64, where 4 fit, and 7 in FP32, where 7 fit of Fapply
+// and 6 of a sweep.  FP64 sweeps with targets of 512, 640, 768, 1024 and 2048: 65^3
+// nodes 9.3, 9.2, 9.5, 10.2, 10.2 us (chunks of 2 planes up to 768, then 1), 129 x
+// 113 x 97 35.1, 36.7, 31.6, 31.5, 32.8, 129^3 47.3, 50.2, 47.2, 44.7, 45.5; 201^3
+// takes the longest chunk for all, 213.  FP32 Fapply / sweep with 1024, 1280, 1536,
+// 1792 and 2048: 97 x 81 x 113 13.4 / 17.3, 12.9 / 17.3, 13.2 / 17.4, 14.3 / 18.0,
+// 14.0 / 18.0 us, 129^3 23.0 / 33.6, 23.1 / 34.6, 22.9 / 33.5, 22.4 / 34.4, 23.3 /
+// 33.1: the runs of one target differ by as much.
 constexpr long kTileTargetIso64 = 3 * 256, kTileTargetIso32 = 7 * 256;
 ael::TileGrid tile_grid_of(const Lvl& L, long target, bool up = false) {
     const char* e = std::getenv("ALAMO_EL_TILE_TARGET");
@@ -2520,8 +2526,7 @@ struct AmrCtx {
     }
     // max |v| over the composite grid: each handle's res (use_res) or b, ghost
     // nodes and nodes strictly covered by a child excluded.  One read of each
-    // field and one wait for the host (a copy to scratch, a mask launch per
-    // child, a reduction and a wait a handle before).
+    // field and one wait for the host.
     int composite_norm(double* norm, bool use_res) {
         long at = 0;
         for (int i = 0; i < n; ++i) {

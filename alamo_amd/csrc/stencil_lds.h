@@ -1,5 +1,6 @@
-// stencil_lds.h -- LDS-staged MajorMinor stencil kernel for the large MG
-// levels.
+// stencil_lds.h -- LDS-staged stencil kernels for the large MG levels:
+// k_stencil_lds for MajorMinor C, described here, and k_stencil_iso for isotropic C
+// (at the end of the file).
 //
 // A workgroup owns a TX x TY tile of (i, j) interior columns and marches it
 // over a chunk of kc planes in k, one node per thread per plane.  u lives in
@@ -12,7 +13,8 @@
 // work (a scheduling barrier keeps the compiler from sinking each load to
 // its use, which would cost one memory round trip per load); the chunk's
 // gradient masks and compact D bases are fetched once, in the prologue,
-// so that no load of a plane waits on another.  Boundary nodes take nbb
+// so that no load of a plane waits on another.  The exception is D in FP64, loaded
+// after C's part of the row, whose registers it takes (kDFirst).  Boundary nodes take nbb
 // workgroups of their own, after the tiles in FP64 and before them in FP32
 // (see the kernel).  Jacobi sweeps compute an interior node's diagonal from
 // its C instead of reading diag.
@@ -592,7 +594,7 @@ __global__ void __launch_bounds__(TS::NT, sizeof(T) == 4 ? 4 : PER && OP == 2 ? 
 // and at most 128 registers leave 4 workgroups a CU in FP64.  An FP64 Jacobi
 // sweep takes its interior diagonal from lambda and mu.  Boundary nodes as in
 // k_stencil_lds.  FP64 sweep: 31.7 us at 129 x 113 x 97 nodes (45.2 by node;
-// 88 B a node: 3.9 TB/s), 211 us at 201^3 (322; 3.4 TB/s, 4.2 with the halos).
+// 88 B a node: 3.9 TB/s), 213 us at 201^3 (322; 3.4 TB/s, 4.2 with the halos).
 template <class TS, int NF>
 struct PlaneShare {
     static constexpr int PRE = (NF * TS::HP + TS::NT - 1) / TS::NT;  // values per thread per plane of NF fields
